@@ -138,7 +138,8 @@ int lf_tri_mult(lf_context* ctx, const lf_tri_mult_args* args);
  * arguments, kernels and results as lf_tri_mult, but its scratch (the a, b and X planes,
  * 3 * c_hidden * N^2 f16, plus 8 * N^2 bytes of LayerNorm statistics with 2-byte activations
  * at c_z = c_hidden = 128; weights are decoded while being staged into LDS, so they take no
- * scratch) lives in a static per-device array of LF_TRI_NOALLOC_SCRATCH_BYTES (reserved on
+ * scratch) lives in a static per-device array of LF_TRI_NOALLOC_SCRATCH_BYTES and 6 MiB for the
+ * padding of the planes' rows (reserved on
  * every device the library loads on, used or not), looked up once per device by
  * lf_context_create; nothing is
  * allocated or freed.  Shapes needing more scratch are rejected with LF_ERR_INVALID (c_hidden

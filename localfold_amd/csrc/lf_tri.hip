@@ -59,13 +59,17 @@ struct TriProjectParams {
   _Float16* out[2];    // a, b: [H][P]
   int N;               // length (P = N * N)
   int kmajor_out;      // store each channel plane transposed: a[h][j][k] for pair (k, j)
+  int ld;              // 128-wide kernels: row pitch of a channel plane (N rounded up to 16)
+  size_t plane;        // ... and a plane's size, N * ld
   int split;           // AF3 in the resident kernels: wp[0] / wg[0] are the whole interleaved
                        // tensors (even stored columns -> a, odd -> b); wp[1] / wg[1] unused
   float2* stats;       // when not NULL (128-wide kernel only): LN_in (mean, 1/std) per pair, by z row
 };
 
 struct TriOutputParams {
-  const _Float16* X;   // [H][P]
+  const _Float16* X;   // [H][P]; 128-wide kernel: [H][N][ld]
+  int N, ld;
+  size_t plane;        // N * ld
   const void* z;
   void* out;
   int accumulate;
@@ -219,8 +223,12 @@ struct TriContractParams {
   const _Float16* R;
   _Float16* X;        // [H][N][N]
   int N;
+  int ld;             // row pitch of L, R and X in the direct-to-LDS kernels (N, or N rounded up to 16)
   float scale;
 };
+
+// What a lane loads in place of a 16-byte piece of k past the row pitch.
+__device__ __attribute__((aligned(16))) const _Float16 tri_zero16[8] = {};
 
 template <int TM, int BK, bool KMAJOR>
 __device__ __forceinline__ void ct_load(_Float16* S, const _Float16* src, int N, int m0, int k0, int tid) {
@@ -376,14 +384,16 @@ __global__ __launch_bounds__(256, MINW) void tri_contract_kernel(TriContractPara
   }
 }
 
-// The outgoing-layout contraction (k contiguous in both operands) when N is a multiple of BK:
-// TM x TM tiles (TM = 128 or 96), K steps of BK double-buffered in LDS and filled by direct global -> LDS
+// The contraction of operands with k contiguous and a row pitch that is a multiple of 16 (the
+// columns from N to the pitch hold zeros): TM x TM tiles (TM = 128 or 96), K steps of BK double-buffered in LDS and filled by direct global -> LDS
 // loads (16 bytes a lane, no register staging), one barrier a step, the next step's loads in
 // flight during the current step's MFMAs.  A wave's load instruction fills 1 KB of LDS
 // contiguously, so the 16-byte chunks of a row are XOR-swizzled by the row (chunk c of row r
 // sits in slot c ^ swz(r)) to keep the MFMA fragment reads of 16 rows off a single bank group.
-// Rows past N are clamped to row N - 1: they only feed output rows or columns that are never
-// stored.
+// Rows past N are clamped to row N - 1: they only feed output rows that are never stored, or
+// columns between N and the pitch.  In a last K step that reaches past the pitch the pieces
+// beyond it come from a zero word (TAIL; without it, a pitch of whole steps, the check alone
+// costs 3% at N = 384).
 // At TM = 128 the two 32 KB stages hold the LDS at two blocks (8 waves) per CU, at TM = 96
 // (24 KB stages) three.  Measured at N = 384 the 128-row kernel beats the register-staged
 // kernel above (30.9 against 33.1 us), and 8-wave blocks or 32-wide K steps with four blocks
@@ -393,7 +403,14 @@ __device__ __forceinline__ int ct_swz(int r) {
   return BK == 64 ? (r & 7) : ((r >> 1) & 3);
 }
 
-template <int BK, int TM>
+// The 16-byte chunk of its rows that thread tid stages: its pieces are a multiple of 8 rows
+// apart, which the swizzle repeats over.
+template <int BK>
+__device__ __forceinline__ int ct_chunk(int tid) {
+  return (tid % (BK / 8)) ^ ct_swz<BK>(tid / (BK / 8));
+}
+
+template <int BK, int TM, bool TAIL>
 __global__ __launch_bounds__(256, TM == 128 ? 2 : 3) void tri_contract_dma_kernel(TriContractParams p) {
   constexpr int NT = 256, FM = TM / 32, FN = TM / 32, WT = TM / 2, WTN = TM / 2, CH = BK / 8,
                 PER = TM * CH / NT, STAGE = TM * BK;
@@ -407,7 +424,7 @@ __global__ __launch_bounds__(256, TM == 128 ? 2 : 3) void tri_contract_dma_kerne
   if (lin < per * 8) lin = (lin & 7) * per + (lin >> 3);
   const int h = lin / tiles, t = lin - h * tiles;
   const int m0 = (t / tm) * TM, n0 = (t % tm) * TM;
-  const size_t plane = (size_t)p.N * p.N;
+  const size_t plane = (size_t)p.N * p.ld;
   const _Float16* L = p.L + h * plane;
   const _Float16* R = p.R + h * plane;
   // this thread's pieces: LDS slot q = it * 256 + tid holds row q / CH, chunk (q % CH) ^ swz
@@ -416,16 +433,21 @@ __global__ __launch_bounds__(256, TM == 128 ? 2 : 3) void tri_contract_dma_kerne
 #pragma unroll
   for (int it = 0; it < PER; ++it) {
     const int q = it * NT + tid, r = q / CH, c = (q % CH) ^ ct_swz<BK>(r);
-    gl[it] = L + (size_t)min(m0 + r, p.N - 1) * p.N + c * 8;
-    gr[it] = R + (size_t)min(n0 + r, p.N - 1) * p.N + c * 8;
+    gl[it] = L + (size_t)min(m0 + r, p.N - 1) * p.ld + c * 8;
+    gr[it] = R + (size_t)min(n0 + r, p.N - 1) * p.ld + c * 8;
   }
+  const int ck = ct_chunk<BK>(tid) * 8;   // this thread's k within a step (the same in every piece)
   auto issue = [&](int k0, int st) __attribute__((always_inline)) {
+    const bool past = TAIL && k0 + BK > p.ld;   // uniform: a last step that reaches past the pitch
 #pragma unroll
     for (int it = 0; it < PER; ++it) {
       const int base = (it * NT + wave * 64) * 8;
+      const _Float16* sl = gl[it] + k0;
+      const _Float16* sr = gr[it] + k0;
+      if (past && k0 + ck >= p.ld) sl = sr = tri_zero16;
 #if __HIP_DEVICE_COMPILE__   // a target builtin: the host pass, which only emits the launch stub, lacks it
-      __builtin_amdgcn_global_load_lds(gl[it] + k0, &S[st][0][base], 16, 0, 0);
-      __builtin_amdgcn_global_load_lds(gr[it] + k0, &S[st][1][base], 16, 0, 0);
+      __builtin_amdgcn_global_load_lds(sl, &S[st][0][base], 16, 0, 0);
+      __builtin_amdgcn_global_load_lds(sr, &S[st][1][base], 16, 0, 0);
 #endif
     }
   };
@@ -436,7 +458,7 @@ __global__ __launch_bounds__(256, TM == 128 ? 2 : 3) void tri_contract_dma_kerne
     for (int j = 0; j < FN; ++j) acc[i][j] = f4{0.f, 0.f, 0.f, 0.f};
   const int r16 = lane & 15, g4 = lane >> 4;
   issue(0, 0);
-  const int nk = p.N / BK;
+  const int nk = (p.ld + BK - 1) / BK;
   for (int ks = 0; ks < nk; ++ks) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();   // step ks in LDS for every wave; every wave done with the other stage
@@ -472,12 +494,12 @@ __global__ __launch_bounds__(256, TM == 128 ? 2 : 3) void tri_contract_dma_kerne
       h4 o;
 #pragma unroll
       for (int r = 0; r < 4; ++r) o[r] = (_Float16)(acc[i][j][r] * p.scale);
-      if (gm < p.N && gn < p.N) *reinterpret_cast<h4*>(X + (size_t)gm * p.N + gn) = o;
+      if (gm < p.N && gn < p.ld) *reinterpret_cast<h4*>(X + (size_t)gm * p.ld + gn) = o;
     }
   }
 }
 
-// Large N (a multiple of 64, at least 768, when whole 256-row tiles add at most 10% to the
+// Large N (at least 768, when whole 256-row tiles add at most 10% to the
 // work of 128-row ones; rows past N clamped as above): 256 x 256 tiles, 8 waves in a 2 x 4 grid, each
 // wave 128 x 64 (32 accumulator tiles), the same direct-to-LDS double buffering as above in
 // two 64 KB stages (one block per CU).  A wave's K step reads 384 bytes of LDS per MFMA
@@ -486,7 +508,7 @@ __global__ __launch_bounds__(256, TM == 128 ? 2 : 3) void tri_contract_dma_kerne
 // measured 0.38 ms (twice the barriers).
 
 
-template <int BK>
+template <int BK, bool TAIL>
 __global__ __launch_bounds__(512) void tri_contract_big_kernel(TriContractParams p) {
   constexpr int TM = 256, NT = 512, FM = 8, FN = 4, WT = 128, WTN = 64, CH = BK / 8, PER = TM * CH / NT,
                 STAGE = TM * BK;
@@ -500,7 +522,7 @@ __global__ __launch_bounds__(512) void tri_contract_big_kernel(TriContractParams
   if (lin < per * 8) lin = (lin & 7) * per + (lin >> 3);
   const int h = lin / tiles, t = lin - h * tiles;
   const int m0 = (t / tm) * TM, n0 = (t % tm) * TM;
-  const size_t plane = (size_t)p.N * p.N;
+  const size_t plane = (size_t)p.N * p.ld;
   const _Float16* L = p.L + h * plane;
   const _Float16* R = p.R + h * plane;
   const _Float16* gl[PER];
@@ -508,16 +530,21 @@ __global__ __launch_bounds__(512) void tri_contract_big_kernel(TriContractParams
 #pragma unroll
   for (int it = 0; it < PER; ++it) {
     const int q = it * NT + tid, r = q / CH, c = (q % CH) ^ ct_swz<BK>(r);
-    gl[it] = L + (size_t)min(m0 + r, p.N - 1) * p.N + c * 8;
-    gr[it] = R + (size_t)min(n0 + r, p.N - 1) * p.N + c * 8;
+    gl[it] = L + (size_t)min(m0 + r, p.N - 1) * p.ld + c * 8;
+    gr[it] = R + (size_t)min(n0 + r, p.N - 1) * p.ld + c * 8;
   }
+  const int ck = ct_chunk<BK>(tid) * 8;   // this thread's k within a step (the same in every piece)
   auto issue = [&](int k0, int st) __attribute__((always_inline)) {
+    const bool past = TAIL && k0 + BK > p.ld;
 #pragma unroll
     for (int it = 0; it < PER; ++it) {
       const int base = (it * NT + wave * 64) * 8;
+      const _Float16* sl = gl[it] + k0;
+      const _Float16* sr = gr[it] + k0;
+      if (past && k0 + ck >= p.ld) sl = sr = tri_zero16;
 #if __HIP_DEVICE_COMPILE__
-      __builtin_amdgcn_global_load_lds(gl[it] + k0, &S[st][0][base], 16, 0, 0);
-      __builtin_amdgcn_global_load_lds(gr[it] + k0, &S[st][1][base], 16, 0, 0);
+      __builtin_amdgcn_global_load_lds(sl, &S[st][0][base], 16, 0, 0);
+      __builtin_amdgcn_global_load_lds(sr, &S[st][1][base], 16, 0, 0);
 #endif
     }
   };
@@ -527,7 +554,7 @@ __global__ __launch_bounds__(512) void tri_contract_big_kernel(TriContractParams
 #pragma unroll
     for (int j = 0; j < FN; ++j) acc[i][j] = f4{0.f, 0.f, 0.f, 0.f};
   const int r16 = lane & 15, g4 = lane >> 4;
-  const int nk = p.N / BK;
+  const int nk = (p.ld + BK - 1) / BK;
   issue(0, 0);
   for (int ks = 0; ks < nk; ++ks) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -570,7 +597,7 @@ __global__ __launch_bounds__(512) void tri_contract_big_kernel(TriContractParams
       h4 o;
 #pragma unroll
       for (int r = 0; r < 4; ++r) o[r] = (_Float16)(acc[i][j][r] * p.scale);
-      if (gm < p.N && gn < p.N) *reinterpret_cast<h4*>(X + (size_t)gm * p.N + gn) = o;
+      if (gm < p.N && gn < p.ld) *reinterpret_cast<h4*>(X + (size_t)gm * p.ld + gn) = o;
     }
   }
 }
@@ -582,12 +609,14 @@ static void launch_contract(lf_context* ctx, const TriContractParams& cp, int H,
   const bool vec = (cp.N % 8) == 0;
   if (!kmajor) {
     const long long t256 = (cp.N + 255) / 256, t128 = (cp.N + 127) / 128;
-    if (TM == 128 && cp.N % 64 == 0 && cp.N >= 768 && t256 * t256 * 65536 * 10 <= t128 * t128 * 16384 * 11) {
-      hipLaunchKernelGGL((tri_contract_big_kernel<64>), dim3((unsigned)(t256 * t256 * H)), dim3(512), 0, ctx->stream,
-                         cp);
+    const bool dma = cp.ld % 8 == 0, tail = cp.ld % 64 != 0;   // rows of whole 16-byte pieces; of whole K steps
+    if (TM == 128 && dma && cp.N >= 768 && t256 * t256 * 65536 * 10 <= t128 * t128 * 16384 * 11) {
+      const dim3 g((unsigned)(t256 * t256 * H));
+      auto k = tail ? tri_contract_big_kernel<64, true> : tri_contract_big_kernel<64, false>;
+      hipLaunchKernelGGL(k, g, dim3(512), 0, ctx->stream, cp);
       return;
     }
-    if (TM == 128 && cp.N % 64 == 0) {
+    if (TM == 128 && dma) {
       // 128-row tiles at two blocks per CU, or, when the grid is only a few waves of blocks
       // and the last one would run mostly empty, 96-row tiles at three per CU.  Measured: at
       // N = 384 (1152 tiles of 128 in 512 slots: 2.25 waves) the 96-row kernel is 3-4%
@@ -597,14 +626,13 @@ static void launch_contract(lf_context* ctx, const TriContractParams& cp, int H,
       const long long b128 = (long long)tm * tm * H, b96 = (long long)t96 * t96 * H;
       const double w128 = (double)((b128 + slots - 1) / slots);
       const double w96 = (double)((b96 + slots * 3 / 2 - 1) / (slots * 3 / 2)) * (96.0 * 96.0) / (128.0 * 128.0);
-      if (b128 <= 4 * slots && w96 < 0.85 * w128)
-        hipLaunchKernelGGL((tri_contract_dma_kernel<64, 96>), dim3((unsigned)b96), dim3(256), 0, ctx->stream, cp);
-      else
-        hipLaunchKernelGGL((tri_contract_dma_kernel<64, 128>), grid, dim3(256), 0, ctx->stream, cp);
+      const bool small = b128 <= 4 * slots && w96 < 0.85 * w128;
+      auto k = small ? (tail ? tri_contract_dma_kernel<64, 96, true> : tri_contract_dma_kernel<64, 96, false>)
+                     : (tail ? tri_contract_dma_kernel<64, 128, true> : tri_contract_dma_kernel<64, 128, false>);
+      hipLaunchKernelGGL(k, dim3((unsigned)(small ? b96 : b128)), dim3(256), 0, ctx->stream, cp);
       return;
     }
-    if (vec) hipLaunchKernelGGL((tri_contract_kernel<TM, BK, MINW, false, true>), grid, dim3(256), 0, ctx->stream, cp);
-    else hipLaunchKernelGGL((tri_contract_kernel<TM, BK, MINW, false, false>), grid, dim3(256), 0, ctx->stream, cp);
+    hipLaunchKernelGGL((tri_contract_kernel<TM, BK, MINW, false, false>), grid, dim3(256), 0, ctx->stream, cp);
   } else {
     if (vec) hipLaunchKernelGGL((tri_contract_kernel<TM, BK, MINW, true, true>), grid, dim3(256), 0, ctx->stream, cp);
     else hipLaunchKernelGGL((tri_contract_kernel<TM, BK, MINW, true, false>), grid, dim3(256), 0, ctx->stream, cp);
@@ -948,16 +976,12 @@ __global__ __launch_bounds__(512) void tri_output_resident_kernel(TriOutputParam
   }
 }
 
-// Project kernels for c_z = c_hidden = 128 (every AF2/AF3 pair width at production size),
-// weights resident in LDS.  The gate weights and biases arrive pre-multiplied by -log2(e),
-// so a gate is rcp(1 + exp2(acc)).  tri_project_v2_kernel (partial tiles) carries TPW 16-row
-// tiles per wave, so with TPW = 2 every weight fragment read from LDS feeds two MFMAs; a wave
-// walks tiles w, w + nw, w + 2nw, ... TPW at a time, the last step running only the tiles it
-// has.  One tile per wave at 12 waves is what runs: two tiles need registers that leave two
-// waves per SIMD, measured slower.
+// The 128-wide kernels' gate weights and biases are pre-multiplied by -log2(e), so a gate is
+// rcp(1 + exp2(acc)).
 constexpr float TRI_NLOG2E = -1.4426950408889634f;
-// waves per block and 16-row tiles per wave of the 128-wide project kernels (16 waves spill)
-constexpr int TRI_P_NWV = 12, TRI_P_TPW = 1;
+// waves per block of the 128-wide project kernel (16 spill), one 16-row tile each (two tiles
+// need registers that leave two waves per SIMD, measured slower)
+constexpr int TRI_P_NWV = 12;
 // waves per block of the output kernel: 12 (three per SIMD, one X buffer each) for 2-byte
 // activations; f32 rows need more registers than three waves per SIMD leave, so 8 (two X
 // buffers each).  Measured at N = 384: 43.9 -> 39.9 us with 12 waves for bf16, while f32 at
@@ -965,154 +989,38 @@ constexpr int TRI_P_NWV = 12, TRI_P_TPW = 1;
 template <int ACT>
 constexpr int tri_o_nwv() { return ACT == DT_F32 ? 8 : 12; }
 
-// The 16 pairs of a project tile: row r is pair src0 + r * sstride, stored at out0 + r of every
-// channel plane, r < nvalid.  Tile t normally holds pairs 16t .. 16t + 15 in place.  With
-// kmajor_out (the incoming direction) tile t = j * ceil(N/16) + kb holds the pairs (16kb + r, j)
-// and stores them at j * N + 16kb + r: each plane then holds a^T (b^T), so the contraction
+// The 16 pairs of a 128-wide kernel's tile: up to 16 consecutive k of one plane row.  Row r is
+// pair src0 + r * sstride, r < nvalid, and sits at out0 + r of every channel plane.  Tile t is
+// piece kb of row j (t = j * ceil(N/16) + kb): pairs (j, 16kb + r), or, with kmajor_out (the
+// incoming direction), pairs (16kb + r, j): each plane then holds a^T (b^T), so the contraction
 // reads both operands with k contiguous, as in the outgoing direction.
+// Plane rows are padded to 16 (pitch ld), so a tile always stores 16 aligned columns, whatever
+// N is: with the pitch N, lengths that are not a multiple of 16 needed element-wise stores here,
+// element-wise transposes in the output kernel and an element-wise contraction (N = 825, f32:
+// 352 / 1697 / 303 us per direction for the three kernels against 214 / 258 / 192).
 struct TileGeom {
   int src0, sstride, out0, nvalid;
 };
 
-__device__ __forceinline__ TileGeom tile_geom(const TriProjectParams& p, int tile) {
-  if (!p.kmajor_out) {
-    const int r0 = tile * 16;
-    return TileGeom{r0, 1, r0, min(16, p.P - r0)};
-  }
-  const int nkb = (p.N + 15) >> 4, j = tile / nkb, kb = tile - j * nkb;
-  return TileGeom{kb * 16 * p.N + j, p.N, j * p.N + kb * 16, min(16, p.N - kb * 16)};
+// WHOLE: N a multiple of 16, every tile has 16 pairs (N = 384: the clamps and the division of a
+// partial tile's geometry cost 2%).
+template <bool WHOLE>
+__device__ __forceinline__ TileGeom tile_geom(int N, int ld, bool kmajor, int tile) {
+  if (WHOLE && !kmajor) return TileGeom{16 * tile, 1, 16 * tile, 16};
+  const int nkb = ld >> 4, j = tile / nkb, kb = tile - j * nkb;
+  const int nv = WHOLE ? 16 : min(16, N - kb * 16);
+  return kmajor ? TileGeom{kb * 16 * N + j, N, j * ld + kb * 16, nv}
+                : TileGeom{j * N + kb * 16, 1, j * ld + kb * 16, nv};
 }
 
-template <int ACT>
-__device__ __forceinline__ void tri_tile_load(FragTile<ACT, 4>& t, float (&m)[4], const TriProjectParams& p, int tile,
-                                              int lane) {
-  const TileGeom g = tile_geom(p, tile);
-  const int r16 = lane & 15, q4 = (lane >> 4) * 4;
-  frag_load_row(t, p.z, (size_t)g.src0 + (size_t)(r16 < g.nvalid ? r16 : 0) * g.sstride, 128, lane);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) m[i] = q4 + i < g.nvalid ? p.mask[g.src0 + (q4 + i) * g.sstride] : 0.f;
-}
-
-template <int ACT, int NWV, int TPW>
-__global__ __launch_bounds__(64 * NWV) void tri_project_v2_kernel(TriProjectParams p) {
-  constexpr int NT = 64 * NWV;
-  __shared__ __attribute__((aligned(16))) _Float16 Ws[4 * 128 * RS_LD];  // a-proj, a-gate', b-proj, b-gate' [h][k]
-  __shared__ __attribute__((aligned(16))) float Bs[4 * 128];              // the four bias vectors (gates scaled)
-  __shared__ __attribute__((aligned(16))) float Gs[2 * 128];              // LN_in scale, offset
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  stage_project_weights<NT>(Ws, p, tid);
-  for (int i = tid; i < 128; i += NT) {
-    Bs[i] = p.bp[0] ? p.bp[0][i] : 0.f;
-    Bs[128 + i] = p.bg[0] ? TRI_NLOG2E * p.bg[0][i] : 0.f;
-    Bs[256 + i] = p.bp[1] ? p.bp[1][i] : 0.f;
-    Bs[384 + i] = p.bg[1] ? TRI_NLOG2E * p.bg[1][i] : 0.f;
-  }
-  stage_vec(Gs, p.ln_s, 128, 1.f, 128, tid, NT);
-  stage_vec(Gs + 128, p.ln_o, 128, 0.f, 128, tid, NT);
-
-  const int r16 = lane & 15, g4 = lane >> 4, q4 = g4 * 4, kq = g4 * 8;
-  const int ntiles = p.kmajor_out ? p.N * ((p.N + 15) >> 4) : (p.P + 15) >> 4, nw = gridDim.x * NWV;
-  const bool vec_store = ((p.kmajor_out ? p.N : p.P) & 3) == 0;
-  int tile = blockIdx.x * NWV + wave;
-  FragTile<ACT, 4> t[TPW];
-  float mk[TPW][4];
-  if (tile < ntiles) {
-#pragma unroll
-    for (int tt = 0; tt < TPW; ++tt) tri_tile_load(t[tt], mk[tt], p, tile + tt * nw < ntiles ? tile + tt * nw : tile, lane);
-  }
-  __syncthreads();
-
-  for (; tile < ntiles; tile += TPW * nw) {
-    bool valid[TPW];
-    int out0[TPW], nval[TPW];
-#pragma unroll
-    for (int tt = 0; tt < TPW; ++tt) {
-      valid[tt] = tile + tt * nw < ntiles;   // wave-uniform
-      const TileGeom g = tile_geom(p, valid[tt] ? tile + tt * nw : tile);
-      out0[tt] = g.out0;
-      nval[tt] = g.nvalid;
-    }
-    h8 xa[TPW][4];
-    if constexpr (TPW == 2) frag_ln_raw2(t[0], t[1], xa[0], xa[1], 128, Gs, Gs + 128, p.eps, p.fast_var, lane);
-    else frag_ln_raw1(t[0], xa[0], 128, Gs, Gs + 128, p.eps, p.fast_var, lane);
-    float m[TPW][4];
-#pragma unroll
-    for (int tt = 0; tt < TPW; ++tt)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) m[tt][i] = mk[tt][i];
-    // loads of the next tiles are issued before this step's stores (one in-order counter)
-    const int nt = tile + TPW * nw;
-    if (nt < ntiles) {
-#pragma unroll
-      for (int tt = 0; tt < TPW; ++tt) tri_tile_load(t[tt], mk[tt], p, nt + tt * nw < ntiles ? nt + tt * nw : nt, lane);
-    }
-#pragma unroll 1
-    for (int pass = 0; pass < 4; ++pass) {
-      const int which = pass >> 1, hh = (pass & 1) * 64;
-      const _Float16* Wp = Ws + (which * 2) * 128 * RS_LD;
-      const _Float16* Wg = Wp + 128 * RS_LD;
-      const float* bp = Bs + which * 256 + hh;
-      const float* bg = bp + 128;
-      f4 acc[TPW][8];
-#pragma unroll
-      for (int t4 = 0; t4 < 4; ++t4) {
-        const float b0 = bp[t4 * 16 + r16], b1 = bg[t4 * 16 + r16];
-#pragma unroll
-        for (int tt = 0; tt < TPW; ++tt) {
-          acc[tt][t4] = f4{b0, b0, b0, b0};
-          acc[tt][4 + t4] = f4{b1, b1, b1, b1};
-        }
-      }
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        h8 wb[8];
-#pragma unroll
-        for (int t4 = 0; t4 < 4; ++t4) {
-          wb[t4] = *reinterpret_cast<const h8*>(Wp + (hh + t4 * 16 + r16) * RS_LD + 32 * j + kq);
-          wb[4 + t4] = *reinterpret_cast<const h8*>(Wg + (hh + t4 * 16 + r16) * RS_LD + 32 * j + kq);
-        }
-#pragma unroll
-        for (int tt = 0; tt < TPW; ++tt) {
-          if (tt > 0 && !valid[tt]) break;
-#pragma unroll
-          for (int u = 0; u < 8; ++u) acc[tt][u] = mfma16(xa[tt][j], wb[u], acc[tt][u]);
-        }
-        __builtin_amdgcn_sched_barrier(0);   // one k-step's weight fragments live at a time
-      }
-      _Float16* dst = which ? p.out[1] : p.out[0];
-#pragma unroll
-      for (int tt = 0; tt < TPW; ++tt) {
-        if (tt > 0 && !valid[tt]) break;
-        const int nvalid = nval[tt];
-#pragma unroll
-        for (int t4 = 0; t4 < 4; ++t4) {
-          const int h = hh + t4 * 16 + r16;
-          h4 o;
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            o[i] = (_Float16)(m[tt][i] * acc[tt][t4][i] *
-                              __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(acc[tt][4 + t4][i])));
-          _Float16* d = dst + (size_t)h * p.P + out0[tt] + q4;
-          if (vec_store && q4 + 4 <= nvalid) {
-            *reinterpret_cast<h4*>(d) = o;
-          } else {
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-              if (q4 + i < nvalid) d[i] = o[i];
-          }
-        }
-      }
-    }
-  }
-}
-
-// Project kernel for c_z = c_hidden = 128 when every tile is whole (P % 16 == 0, or N % 16 == 0
-// for the transposed incoming store): the v2 work as straight-line code.  The next tile's rows
-// and mask are loaded at the top of a step (clamped, never skipped), the four passes are
+// Project kernel for c_z = c_hidden = 128, straight-line code per 16-pair tile.  The next tile's
+// rows and mask are loaded at the top of a step (clamped, never skipped), the four passes are
 // unrolled, and the next rows are taken into registers (an asm use forces the wait) after the
 // last pass's MFMAs and before its stores: every wait on the in-order vector-memory counter
 // then covers loads issued earlier in the same step, never the stores that follow them.
-template <int ACT, int NWV, bool ST>
+// Rows past nvalid repeat the last one with a zero mask, which is what the planes' padding
+// holds.  OFS: the lane offset of a store, 32 bits while 16 planes span less than 4 GB.
+template <int ACT, int NWV, bool ST, bool WHOLE, typename OFS>
 __global__ __launch_bounds__(64 * NWV) void tri_project_v3_kernel(TriProjectParams p) {
   constexpr int NT = 64 * NWV;
   __shared__ __attribute__((aligned(16))) _Float16 Ws[4 * 128 * RS_LD];  // a-proj, a-gate', b-proj, b-gate' [h][k]
@@ -1123,18 +1031,18 @@ __global__ __launch_bounds__(64 * NWV) void tri_project_v3_kernel(TriProjectPara
   // A operand of the bias MFMA: ones at k = 0, 1 (lanes 0-15 supply k 0..3), zeros elsewhere
   const _Float16 one = (_Float16)(g4 == 0 ? 1.f : 0.f);
   const h4 ones = h4{one, one, (_Float16)0.f, (_Float16)0.f};
-  const int ntiles = p.kmajor_out ? p.N * (p.N >> 4) : p.P >> 4, nw = gridDim.x * NWV;
-  auto fetch = [&](int tl, FragTile<ACT, 4>& t, float (&m)[4]) __attribute__((always_inline)) {
-    const TileGeom g = tile_geom(p, tl);
-    frag_load_row(t, p.z, (size_t)g.src0 + (size_t)r16 * g.sstride, 128, lane);
+  const int ntiles = p.N * (p.ld >> 4), nw = gridDim.x * NWV;
+  auto fetch = [&](const TileGeom& g, FragTile<ACT, 4>& t, float (&m)[4]) __attribute__((always_inline)) {
+    frag_load_row(t, p.z, (size_t)g.src0 + (size_t)(WHOLE ? r16 : min(r16, g.nvalid - 1)) * g.sstride, 128, lane);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) m[i] = p.mask[g.src0 + (q4 + i) * g.sstride];
+    for (int i = 0; i < 4; ++i) m[i] = p.mask[g.src0 + (WHOLE ? q4 + i : min(q4 + i, g.nvalid - 1)) * g.sstride];
   };
   // the first tile's rows load while the weights are decoded into LDS (clamped, never skipped)
   int tile = blockIdx.x * NWV + wave;
   FragTile<ACT, 4> tc;
   float mc[4];
-  fetch(tile < ntiles ? tile : 0, tc, mc);
+  TileGeom tg = tile_geom<WHOLE>(p.N, p.ld, p.kmajor_out, tile < ntiles ? tile : 0);
+  fetch(tg, tc, mc);
   stage_project_weights<NT>(Ws, p, tid);
   // a bias b as the B operand of a 16x16x16 MFMA: k rows 0 and 1 hold hi = f16(b) and
   // lo = f16(b - hi), which the ones in the A operand sum back to b within 2^-22 relative
@@ -1152,24 +1060,25 @@ __global__ __launch_bounds__(64 * NWV) void tri_project_v3_kernel(TriProjectPara
   stage_vec(Gs + 128, p.ln_o, 128, 0.f, 128, tid, NT);
   __syncthreads();
   if (tile >= ntiles) return;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) mc[i] = WHOLE || q4 + i < tg.nvalid ? mc[i] : 0.f;
   for (; tile < ntiles; tile += nw) {
-    const TileGeom tg = tile_geom(p, tile);
-    const int out0 = tg.out0;
-    const uint32_t lofs = ((uint32_t)r16 * (uint32_t)p.P + (uint32_t)(out0 + q4)) * (uint32_t)sizeof(_Float16);
+    const OFS lofs = ((OFS)r16 * (OFS)p.plane + (OFS)(tg.out0 + q4)) * (OFS)sizeof(_Float16);
     h8 xa[4];
     if constexpr (ST) {
       float m0, i0;
       frag_stats_raw(tc, 128, p.eps, p.fast_var, m0, i0);
       // the output kernel normalises the same z rows again for its gate: it reads these
-      if (lane < 16) p.stats[tg.src0 + r16 * tg.sstride] = make_float2(m0, i0);
+      if (lane < 16) p.stats[tg.src0 + (WHOLE ? r16 : min(r16, tg.nvalid - 1)) * tg.sstride] = make_float2(m0, i0);
       frag_ln_given(tc, xa, Gs, Gs + 128, m0, i0, lane);
     } else {
       frag_ln_raw1(tc, xa, 128, Gs, Gs + 128, p.eps, p.fast_var, lane);
     }
     const int nt = tile + nw < ntiles ? tile + nw : tile;   // the last step reloads its own tile
+    const TileGeom tgn = tile_geom<WHOLE>(p.N, p.ld, p.kmajor_out, nt);
     FragTile<ACT, 4> tn;
     float mn[4];
-    fetch(nt, tn, mn);
+    fetch(tgn, tn, mn);
     auto pass = [&](auto pass_tag) __attribute__((always_inline)) {
       constexpr int PS = decltype(pass_tag)::value, which = PS >> 1, hh = (PS & 1) * 64;
       const _Float16* Wp = Ws + (which * 2) * 128 * RS_LD;
@@ -1198,8 +1107,8 @@ __global__ __launch_bounds__(64 * NWV) void tri_project_v3_kernel(TriProjectPara
         launder(tn);
         asm volatile("" : "+v"(mn[0]), "+v"(mn[1]), "+v"(mn[2]), "+v"(mn[3]));
       }
-      // a wave-uniform base per 16 channels plus one 32-bit lane offset (P < 2^27): scalar
-      // base + vector offset stores, no 64-bit address arithmetic per store
+      // a wave-uniform base per 16 channels plus one 32-bit lane offset (planes below 2^27
+      // elements): scalar base + vector offset stores, no 64-bit address arithmetic per store
       char* dst = reinterpret_cast<char*>(which ? p.out[1] : p.out[0]);
 #pragma unroll
       for (int t4 = 0; t4 < 4; ++t4) {
@@ -1207,7 +1116,7 @@ __global__ __launch_bounds__(64 * NWV) void tri_project_v3_kernel(TriProjectPara
 #pragma unroll
         for (int i = 0; i < 4; ++i)
           o[i] = (_Float16)(mc[i] * acc[t4][i] * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(acc[4 + t4][i])));
-        *reinterpret_cast<h4*>(dst + (size_t)(hh + t4 * 16) * p.P * sizeof(_Float16) + lofs) = o;
+        *reinterpret_cast<h4*>(dst + (size_t)(hh + t4 * 16) * p.plane * sizeof(_Float16) + lofs) = o;
       }
     };
     pass(std::integral_constant<int, 0>{});
@@ -1218,32 +1127,21 @@ __global__ __launch_bounds__(64 * NWV) void tri_project_v3_kernel(TriProjectPara
     __builtin_amdgcn_sched_barrier(0);
     pass(std::integral_constant<int, 3>{});
     tc = tn;
+    tg = tgn;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) mc[i] = mn[i];
+    for (int i = 0; i < 4; ++i) mc[i] = WHOLE || q4 + i < tgn.nvalid ? mn[i] : 0.f;
   }
 }
 
 constexpr int O2_LD = 136;   // X patch pitch (halves)
 
-// Xw[r][h] = X[h][row0 + r] for r < 16, element by element (rows past nvalid zero): the
-// path for partial tiles and for P % 8 != 0
-template <int ACT>
-__device__ __forceinline__ void x_transpose(_Float16* Xw, const _Float16* X, int P, int row0, int nvalid, int lane) {
-#pragma unroll 1
-  for (int idx = lane; idx < 128 * 16; idx += 64) {
-    const int h = idx >> 4, r = idx & 15;
-    const _Float16 v = X[(size_t)h * P + row0 + (r < nvalid ? r : 0)];
-    Xw[r * O2_LD + h] = r < nvalid ? v : (_Float16)0.f;
-  }
-}
-
-// x_transpose for a whole tile with P % 8 == 0, in two halves: the 16-byte global loads
-// (issued a tile ahead) and the transposing LDS stores.
-__device__ __forceinline__ void x_fetch(h8 (&xv)[4], const _Float16* X, int P, int row0, int lane) {
+// Xw[r][h] = X[h][x0 + r] for r < 16 (x0 a multiple of 16) in two halves: the 16-byte global
+// loads (issued a tile ahead) and the transposing LDS stores.
+__device__ __forceinline__ void x_fetch(h8 (&xv)[4], const _Float16* X, size_t plane, int x0, int lane) {
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const int idx = lane + 64 * j, h = idx >> 1, seg = idx & 1;
-    xv[j] = *reinterpret_cast<const h8*>(X + (size_t)h * P + row0 + seg * 8);
+    xv[j] = *reinterpret_cast<const h8*>(X + (size_t)h * plane + x0 + seg * 8);
   }
 }
 
@@ -1261,13 +1159,15 @@ __device__ __forceinline__ void x_put(_Float16* Xw, const h8 (&xv)[4], int lane)
 // (clamped, never skipped) at the top of a step and transposed into the wave's other LDS
 // buffer between the second pass's MFMAs and that pass's stores (two X buffers, 8 waves), or
 // loaded between the two passes and transposed after the tile into its one buffer (12 waves,
-// whose LDS and registers allow only that); the residual comes from the z rows already held.  Every wait on the in-order vector-memory counter then
-// covers loads issued earlier in the same step and none of the stores issued after them.  A
-// partial last tile (P % 16 pairs) runs once after the loop, masked, on the wave owning it.
+// whose LDS and registers allow only that); the residual comes from the z rows already held.
+// Every wait on the in-order vector-memory counter then covers loads issued earlier in the same
+// step and none of the stores issued after them.  In a tile with fewer than 16 pairs (the end of
+// a plane row) the lanes past its end repeat the last pair, loads, arithmetic and store: no
+// branch and no masked store.
 // The weights are the MFMA A operand (resident in LDS), so a lane's accumulators hold four
 // consecutive channels of one pair; the gate weights and bias arrive pre-multiplied by
 // -log2(e): sigmoid = rcp(1 + exp2(acc)).
-template <int ACT, int NWV, bool VECX, bool ZS>
+template <int ACT, int NWV, bool ZS, bool WHOLE>
 __global__ __launch_bounds__(64 * NWV) void tri_output_v3_kernel(TriOutputParams p) {
   constexpr int NT = 64 * NWV;
   // X patch buffers per wave: two (the next tile's X is transposed during the current tile's
@@ -1279,7 +1179,7 @@ __global__ __launch_bounds__(64 * NWV) void tri_output_v3_kernel(TriOutputParams
   __shared__ __attribute__((aligned(16))) _Float16 Xs[NWV][XB][16 * O2_LD];
   __shared__ __attribute__((aligned(16))) float Vs[6 * 128];         // bz, bg', centre-norm s/o, LN_in s/o
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int nfull = p.P >> 4, nw = gridDim.x * NWV;
+  const int ntiles = p.N * (p.ld >> 4), nw = gridDim.x * NWV;
   // the first tile's z rows and X columns load while the weights are decoded into LDS
   // (clamped, never skipped)
   int tile = blockIdx.x * NWV + wave;
@@ -1287,11 +1187,13 @@ __global__ __launch_bounds__(64 * NWV) void tri_output_v3_kernel(TriOutputParams
   FragTile<ACT, 4> zc;
   float2 zs = make_float2(0.f, 1.f);
   h8 xv[4];
+  TileGeom tg = tile_geom<WHOLE>(p.N, p.ld, false, tile < ntiles ? tile : 0);
+  // the lane's pair of a tile (its z row, statistics and output row)
+  auto pair_of = [&](const TileGeom& g) __attribute__((always_inline)) { return g.src0 + (WHOLE ? r16 : min(r16, g.nvalid - 1)); };
   {
-    const int t0 = tile < nfull ? tile : 0;
-    frag_load(zc, p.z, (size_t)t0 * 16, 16, 128, lane);
-    if constexpr (ZS) zs = p.stats[t0 * 16 + r16];
-    if constexpr (VECX) x_fetch(xv, p.X, p.P, t0 * 16, lane);
+    frag_load_row(zc, p.z, (size_t)pair_of(tg), 128, lane);
+    if constexpr (ZS) zs = p.stats[pair_of(tg)];
+    x_fetch(xv, p.X, p.plane, tg.out0, lane);
   }
   // the biases and LayerNorm vectors (threads 0-127, one channel each) are loaded before the
   // weights, so their round trip overlaps the weight stage's instead of following it
@@ -1319,14 +1221,15 @@ __global__ __launch_bounds__(64 * NWV) void tri_output_v3_kernel(TriOutputParams
   // channels.  A pass stages its f32 update in Xc (the X fragments are in registers by then)
   // and each lane writes its own pair r16, channels c0 + 32jj + 8*g4 .. +7: the layout of its
   // z fragment, which holds the residual.  `between` runs after the second pass's MFMAs.
-  auto run_tile = [&](auto full_tag, const FragTile<ACT, 4>& zc, float2 zs, _Float16* Xc, int row0, int nval,
-                      auto&& mid, auto&& between) __attribute__((always_inline)) {
-    constexpr bool FULL = decltype(full_tag)::value;
+  auto run_tile = [&](const FragTile<ACT, 4>& zc, float2 zs, _Float16* Xc, const TileGeom& g, auto&& mid,
+                      auto&& between) __attribute__((always_inline)) {
+    const size_t orow = (size_t)pair_of(g) * 128;
     h8 ax[4], az[4];
     {
       FragTile<DT_F16, 4> x;
+      const _Float16* xr = Xc + (WHOLE ? r16 : min(r16, g.nvalid - 1)) * O2_LD + kq;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) x.raw[j][0] = *reinterpret_cast<const u32x4*>(Xc + r16 * O2_LD + 32 * j + kq);
+      for (int j = 0; j < 4; ++j) x.raw[j][0] = *reinterpret_cast<const u32x4*>(xr + 32 * j);
       frag_ln_raw1(x, ax, 128, Vs + 256, Vs + 384, p.eps_x, p.fast_var, lane);
     }
     {
@@ -1385,12 +1288,10 @@ __global__ __launch_bounds__(64 * NWV) void tri_output_v3_kernel(TriOutputParams
 #pragma unroll
           for (int e = 0; e < 8; ++e) v[e] += zc.get(2 * PS + jj, e);
         }
-        const size_t idx = (size_t)(row0 + r16) * 128 + c0 + 32 * jj + 8 * g4;
+        const size_t idx = orow + c0 + 32 * jj + 8 * g4;
         const float lo[4] = {v[0], v[1], v[2], v[3]}, hi[4] = {v[4], v[5], v[6], v[7]};
-        if (FULL || r16 < nval) {
-          st4v<ACT>(p.out, idx, lo);
-          st4v<ACT>(p.out, idx + 4, hi);
-        }
+        st4v<ACT>(p.out, idx, lo);
+        st4v<ACT>(p.out, idx + 4, hi);
       }
     };
     pass(std::integral_constant<int, 0>{});
@@ -1400,65 +1301,52 @@ __global__ __launch_bounds__(64 * NWV) void tri_output_v3_kernel(TriOutputParams
     if constexpr (XB == 1) between();
   };
 
-  if (tile < nfull) {
-    if constexpr (VECX) {
-      x_put(Xs[wave][0], xv, lane);
-    } else {
-      x_transpose<ACT>(Xs[wave][0], p.X, p.P, tile * 16, 16, lane);
-    }
-    int cur = 0;
-    for (; tile < nfull; tile += nw) {
-      const int nt = tile + nw < nfull ? tile + nw : tile;   // the last step reloads its own tile
-      FragTile<ACT, 4> zn;
-      float2 zsn = zs;
-      h8 xn[4];
-      // the next tile's rows load at the top of the step (two X buffers), or between the two
-      // passes (one buffer: fewer registers live through the first pass)
-      auto fetch_next = [&]() __attribute__((always_inline)) {
-        frag_load(zn, p.z, (size_t)nt * 16, 16, 128, lane);
-        if constexpr (ZS) zsn = p.stats[nt * 16 + r16];
-        if constexpr (VECX) x_fetch(xn, p.X, p.P, nt * 16, lane);
-      };
-      if constexpr (XB == 2) fetch_next();
-      _Float16* Xn = Xs[wave][XB == 2 ? cur ^ 1 : 0];
-      run_tile(std::true_type{}, zc, zs, Xs[wave][XB == 2 ? cur : 0], tile * 16, 16, [&]() __attribute__((always_inline)) {
-        if constexpr (XB == 1) fetch_next();
-      }, [&]() __attribute__((always_inline)) {
-        if constexpr (VECX) x_put(Xn, xn, lane);
-        else x_transpose<ACT>(Xn, p.X, p.P, nt * 16, 16, lane);
-      });
-      // take the next rows now (an asm use forces the wait here, within this step, where the
-      // counter wait cannot cover this step's stores), not at their first use next step
-      launder(zn);
-      if constexpr (ZS) asm volatile("" : "+v"(zsn.x), "+v"(zsn.y));
-      zc = zn;
-      zs = zsn;
-      if constexpr (XB == 2) cur ^= 1;
-    }
-  }
-  if (tile == nfull && nfull * 16 < p.P) {
-    const int row0 = nfull * 16, nval = p.P - row0;
-    FragTile<ACT, 4> zc;
-    frag_load(zc, p.z, (size_t)row0, nval, 128, lane);
-    const float2 zt = ZS ? p.stats[row0 + (r16 < nval ? r16 : 0)] : make_float2(0.f, 1.f);
-    x_transpose<ACT>(Xs[wave][0], p.X, p.P, row0, nval, lane);
-    run_tile(std::false_type{}, zc, zt, Xs[wave][0], row0, nval, []() {}, []() {});
+  if (tile >= ntiles) return;
+  x_put(Xs[wave][0], xv, lane);
+  int cur = 0;
+  for (; tile < ntiles; tile += nw) {
+    const int nt = tile + nw < ntiles ? tile + nw : tile;   // the last step reloads its own tile
+    const TileGeom tgn = tile_geom<WHOLE>(p.N, p.ld, false, nt);
+    FragTile<ACT, 4> zn;
+    float2 zsn = zs;
+    h8 xn[4];
+    // the next tile's rows load at the top of the step (two X buffers), or between the two
+    // passes (one buffer: fewer registers live through the first pass)
+    auto fetch_next = [&]() __attribute__((always_inline)) {
+      frag_load_row(zn, p.z, (size_t)pair_of(tgn), 128, lane);
+      if constexpr (ZS) zsn = p.stats[pair_of(tgn)];
+      x_fetch(xn, p.X, p.plane, tgn.out0, lane);
+    };
+    if constexpr (XB == 2) fetch_next();
+    _Float16* Xn = Xs[wave][XB == 2 ? cur ^ 1 : 0];
+    run_tile(zc, zs, Xs[wave][XB == 2 ? cur : 0], tg, [&]() __attribute__((always_inline)) {
+      if constexpr (XB == 1) fetch_next();
+    }, [&]() __attribute__((always_inline)) { x_put(Xn, xn, lane); });
+    // take the next rows now (an asm use forces the wait here, within this step, where the
+    // counter wait cannot cover this step's stores), not at their first use next step
+    launder(zn);
+    if constexpr (ZS) asm volatile("" : "+v"(zsn.x), "+v"(zsn.y));
+    zc = zn;
+    zs = zsn;
+    tg = tgn;
+    if constexpr (XB == 2) cur ^= 1;
   }
 }
 
 template <int ACT>
 static void launch_project(lf_context* ctx, const TriProjectParams& pp, bool resident, int kz) {
   const int P = pp.P;
-  if (resident && pp.C == 128 && pp.H == 128) {
-    const int tiles = (P + 15) / 16;
+  if (pp.ld) {   // the 128-wide kernel
+    const int tiles = pp.N * (pp.ld / 16);
     dim3 g(std::max(1, std::min(ctx->num_cus, (tiles + TRI_P_NWV - 1) / TRI_P_NWV)));
-    const bool whole = pp.kmajor_out ? pp.N % 16 == 0 : P % 16 == 0;
-    if (whole && P < (1 << 27) && pp.stats)   // 32-bit per-lane store offsets
-      hipLaunchKernelGGL((tri_project_v3_kernel<ACT, TRI_P_NWV, true>), g, dim3(64 * TRI_P_NWV), 0, ctx->stream, pp);
-    else if (whole && P < (1 << 27))
-      hipLaunchKernelGGL((tri_project_v3_kernel<ACT, TRI_P_NWV, false>), g, dim3(64 * TRI_P_NWV), 0, ctx->stream, pp);
+    const dim3 b(64 * TRI_P_NWV);
+    constexpr bool ST = ACT != DT_F32;
+    if (pp.plane >= (size_t)1 << 27)   // 64-bit store offsets
+      hipLaunchKernelGGL((tri_project_v3_kernel<ACT, TRI_P_NWV, ST, false, uint64_t>), g, b, 0, ctx->stream, pp);
+    else if (pp.N % 16 == 0)
+      hipLaunchKernelGGL((tri_project_v3_kernel<ACT, TRI_P_NWV, ST, true, uint32_t>), g, b, 0, ctx->stream, pp);
     else
-      hipLaunchKernelGGL((tri_project_v2_kernel<ACT, TRI_P_NWV, TRI_P_TPW>), g, dim3(64 * TRI_P_NWV), 0, ctx->stream, pp);
+      hipLaunchKernelGGL((tri_project_v3_kernel<ACT, TRI_P_NWV, ST, false, uint32_t>), g, b, 0, ctx->stream, pp);
     return;
   }
   if (resident) {
@@ -1476,19 +1364,14 @@ static void launch_project(lf_context* ctx, const TriProjectParams& pp, bool res
 template <int ACT>
 static void launch_output(lf_context* ctx, const TriOutputParams& op, bool resident, int kz, int kh) {
   const int P = op.P;
-  if (resident && op.C == 128 && op.H == 128) {
+  if (op.ld) {   // the 128-wide kernel; the z statistics of 2-byte activations come from the project kernel
     constexpr int NWV = tri_o_nwv<ACT>();
-    const int tiles = (P + 15) / 16;
+    const int tiles = op.N * (op.ld / 16);
     dim3 g(std::max(1, std::min(ctx->num_cus, (tiles + NWV - 1) / NWV)));
-    // the z statistics come from the project kernel when it stored them (op.stats)
-    if ((P & 7) == 0 && op.stats)
-      hipLaunchKernelGGL((tri_output_v3_kernel<ACT, NWV, true, true>), g, dim3(64 * NWV), 0, ctx->stream, op);
-    else if ((P & 7) == 0)
-      hipLaunchKernelGGL((tri_output_v3_kernel<ACT, NWV, true, false>), g, dim3(64 * NWV), 0, ctx->stream, op);
-    else if (op.stats)
-      hipLaunchKernelGGL((tri_output_v3_kernel<ACT, NWV, false, true>), g, dim3(64 * NWV), 0, ctx->stream, op);
+    if (op.N % 16 == 0)
+      hipLaunchKernelGGL((tri_output_v3_kernel<ACT, NWV, ACT != DT_F32, true>), g, dim3(64 * NWV), 0, ctx->stream, op);
     else
-      hipLaunchKernelGGL((tri_output_v3_kernel<ACT, NWV, false, false>), g, dim3(64 * NWV), 0, ctx->stream, op);
+      hipLaunchKernelGGL((tri_output_v3_kernel<ACT, NWV, ACT != DT_F32, false>), g, dim3(64 * NWV), 0, ctx->stream, op);
     return;
   }
   if (resident) {
@@ -1566,28 +1449,35 @@ static int tri_mult_impl(lf_context* ctx, const lf_tri_mult_args& a, void* scrat
   LF_TRY(make_view(w.wz, H, C, "linearZWeight", &views[4]));
   LF_TRY(make_view(w.wg, C, C, "linearGWeight", &views[5]));
 
-  // the 128-wide project kernel for whole 16-pair tiles (32-bit per-lane store offsets) also
-  // stores each pair's LN_in statistics for the output kernel, for 16-bit activations; with
-  // f32 activations the hand-over measured neutral (output kernel -3%, project kernel +3%:
-  // its f32 tiles leave less room to hide the extra store), so f32 recomputes them
+  // the 128-wide kernels: channel planes of N rows padded to 16 (pitch ld), and for 16-bit
+  // activations each pair's LN_in statistics handed from the project kernel to the output
+  // kernel; with f32 activations the hand-over measured neutral (output kernel -3%, project
+  // kernel +3%: its f32 tiles leave less room to hide the extra store), so f32 recomputes them
   const bool wide = C == 128 && H == 128 && N >= 16;
-  const bool v3 = wide && a.act_dtype != LF_F32 && (a.direction != LF_OUTGOING ? N % 16 == 0 : P % 16 == 0) &&
-                  P < (1 << 27);
-  const size_t plane = (size_t)H * P * sizeof(_Float16);
-  size_t sizes[4] = {plane, plane, plane, v3 ? (size_t)P * sizeof(float2) : 0};
+  const bool hand = wide && a.act_dtype != LF_F32;
+  const int ld = wide ? (N + 15) & ~15 : N;
+  const size_t plane = (size_t)H * N * ld * sizeof(_Float16), stats = hand ? (size_t)P * sizeof(float2) : 0;
+  size_t sizes[4] = {plane, plane, plane, stats};
   void* bufs[4] = {};
-  const int nbufs = v3 ? 4 : 3;
+  const int nbufs = hand ? 4 : 3;
   if (scratch) {
+    // What is accepted is the documented size: the unpadded planes, and the statistics where
+    // whole 16-pair tiles hand them over.  The padding and the other statistics lie in the
+    // array's slack.
+    auto up = [](size_t b) { return (b + 255) & ~size_t(255); };
+    const bool whole = a.direction != LF_OUTGOING ? N % 16 == 0 : P % 16 == 0;
+    const size_t need = 3 * up((size_t)H * P * sizeof(_Float16)) + (hand && whole ? up(stats) : 0);
+    if (need > LF_TRI_NOALLOC_SCRATCH_BYTES)
+      return set_error(LF_ERR_INVALID, "tri_mult_noalloc: N=" + std::to_string(N) + ", c_hidden=" +
+                                           std::to_string(H) + " needs " + std::to_string(need) +
+                                           " bytes of scratch; the static scratch holds " +
+                                           std::to_string(LF_TRI_NOALLOC_SCRATCH_BYTES));
     size_t total = 0;
     for (int i = 0; i < nbufs; ++i) {
       bufs[i] = static_cast<char*>(scratch) + total;
-      total += (sizes[i] + 255) & ~size_t(255);
+      total += up(sizes[i]);
     }
-    if (total > scratch_cap)
-      return set_error(LF_ERR_INVALID, "tri_mult_noalloc: N=" + std::to_string(N) + ", c_hidden=" +
-                                           std::to_string(H) + " needs " + std::to_string(total) +
-                                           " bytes of scratch; the static scratch holds " +
-                                           std::to_string(scratch_cap));
+    if (total > scratch_cap) return set_error(LF_ERR_INVALID, "tri_mult_noalloc: static scratch too small");
   } else {
     LF_TRY(workspace(ctx, sizes, bufs, nbufs));
   }
@@ -1597,10 +1487,12 @@ static int tri_mult_impl(lf_context* ctx, const lf_tri_mult_args& a, void* scrat
   _Float16* X = static_cast<_Float16*>(bufs[2]);
   WSrc ex[6];
   // the 128-wide project kernel takes its gate weights pre-multiplied by -log2(e)
-  const bool v2 = C == 128 && H == 128 && N >= 16;
+  const float gate = wide ? TRI_NLOG2E : 1.f;
   // incoming: the 128-wide project kernel stores a and b transposed per channel
-  pp.kmajor_out = v2 && a.direction != LF_OUTGOING;
-  const float gate = v2 ? TRI_NLOG2E : 1.f;
+  pp.kmajor_out = wide && a.direction != LF_OUTGOING;
+  pp.ld = op.ld = wide ? ld : 0;
+  pp.plane = op.plane = (size_t)N * ld;
+  op.N = N;
   for (int i = 0; i < 6; ++i) ex[i] = wsrc(views[i], i % 2 ? gate : 1.f);
   pp.wp[0] = ex[0];
   pp.wg[0] = ex[1];
@@ -1633,6 +1525,7 @@ static int tri_mult_impl(lf_context* ctx, const lf_tri_mult_args& a, void* scrat
   const float scale = std::ldexp(1.0f, -sexp);
   TriContractParams cp{};
   cp.N = N;
+  cp.ld = ld;
   cp.scale = scale;
   cp.X = X;
   const bool outgoing = a.direction == LF_OUTGOING;
@@ -1679,7 +1572,10 @@ int tri_mult(lf_context* ctx, const lf_tri_mult_args& a) { return tri_mult_impl(
 // its own copy at its own address, looked up once per device (with that device current) by
 // tri_noalloc_init, which lf_context_create calls; host code only ever passes that address,
 // never the array's name, which on the host is a stand-in and not a device address.
-static __device__ __align__(256) unsigned char scratch[LF_TRI_NOALLOC_SCRATCH_BYTES];
+// Beyond the documented size it holds the plane rows' padding to 16 and the LayerNorm statistics:
+// at most 5.3 MiB over the shapes accepted (N = 417: 3 * 128 * 417 * 432 f16 and 8 * 417^2).
+constexpr size_t TRI_NOALLOC_BYTES = (size_t)LF_TRI_NOALLOC_SCRATCH_BYTES + ((size_t)6 << 20);
+static __device__ __align__(256) unsigned char scratch[TRI_NOALLOC_BYTES];
 
 namespace {
 constexpr int kMaxDevices = 64;
@@ -1705,7 +1601,7 @@ int tri_mult_noalloc(lf_context* ctx, const lf_tri_mult_args& a) {
     std::lock_guard<std::mutex> lock(g_scratch_mu);
     p = g_scratch_ptr[ctx->device];
   }
-  return tri_mult_impl(ctx, a, p, LF_TRI_NOALLOC_SCRATCH_BYTES);
+  return tri_mult_impl(ctx, a, p, TRI_NOALLOC_BYTES);
 }
 
 }  // namespace lf

@@ -90,6 +90,29 @@ def test_af3_dialect(ctx, direction, divide, n):
     H.assert_close(out, ref, label=f"af3/{direction}/{divide}")
 
 
+@pytest.mark.parametrize("n,direction,act", [
+    (16, "outgoing", "bfloat16"), (17, "incoming", "bfloat16"), (31, "outgoing", "float32"),
+    (33, "incoming", "float16"), (65, "outgoing", "float16"), (79, "incoming", "float32"),
+    (100, "outgoing", "bfloat16"), (191, "incoming", "bfloat16"), (901, "incoming", "float32")])
+def test_padded_plane_rows(ctx, n, direction, act):
+    """Lengths on both sides of a multiple of 16 and of 64: the channel planes' rows padded to 16,
+    tiles with 1 to 16 pairs, a last K step that ends inside and at its end (N = 901: on the
+    256-row tiles), the handed-over statistics of 2-byte activations, an update added in place."""
+    import torch
+    from localfold_amd import device as D
+    inp = S.deterministic_triangle_input(n, 128, 128, 100 + n)
+    dw = D.DeviceWeights(ctx.device)
+    ws = D.tri_mult_weights(dw, inp["weights"])
+    z = torch.as_tensor(inp["z"]).to(ctx.device).to(getattr(torch, act))
+    zin = z.float().cpu().numpy()
+    m = torch.as_tensor(np.asarray(inp["mask"], np.float32)).to(ctx.device)
+    D.tri_mult(ctx, z, m, ws, direction, out=z, accumulate=True)
+    torch.cuda.synchronize()
+    ref = zin + ops.tri_mult_af2(zin, inp["mask"], inp["weights"], direction)
+    # |z + update| < 4 here: storing it rounds by at most 2^-8 (bf16) or 2^-11 (f16) of 4
+    H.assert_close(z.float().cpu().numpy(), ref, max_abs=2e-2, label=f"padded {n}/{direction}/{act}")
+
+
 def test_af3_dialect_large_contraction_tiles(ctx):
     """AF3 at N = 768 (incoming, divided by the length, bf16 pair): the split projection of
     the interleaved tensors feeding the 256 x 256-tile contraction; against the oracle."""
