@@ -21,10 +21,10 @@ namespace lf {
 // The outer products: O[(i*N + j)][a*co + b] = sum_s L[i][a][s] R[j][b][s], i.e. the NT GEMM
 // (N*co) x (N*co) x S of the rows m = i*co + a and n = j*co + b, stored pair-major f16.
 struct OuterParams {
-  const _Float16* L;   // [N*co][S]
+  const _Float16* L;   // [N*co][S]; the 256-row tiles read past N*co to the next whole tile
   const _Float16* R;   // [N*co][S]
   _Float16* O;         // [N*N][co*co]
-  int N, co, S;
+  int N, co, S;        // S: the sequences rounded up to 8 (the padding holds zeros)
 };
 
 constexpr int OT = 128, OT_BK = 64, OT_LD = OT_BK + 8;
@@ -35,17 +35,11 @@ struct OtRegs {
 
 // [128 rows][64 k] of a sequence-contiguous operand: global -> registers (issued a K step
 // ahead) -> LDS.  Rows past M and k past S read as zero.
-__device__ __forceinline__ void ot_fetch(OtRegs& r, const _Float16* src, int M, int S, int m0, int k0, int tid,
-                                         bool vec) {
+__device__ __forceinline__ void ot_fetch(OtRegs& r, const _Float16* src, int M, int S, int m0, int k0, int tid) {
 #pragma unroll
   for (int it = 0; it < 4; ++it) {
     const int e = tid + it * 256, m = m0 + (e >> 3), k = k0 + (e & 7) * 8;
-    if (vec) {
-      r.v[it] = (m < M && k < S) ? *reinterpret_cast<const h8*>(src + (size_t)m * S + k) : h8{0, 0, 0, 0, 0, 0, 0, 0};
-    } else {
-#pragma unroll
-      for (int u = 0; u < 8; ++u) r.v[it][u] = (m < M && k + u < S) ? src[(size_t)m * S + k + u] : (_Float16)0.f;
-    }
+    r.v[it] = (m < M && k < S) ? *reinterpret_cast<const h8*>(src + (size_t)m * S + k) : h8{0, 0, 0, 0, 0, 0, 0, 0};
   }
 }
 
@@ -90,7 +84,6 @@ __global__ __launch_bounds__(256) void opm_outer_kernel(OuterParams p) {
     nt = lin % tm;
   }
   const int m0 = mt * OT, n0 = nt * OT;
-  const bool vec = (p.S & 7) == 0;
   f4 acc[4][4];
   zero_acc(acc);
   const int r16 = lane & 15, g4 = lane >> 4, kq = g4 * 8;
@@ -107,8 +100,8 @@ __global__ __launch_bounds__(256) void opm_outer_kernel(OuterParams p) {
         rb.v[it] = *reinterpret_cast<const h8*>(pb + it * rstep + k0);
       }
     } else {
-      ot_fetch(ra, p.L, M, p.S, m0, k0, tid, vec);
-      ot_fetch(rb, p.R, M, p.S, n0, k0, tid, vec);
+      ot_fetch(ra, p.L, M, p.S, m0, k0, tid);
+      ot_fetch(rb, p.R, M, p.S, n0, k0, tid);
     }
   };
   // one barrier per K step: the next step's tiles are fetched before this step's MFMAs and
@@ -166,31 +159,25 @@ __global__ __launch_bounds__(256) void opm_outer_kernel(OuterParams p) {
 constexpr int OB = 256;
 constexpr size_t OB_SMEM = (size_t)2 * 2 * OB * OT_LD * sizeof(_Float16);   // 147,456 bytes
 
-// The XCD band order of the 256-tile grid: tile (mt, nt) of block blockIdx.x.
+// The XCD band order of the 256-tile grid: tile (mt, nt) of block blockIdx.x.  The tiles are
+// numbered in bands of G = ceil(tm / 8) tile rows, column by column within a band, and each XCD
+// (block ids are dealt round-robin over 8) takes a contiguous eighth of the numbers: about one
+// band, whose L tiles stay in its L2 while each R tile is read once.
 __device__ __forceinline__ void opm_big_order(const OuterParams& p, int& mt, int& nt) {
-  const int M = p.N * p.co, tm = M / OB;
-  const int total = (int)gridDim.x, per = total >> 3;
-  const int lin = (int)blockIdx.x;
-  if (lin < per * 8) {
-    const int x = lin & 7, q = lin >> 3;
-    if (per % tm == 0) {
-      const int rows = per / tm;
-      mt = x * rows + q % rows;
-      nt = q / rows;
-    } else {
-      const int t = x * per + q;
-      mt = t / tm;
-      nt = t % tm;
-    }
-  } else {
-    mt = lin / tm;
-    nt = lin % tm;
-  }
+  const int tm = (p.N * p.co + OB - 1) / OB, G = (tm + 7) >> 3;
+  const int per = (int)gridDim.x >> 3;
+  int t = (int)blockIdx.x;
+  if (t < per * 8) t = (t & 7) * per + (t >> 3);
+  const int band = t / (G * tm), w = t - band * G * tm, rows = min(G, tm - band * G);
+  nt = w / rows;
+  mt = band * G + w - nt * rows;
 }
 
 // The 256x256 tile at (m0, n0) accumulated into acc: lane holds rows m0 + wm*128 + 16i + r16,
 // columns n0 + wn*64 + 16j + 4g4 + u (wm = wave / 4, wn = wave % 4).  Ends after a barrier,
-// so the caller may reuse the LDS.
+// so the caller may reuse the LDS.  TAIL: S is not a multiple of the K step: the pieces past it
+// are loaded from k = 0 and stored as zeros.
+template <bool TAIL>
 __device__ __forceinline__ void opm_big_tile(const OuterParams& p, int m0, int n0, f4 (&acc)[8][4], _Float16* obs) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 2, wn = wave & 3;
@@ -202,20 +189,22 @@ __device__ __forceinline__ void opm_big_tile(const OuterParams& p, int m0, int n
   const size_t rstep = (size_t)64 * p.S;
   h8 ra[4], rb[4];
   auto fetch = [&](int k0) __attribute__((always_inline)) {
+    const int ko = !TAIL || k0 + (tid & 7) * 8 < p.S ? k0 : -(tid & 7) * 8;
 #pragma unroll
     for (int it = 0; it < 4; ++it) {
-      ra[it] = *reinterpret_cast<const h8*>(pa + it * rstep + k0);
-      rb[it] = *reinterpret_cast<const h8*>(pb + it * rstep + k0);
+      ra[it] = *reinterpret_cast<const h8*>(pa + it * rstep + ko);
+      rb[it] = *reinterpret_cast<const h8*>(pb + it * rstep + ko);
     }
   };
-  auto put = [&](int buf) __attribute__((always_inline)) {
+  auto put = [&](int buf, int k0) __attribute__((always_inline)) {
     _Float16* A = obs + buf * STAGE;
     _Float16* B = A + OB * OT_LD;
+    const bool in = !TAIL || k0 + (tid & 7) * 8 < p.S;
 #pragma unroll
     for (int it = 0; it < 4; ++it) {
       const int r = (tid >> 3) + 64 * it, c = (tid & 7) * 8;
-      *reinterpret_cast<h8*>(A + r * OT_LD + c) = ra[it];
-      *reinterpret_cast<h8*>(B + r * OT_LD + c) = rb[it];
+      *reinterpret_cast<h8*>(A + r * OT_LD + c) = in ? ra[it] : h8{0, 0, 0, 0, 0, 0, 0, 0};
+      *reinterpret_cast<h8*>(B + r * OT_LD + c) = in ? rb[it] : h8{0, 0, 0, 0, 0, 0, 0, 0};
     }
   };
 #pragma unroll
@@ -223,7 +212,7 @@ __device__ __forceinline__ void opm_big_tile(const OuterParams& p, int m0, int n
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] = f4{0.f, 0.f, 0.f, 0.f};
   fetch(0);
-  put(0);
+  put(0, 0);
   __syncthreads();
   for (int k0 = 0, kb = 0; k0 < p.S; k0 += OT_BK, kb ^= 1) {
     const bool more = k0 + OT_BK < p.S;
@@ -249,7 +238,7 @@ __device__ __forceinline__ void opm_big_tile(const OuterParams& p, int m0, int n
         acur = anext;
       }
     }
-    if (more) put(kb ^ 1);
+    if (more) put(kb ^ 1, k0 + OT_BK);
     __syncthreads();
   }
 }
@@ -267,7 +256,7 @@ __global__ __launch_bounds__(512) void opm_outer_big_kernel(OuterParams p) {
   opm_big_order(p, mt, nt);
   const int m0 = mt * OB, n0 = nt * OB;
   f4 acc[8][4];
-  opm_big_tile(p, m0, n0, acc, obs);
+  opm_big_tile<false>(p, m0, n0, acc, obs);
   const unsigned co = (unsigned)p.co;
   const long long cc = (long long)p.co * p.co;
   long long colpart[4];
@@ -309,7 +298,7 @@ struct OpmFusedParams {
   void* out;
 };
 
-template <int ACT>
+template <int ACT, bool TAIL>
 __global__ __launch_bounds__(512) void opm_fused_kernel(OpmFusedParams f) {
   extern __shared__ __attribute__((aligned(16))) _Float16 obs[];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -323,15 +312,15 @@ __global__ __launch_bounds__(512) void opm_fused_kernel(OpmFusedParams f) {
   float inv[4], res[4][4];
 #pragma unroll
   for (int pt = 0; pt < 4; ++pt) {
-    const int pl = pt * 16 + r16;
-    const size_t row = (size_t)(mt * 8 + (pl >> 3)) * N + nt * 8 + (pl & 7);
+    const int pl = pt * 16 + r16;   // (residues past N in an edge tile: clamped here, not stored)
+    const size_t row = (size_t)min(mt * 8 + (pl >> 3), N - 1) * N + min(nt * 8 + (pl & 7), N - 1);
     inv[pt] = f.den[row];
     if (f.resid) ld4v<ACT>(f.resid, row * 128 + c, res[pt]);
     else res[pt][0] = res[pt][1] = res[pt][2] = res[pt][3] = 0.f;
   }
   {
     f4 acc[8][4];
-    opm_big_tile(f.o, mt * OB, nt * OB, acc, obs);
+    opm_big_tile<TAIL>(f.o, mt * OB, nt * OB, acc, obs);
     // tile row wm*128 + 16i + r16 = (residue, a), column wn*64 + 16j + 4g4 + u = (residue, b)
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
@@ -381,39 +370,44 @@ __global__ __launch_bounds__(512) void opm_fused_kernel(OpmFusedParams f) {
   for (int i = 0; i < 4; ++i) bias[i] = f.bias ? f.bias[c + i] : 0.f;
 #pragma unroll
   for (int pt = 0; pt < 4; ++pt) {
-    const int pl = pt * 16 + r16;
-    const size_t row = (size_t)(mt * 8 + (pl >> 3)) * N + nt * 8 + (pl & 7);
+    const int pl = pt * 16 + r16, i = mt * 8 + (pl >> 3), j = nt * 8 + (pl & 7);
+    if (i >= N || j >= N) continue;
+    const size_t row = (size_t)i * N + j;
     const float rinv = 1.f / inv[pt];
     float v[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] = (d[pt][i] + bias[i]) * rinv + res[pt][i];
+    for (int u = 0; u < 4; ++u) v[u] = (d[pt][u] + bias[u]) * rinv + res[pt][u];
     st4v<ACT>(f.out, row * 128 + c, v);
   }
 }
 
-// den[i*N + j] = eps + sum_s m[s][i] m[s][j]: a 16x16 tile per block, one output per thread
-// (N = 384 gives 576 blocks), the mask columns staged through LDS 64 sequences at a time
-// (reads of a staged row are broadcasts or conflict-free); sums run in sequence order.
-constexpr int CT_S = 64;
+// den[i*N + j] = eps + sum_s m[s][i] m[s][j]: a 16x16 tile per block (N = 384 gives 576 blocks),
+// the mask columns staged through LDS 256 sequences at a time (reads of a staged row are
+// broadcasts or conflict-free).  Four threads share an output, 64 of the staged sequences each:
+// with one thread per output the serial sum bound it (N = 301, S = 508: 23.5 -> 14.7 us).
+constexpr int CT_S = 256;
 
-__global__ __launch_bounds__(256) void opm_count_kernel(const float* mask, float* den, int S, int N, float eps) {
-  __shared__ float Mi[CT_S][16], Mj[CT_S][16];
-  const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
+__global__ __launch_bounds__(1024) void opm_count_kernel(const float* mask, float* den, int S, int N, float eps) {
+  __shared__ float Mi[CT_S][16], Mj[CT_S][16], part[4][256];
+  const int tid = threadIdx.x, t = tid & 255, grp = tid >> 8, tx = t & 15, ty = t >> 4;
   const int i0 = blockIdx.y * 16, j0 = blockIdx.x * 16;
   float acc = 0.f;
   for (int s0 = 0; s0 < S; s0 += CT_S) {
-    for (int e = tid; e < CT_S * 16; e += 256) {
+#pragma unroll
+    for (int e = tid; e < CT_S * 16; e += 1024) {
       const int ss = e >> 4, c = e & 15, sg = s0 + ss;
       Mi[ss][c] = (sg < S && i0 + c < N) ? mask[(size_t)sg * N + i0 + c] : 0.f;
       Mj[ss][c] = (sg < S && j0 + c < N) ? mask[(size_t)sg * N + j0 + c] : 0.f;
     }
     __syncthreads();
 #pragma unroll 16
-    for (int ss = 0; ss < CT_S; ++ss) acc = fmaf(Mi[ss][ty], Mj[ss][tx], acc);
+    for (int ss = 64 * grp; ss < 64 * grp + 64; ++ss) acc = fmaf(Mi[ss][ty], Mj[ss][tx], acc);
     __syncthreads();
   }
+  part[grp][t] = acc;
+  __syncthreads();
   const int i = i0 + ty, j = j0 + tx;
-  if (i < N && j < N) den[(size_t)i * N + j] = eps + acc;
+  if (grp == 0 && i < N && j < N) den[(size_t)i * N + j] = eps + ((part[0][t] + part[1][t]) + (part[2][t] + part[3][t]));
 }
 
 // The big kernels' dynamic LDS (above the 64 KB default) is opted into once per process.
@@ -422,9 +416,12 @@ static bool big_smem_ok(lf_context*) {
     return hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)OB_SMEM) == hipSuccess;
   };
   static const bool ok = opt(reinterpret_cast<const void*>(opm_outer_big_kernel)) &&
-                         opt(reinterpret_cast<const void*>(opm_fused_kernel<DT_F32>)) &&
-                         opt(reinterpret_cast<const void*>(opm_fused_kernel<DT_F16>)) &&
-                         opt(reinterpret_cast<const void*>(opm_fused_kernel<DT_BF16>));
+                         opt(reinterpret_cast<const void*>(opm_fused_kernel<DT_F32, false>)) &&
+                         opt(reinterpret_cast<const void*>(opm_fused_kernel<DT_F32, true>)) &&
+                         opt(reinterpret_cast<const void*>(opm_fused_kernel<DT_F16, false>)) &&
+                         opt(reinterpret_cast<const void*>(opm_fused_kernel<DT_F16, true>)) &&
+                         opt(reinterpret_cast<const void*>(opm_fused_kernel<DT_BF16, false>)) &&
+                         opt(reinterpret_cast<const void*>(opm_fused_kernel<DT_BF16, true>));
   return ok;
 }
 
@@ -440,7 +437,7 @@ int outer_product_mean(lf_context* ctx, const lf_opm_args& a) {
   LF_REQUIRE(a.epsilon > 0.f && a.norm_epsilon > 0.f, "outer product mean: epsilons must be positive");
   const lf_opm_weights& w = *a.w;
   const int S = a.sequences, N = a.length, co = a.c_outer, cz = a.c_z;
-  const long long pairs = (long long)N * N, rows = (long long)S * N;
+  const long long pairs = (long long)N * N;
   WView views[3];
   LF_TRY(make_view(w.wl, a.c_m, co, "leftWeight", &views[0]));
   LF_TRY(make_view(w.wr, a.c_m, co, "rightWeight", &views[1]));
@@ -448,12 +445,18 @@ int outer_product_mean(lf_context* ctx, const lf_opm_args& a) {
   // l, r = mask * (LN(msa) W + b), stored [i][a][s]
   LnProjParams pp{};
   pp.x = a.msa;
-  pp.rows = (int)rows;
   pp.C = a.c_m;
-  // logical row r = i*S + s reads MSA row s*N + i, so a wave's rows are consecutive sequences
-  // of one residue: 16 lanes write 32 contiguous bytes of the sequence-contiguous l and r
-  pp.rmQ = S;
+  // logical row r = i*Sp + s reads MSA row s*N + i, so a wave's rows are consecutive sequences
+  // of one residue: 16 lanes write 32 contiguous bytes of the sequence-contiguous l and r.  The
+  // sequences are padded to Sp, a multiple of 8, with zero rows: every depth gets vector stores
+  // here and 16-byte loads in the outer products
+  const int Sp = (S + 7) & ~7;
+  LF_REQUIRE((long long)N * Sp < (1LL << 31), "outer product mean: too many rows");
+  pp.rows = N * Sp;
+  pp.rmQ = Sp;
   pp.rmB = N;
+  pp.rmN = S;
+  pp.span_slack = (long long)N * co * (Sp - S);
   pp.ln_s = w.norm_scale;
   pp.ln_o = w.norm_offset;
   pp.eps = a.epsilon;
@@ -463,9 +466,10 @@ int outer_product_mean(lf_context* ctx, const lf_opm_args& a) {
   pp.g[1] = Group{views[1], WView{}, co, OP_ROWMASK, 1.f, w.br, nullptr, Dst{}};
   pp.ngroups = 2;
 
-  const size_t lr = (size_t)N * co * S * sizeof(_Float16);
-  // c_outer 32, c_z 128, whole 256 tiles: the output GEMM runs inside the outer-product kernel
-  const bool fused = co == 32 && cz == 128 && (N * co) % OB == 0 && S % OT_BK == 0 && big_smem_ok(ctx);
+  // c_outer 32, c_z 128: the output GEMM runs inside the outer-product kernel, whose edge tiles
+  // read l and r up to a whole 256-row tile (8 residues; what is there reaches no stored output)
+  const bool fused = co == 32 && cz == 128 && big_smem_ok(ctx);
+  const size_t lr = (size_t)(fused ? (N + 7) & ~7 : N) * co * Sp * sizeof(_Float16);
   const size_t ob = fused ? 0 : (size_t)pairs * co * co * sizeof(_Float16);
   size_t sizes[6] = {lr, lr, ob, (size_t)pairs * sizeof(float), expanded_bytes(views[2]), lnproj_packed_bytes(pp)};
   void* bufs[6];
@@ -476,9 +480,9 @@ int outer_product_mean(lf_context* ctx, const lf_opm_args& a) {
   ExpandList xl;
   WExp wo;
   LF_TRY(expand_add_plain(ctx, xl, views[2], bufs[4], &wo, 1.f, "opm.expand"));
-  // logical row r = i*S + s, column a -> (i*co + a)*S + s
-  pp.g[0].dst = Dst{L, DT_F16, S, (long long)co * S, 1, co, 0, S};
-  pp.g[1].dst = Dst{R, DT_F16, S, (long long)co * S, 1, co, 0, S};
+  // logical row r = i*Sp + s, column a -> (i*co + a)*Sp + s
+  pp.g[0].dst = Dst{L, DT_F16, Sp, (long long)co * Sp, 1, co, 0, Sp};
+  pp.g[1].dst = Dst{R, DT_F16, Sp, (long long)co * Sp, 1, co, 0, Sp};
   LF_TRY(lnproj_prepare(ctx, pp, bufs[5], &xl, "opm.project"));
   LF_TRY(expand_flush(ctx, xl, "opm.expand"));
   LF_TRY(lnproj_run(ctx, pp, a.msa_dtype, "opm.project"));
@@ -490,32 +494,31 @@ int outer_product_mean(lf_context* ctx, const lf_opm_args& a) {
     if (!filled) {
       {
         LaunchScope ls(ctx, "opm.count");
-        hipLaunchKernelGGL(opm_count_kernel, dim3((N + 15) / 16, (N + 15) / 16), dim3(256), 0, ctx->stream, a.mask,
+        hipLaunchKernelGGL(opm_count_kernel, dim3((N + 15) / 16, (N + 15) / 16), dim3(1024), 0, ctx->stream, a.mask,
                            den, S, N, a.norm_epsilon);
       }
       LF_TRY(check_hip(hipGetLastError(), "opm count launch"));
     }
   }
   if (fused) {
-    OpmFusedParams f{OuterParams{L, R, nullptr, N, co, S}, wo.p, wo.kp, w.bo, den,
+    OpmFusedParams f{OuterParams{L, R, nullptr, N, co, Sp}, wo.p, wo.kp, w.bo, den,
                      a.accumulate ? a.pair_in : nullptr, a.out};
-    const int tb = N * co / OB;
+    const int tb = (N * co + OB - 1) / OB;
+    const bool tail = Sp % OT_BK != 0;
     LaunchScope ls(ctx, "opm.fused");
-    if (a.pair_dtype == LF_F32)
-      hipLaunchKernelGGL(opm_fused_kernel<DT_F32>, dim3((unsigned)(tb * tb)), dim3(512), OB_SMEM, ctx->stream, f);
-    else if (a.pair_dtype == LF_F16)
-      hipLaunchKernelGGL(opm_fused_kernel<DT_F16>, dim3((unsigned)(tb * tb)), dim3(512), OB_SMEM, ctx->stream, f);
-    else
-      hipLaunchKernelGGL(opm_fused_kernel<DT_BF16>, dim3((unsigned)(tb * tb)), dim3(512), OB_SMEM, ctx->stream, f);
+    auto k = a.pair_dtype == LF_F32   ? (tail ? opm_fused_kernel<DT_F32, true> : opm_fused_kernel<DT_F32, false>)
+             : a.pair_dtype == LF_F16 ? (tail ? opm_fused_kernel<DT_F16, true> : opm_fused_kernel<DT_F16, false>)
+                                      : (tail ? opm_fused_kernel<DT_BF16, true> : opm_fused_kernel<DT_BF16, false>);
+    hipLaunchKernelGGL(k, dim3((unsigned)(tb * tb)), dim3(512), OB_SMEM, ctx->stream, f);
     return check_hip(hipGetLastError(), "opm fused launch");
   }
   {  // O[(i, j)][a*co + b] = sum_s l[i][a][s] r[j][b][s]
-    OuterParams op{L, R, O, N, co, S};
+    OuterParams op{L, R, O, N, co, Sp};
     const int tm = (N * co + OT - 1) / OT;
     LaunchScope ls(ctx, "opm.outer");
-    const bool full = (N * co) % OT == 0 && S % OT_BK == 0;
+    const bool full = (N * co) % OT == 0 && Sp % OT_BK == 0;
     const int tb = N * co / OB;
-    if ((N * co) % OB == 0 && S % OT_BK == 0 && big_smem_ok(ctx)) {
+    if ((N * co) % OB == 0 && Sp % OT_BK == 0 && big_smem_ok(ctx)) {
       hipLaunchKernelGGL(opm_outer_big_kernel, dim3((unsigned)(tb * tb)), dim3(512), OB_SMEM, ctx->stream, op);
     } else if (full)
       hipLaunchKernelGGL(opm_outer_kernel<true>, dim3((unsigned)(tm * tm)), dim3(256), 0, ctx->stream, op);

@@ -34,7 +34,7 @@ __device__ __forceinline__ void chunk_store(_Float16* Ws, const u32x4 (&regs)[NR
 __device__ __forceinline__ int dst_row32(const Dst& d, int row) {
   const unsigned q = (unsigned)d.Q;
   const unsigned b = (unsigned)row / q, n = (unsigned)row - b * q;
-  return (int)b * (int)d.sB + (int)n * (int)d.sN;
+  return (int)(b * (unsigned)d.sB + n * (unsigned)d.sN);   // 32 bits, read as unsigned
 }
 __device__ __forceinline__ int dst_col32(const Dst& d, int col) {
   const unsigned dd = (unsigned)d.D;
@@ -85,12 +85,12 @@ __device__ __forceinline__ void store4(_Float16* out, int rowpart, int4 co, bool
   const bool vec = row_ok && co.x >= 0 && co.y == co.x + 1 && co.z == co.x + 2 && co.w == co.x + 3 &&
                    ((rowpart + co.x) & 3) == 0;
   if (__all(vec)) {
-    *reinterpret_cast<h4*>(out + rowpart + co.x) = pack_h4(v);
+    *reinterpret_cast<h4*>(out + (uint32_t)(rowpart + co.x)) = pack_h4(v);
   } else if (row_ok) {
-    if (co.x >= 0) out[rowpart + co.x] = (_Float16)v[0];
-    if (co.y >= 0) out[rowpart + co.y] = (_Float16)v[1];
-    if (co.z >= 0) out[rowpart + co.z] = (_Float16)v[2];
-    if (co.w >= 0) out[rowpart + co.w] = (_Float16)v[3];
+    if (co.x >= 0) out[(uint32_t)(rowpart + co.x)] = (_Float16)v[0];
+    if (co.y >= 0) out[(uint32_t)(rowpart + co.y)] = (_Float16)v[1];
+    if (co.z >= 0) out[(uint32_t)(rowpart + co.z)] = (_Float16)v[2];
+    if (co.w >= 0) out[(uint32_t)(rowpart + co.w)] = (_Float16)v[3];
   }
 }
 
@@ -100,12 +100,12 @@ __device__ __forceinline__ void store4t(_Float16* out, int4 rp, int co, int nrow
   const bool vec = nrow == 4 && co >= 0 && rp.y == rp.x + 1 && rp.z == rp.x + 2 && rp.w == rp.x + 3 &&
                    ((rp.x + co) & 3) == 0;
   if (__all(vec)) {
-    *reinterpret_cast<h4*>(out + rp.x + co) = pack_h4(v);
+    *reinterpret_cast<h4*>(out + (uint32_t)(rp.x + co)) = pack_h4(v);
   } else if (co >= 0) {
-    if (nrow > 0) out[rp.x + co] = (_Float16)v[0];
-    if (nrow > 1) out[rp.y + co] = (_Float16)v[1];
-    if (nrow > 2) out[rp.z + co] = (_Float16)v[2];
-    if (nrow > 3) out[rp.w + co] = (_Float16)v[3];
+    if (nrow > 0) out[(uint32_t)(rp.x + co)] = (_Float16)v[0];
+    if (nrow > 1) out[(uint32_t)(rp.y + co)] = (_Float16)v[1];
+    if (nrow > 2) out[(uint32_t)(rp.z + co)] = (_Float16)v[2];
+    if (nrow > 3) out[(uint32_t)(rp.w + co)] = (_Float16)v[3];
   }
 }
 
@@ -249,14 +249,20 @@ __global__ __launch_bounds__(512, KS <= 4 ? 4 : 2) void lnproj_kernel(LnProjPara
     const int g = i / LP_ROWS, r = i - g * LP_ROWS;
     Rp[g][r] = row_block + r < p.rows ? dst_row32(p.g[g].dst, row_block + r) : 0;
   }
+  auto srow_of = [&](int r) {
+    if (p.rmN > 0) {
+      const int bb = r / p.rmQ, q = min(r - bb * p.rmQ, p.rmN - 1);
+      return p.rmB > 0 ? q * p.rmB + bb : bb * p.rmN + q;
+    }
+    return p.rmB > 0 ? (r % p.rmQ) * p.rmB + r / p.rmQ : r;
+  };
   if (p.rowmask && tid < LP_ROWS) {
     const int r = row_block + tid;
-    Rm[tid] = r < p.rows ? p.rowmask[p.rmB > 0 ? (r % p.rmQ) * p.rmB + r / p.rmQ : r] : 0.f;
+    Rm[tid] = r < p.rows && (p.rmN <= 0 || r % p.rmQ < p.rmN) ? p.rowmask[srow_of(r)] : 0.f;
   }
 
   // this wave's two 16-row tiles, LayerNorm'd into B fragments
   const int rbase = row_block + wave * 32;
-  auto srow_of = [&](int r) { return p.rmB > 0 ? (r % p.rmQ) * p.rmB + r / p.rmQ : r; };
   h8 xb[2][KS];
   chunk_store<KP, NREG>(Ws[0][0], regs, tid);
   if constexpr (NB == 2) {   // the second chunk of the first pair (clamped)
@@ -365,7 +371,8 @@ int lnproj_prepare(lf_context* ctx, LnProjParams& p, void* packed, ExpandList* x
     const long long span = (long long)((p.rows - 1) / d.Q) * d.sB + (long long)std::min(p.rows - 1, d.Q - 1) * d.sN +
                            (long long)((p.g[g].ncols - 1) / d.D) * d.sH +
                            (long long)std::min(p.g[g].ncols - 1, d.D - 1) * d.sD;
-    if (span >= (1LL << 31)) return set_error(LF_ERR_INVALID, std::string(label) + ": destination above 2^31 elements");
+    if (span >= (1LL << 31) + p.span_slack)
+      return set_error(LF_ERR_INVALID, std::string(label) + ": destination above 2^31 elements");
     const bool cols_contig = d.D % 4 == 0 && d.sD == 1;
     const bool rows_contig = d.sN == 1 && d.Q % 4 == 0;
     p.g[g].tr = !cols_contig && rows_contig;

@@ -112,6 +112,24 @@ def test_opm_af2(ctx, blockw, s, n):
     H.assert_close(pair.cpu().numpy(), ref, label=f"opm {s}x{n}")
 
 
+@pytest.mark.parametrize("s,n", [(3, 9), (8, 7), (63, 17), (72, 8), (126, 33), (250, 15), (260, 65)])
+def test_opm_ragged(ctx, blockw, s, n):
+    """Sequences on both sides of a multiple of 8 (the padding of l and r) and of 64 (the K step),
+    lengths on both sides of a multiple of 8 (edge tiles), more than one count round (s > 256)."""
+    import torch
+    from localfold_amd import device as D
+    act = S.synthetic_activations(s, n, 256, 128, seed=300 + s)
+    mask = (S.Stream(500 + s).uniform(s * n).reshape(s, n) > 0.3).astype(np.float32)
+    w = blockw["outerProductMean"]
+    dw = D.DeviceWeights(ctx.device)
+    ws = D.opm_weights(dw, w)
+    pair = _dev(ctx, act["pair"])
+    D.outer_product_mean(ctx, _dev(ctx, act["msa"]), _dev(ctx, mask), ws, 32, 128, pair=pair, out=pair, accumulate=True)
+    torch.cuda.synchronize()
+    ref = act["pair"].astype(np.float64) + ops.outer_product_mean_af2(act["msa"], mask, w)
+    H.assert_close(pair.cpu().numpy(), ref, label=f"opm {s}x{n}")
+
+
 @pytest.mark.parametrize("dt,accumulate", [("bfloat16", True), ("float16", False), ("float32", False)])
 def test_opm_fused_output(ctx, blockw, dt, accumulate):
     """c_outer 32, c_z 128 with whole 256-row outer tiles (N = 64, S = 64) takes the fused kernel:
@@ -141,6 +159,20 @@ def test_opm_fused_output(ctx, blockw, dt, accumulate):
     half_ulp = {"bfloat16": 2.0 ** -8, "float16": 2.0 ** -11, "float32": 0.0}[dt]
     H.assert_close(out.float().cpu().numpy(), ref, max_abs=H.MAX_ABS + half_ulp * float(np.abs(ref).max()),
                    label=f"opm fused {dt} accumulate={accumulate}")
+
+
+@pytest.mark.parametrize("s,n", [(13, 21), (64, 24)])
+def test_opm_other_widths(ctx, s, n):
+    """c_outer 16, c_z 64: the materialised outer product, ragged and whole sequences."""
+    import torch
+    from localfold_amd import device as D
+    w = S.synthetic_block_weights(c_m=64, c_z=64, c_outer=16, heads_msa=4, heads_pair=4, tri_hidden=64, msa_hidden=64,
+                                  pair_hidden=64, seed=2)["outerProductMean"]
+    act = S.synthetic_activations(s, n, 64, 64, seed=77)
+    dw = D.DeviceWeights(ctx.device)
+    out = D.outer_product_mean(ctx, _dev(ctx, act["msa"]), _dev(ctx, act["msaMask"]), D.opm_weights(dw, w), 16, 64)
+    torch.cuda.synchronize()
+    H.assert_close(out.cpu().numpy(), ops.outer_product_mean_af2(act["msa"], act["msaMask"], w), label=f"opm {s}x{n}")
 
 
 def test_opm_af3(ctx):
