@@ -45,7 +45,10 @@ struct FlashParams {
   int fix;                // dq < DP or Q not a whole number of chunks: the kernel (the FIX
                           // instantiation) zeroes the unwritten parts of q, k and v^T as it
                           // reads them
-  int nqb;                // query blocks per (b, h)
+  int nqb;                // query blocks per (b, h); flash_res_kernel: query splits
+  int nw;                 // flash_res_kernel: waves per block
+  const float* mask;      // flash_res_kernel: key k of batch row b is mask[b * mask_b + k * mask_k]
+  int mask_b, mask_k;
   long long nblocks;
 };
 
@@ -58,6 +61,8 @@ constexpr float FA_CLAMP = 1e8f * LOG2E;
 // units): until then p = exp2(x - m) <= 2^FA_RESCALE, well inside f16 range, and the
 // O rescale is skipped.
 constexpr float FA_RESCALE = 8.f;
+// flash_res_kernel's bounds on a chunk's row sums of p (see there)
+constexpr float FA_LOW = 0.0625f, FA_HIGH = 4096.f;
 
 // kb[b][k] for k < Qp (keys padded to whole chunks): 1e9 log2(e) (mask - 1), and -1e30 past Q
 __global__ __launch_bounds__(256) void keybias_kernel(const float* mask, float* kb, int B, int Q, int Qp,
@@ -645,6 +650,390 @@ __global__ __launch_bounds__(64 * (8 / QT)) void flash_kernel(FlashParams p) {
   }
 }
 
+// Flash attention with a (batch row, head)'s whole K, V^T and key bias resident in LDS: a block
+// of p.nw waves stages them once, then every wave walks its 16-query tiles over all the keys
+// with no further barrier and no store to LDS, the pair bias coming straight from L2 into
+// registers.  The chunk arithmetic (lazy running max, bias and row sums through the matrix
+// core) is flash_kernel's.  That kernel gives a block 128 queries and restages every 64-key
+// chunk for each of them: K/V cross L2 once per 128 queries, each chunk costs 8 waves a barrier,
+// and a block's prologue and epilogue (a quarter of its time at 8 chunks) are paid per 128
+// queries.  Measured (us per launch): triangle attention at
+// N = 512 with 4 x 32 heads 219 -> 157, N = 1024 1374 -> 974, MSA row attention 512 x 384 259 -> 197,
+// column attention 508 x 259 181 -> 129.  There the SIMDs issue 224 cycles of MFMA and 250 of VALU per
+// 16 queries x 64 keys, in 590: the two overlap little, so every VALU instruction left out counts.
+//
+// S^T tile kt of a chunk holds in row 4*g + i the key 32*(kt/2) + 8*g + 4*(kt%2) + i, so a lane's
+// 16 scores are keys 8*g4 .. +7 of each 32-key half: its V^T pieces are two 16-byte LDS reads.
+// Rows are padded (K by 8 halves, V^T by 8): the 16-byte reads of 8 lanes fall in distinct banks.
+template <int DP>
+struct FlashRes {
+  static constexpr int KLD = DP + 8, NDT = DP / 16, SEGS = DP / 8;
+  // K [Qp][KLD], V^T [DP][Qp + 8], key bias [Qp] f32, key masks [Qp] u16, what each chunk holds
+  __host__ __device__ static size_t lds(int Qp) {
+    return (size_t)Qp * KLD * 2 + (size_t)DP * (Qp + 8) * 2 + (size_t)Qp * 6 + (size_t)(Qp / FA_KC) * 4;
+  }
+};
+
+template <bool BIAS, int DP>
+__global__ __launch_bounds__(1024) void flash_res_kernel(FlashParams p) {
+  using R = FlashRes<DP>;
+  constexpr int KLD = R::KLD, NDT = R::NDT, SEGS = R::SEGS;
+  using QF = typename std::conditional<DP == 32, h8, h4>::type;
+  extern __shared__ __attribute__((aligned(16))) char flash_smem[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r16 = lane & 15, g4 = lane >> 4, nthr = p.nw * 64;
+  const int nkc = (p.Q + FA_KC - 1) / FA_KC, Qp = nkc * FA_KC, VLD = Qp + 8;
+  _Float16* Ks = reinterpret_cast<_Float16*>(flash_smem);
+  _Float16* Vs = Ks + (size_t)Qp * KLD;
+  float* Kb = reinterpret_cast<float*>(Vs + (size_t)DP * VLD);
+  uint16_t* Km = reinterpret_cast<uint16_t*>(Kb + Qp);
+  int* Kind = reinterpret_cast<int*>(Km + Qp);
+
+  // XCD-aware order: each XCD walks a contiguous range of (split, batch row) for one head, whose
+  // pair bias stays in its L2
+  long long lb = blockIdx.x;
+  const long long per = p.nblocks / 8;
+  if (lb < per * 8) lb = (lb % 8) * per + lb / 8;
+  const int split = (int)(lb % p.nqb);
+  const int b = (int)((lb / p.nqb) % p.B);
+  const int h = (int)(lb / ((long long)p.nqb * p.B));
+  const size_t bh = (size_t)b * p.H + h;
+  const _Float16* qh = p.q + bh * Qp * DP;
+  const _Float16* kh = p.k + bh * Qp * DP;
+  const _Float16* vh = p.vt + bh * DP * Qp;
+
+  // Stage, in pieces of 8 halves, four in flight per thread.  What the projection leaves unwritten
+  // (keys past Q, head dims past dq of K) is zeroed on the way.
+  auto keep = [](uint4& v, int n) __attribute__((always_inline)) {   // the piece's first n halves
+    v.x &= (n > 0 ? 0xffffu : 0u) | (n > 1 ? 0xffff0000u : 0u);
+    v.y &= (n > 2 ? 0xffffu : 0u) | (n > 3 ? 0xffff0000u : 0u);
+    v.z &= (n > 4 ? 0xffffu : 0u) | (n > 5 ? 0xffff0000u : 0u);
+    v.w &= (n > 6 ? 0xffffu : 0u) | (n > 7 ? 0xffff0000u : 0u);
+  };
+  // (K: consecutive threads consecutive pieces; V^T: a wave's lanes pieces of one row, so a piece's
+  // row needs no division)
+  const int kp = Qp * SEGS, vp = Qp / 8, vgrp = (vp + 63) >> 6;   // V pieces per row; 64-piece groups
+  const int ksteps = (kp + 4 * nthr - 1) / (4 * nthr), vsteps = (DP * vgrp + 4 * p.nw - 1) / (4 * p.nw);
+  for (int st = 0; st < max(ksteps, vsteps); ++st) {
+    uint4 rk[4], rv[4];
+    int vrow[4], vpc[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      rk[u] = *reinterpret_cast<const uint4*>(kh + (size_t)min((st * 4 + u) * nthr + tid, kp - 1) * 8);
+      const int g = (st * 4 + u) * p.nw + wave;   // uniform
+      vrow[u] = g % DP;
+      vpc[u] = (g / DP) * 64 + lane;
+      rv[u] = *reinterpret_cast<const uint4*>(vh + (size_t)vrow[u] * Qp + min(vpc[u], vp - 1) * 8);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int i = (st * 4 + u) * nthr + tid, key = i / SEGS, seg = i % SEGS;
+      if (p.fix) {
+        keep(rk[u], key < p.Q ? p.dq - seg * 8 : 0);
+        keep(rv[u], p.Q - vpc[u] * 8);
+      }
+      if (i < kp) *reinterpret_cast<uint4*>(Ks + key * KLD + seg * 8) = rk[u];
+      if (vpc[u] < vp) *reinterpret_cast<uint4*>(Vs + vrow[u] * VLD + vpc[u] * 8) = rv[u];
+    }
+  }
+  // Key bias 1e9 log2(e) (mask - 1), -1e30 past Q, and per chunk what its keys are: bit 0 an
+  // unmasked one, bit 1 a masked one (its clamped logit leaves it weight 0 beside any unmasked
+  // key) or one past Q, bit 2 one in between
+  for (int c = wave; c < nkc; c += p.nw) {
+    const int k = c * FA_KC + lane;
+    const float m = p.mask[(size_t)b * p.mask_b + (size_t)min(k, p.Q - 1) * p.mask_k];
+    const float v = k < p.Q ? (1e9f * LOG2E) * (m - 1.0f) : -1e30f;
+    Kb[k] = v;
+    Km[k] = v == 0.f ? 0xffff : 0;
+    const bool on = __any(v == 0.f), off = __any(v < -1e9f), part = __any(!(v == 0.f || v < -1e9f));
+    if (lane == 0) Kind[c] = (on ? 1 : 0) | (off ? 2 : 0) | (part ? 4 : 0);
+  }
+
+  const int ntiles = (p.Q + 15) >> 4, tstep = p.nw * p.nqb;
+  int tile = wave * p.nqb + split;
+  const int qd = DP == 32 ? 8 * g4 : 4 * g4;   // the lane's head dims of a Q / K fragment, and of O
+  const bool wide = p.d == DP;
+  h8 ones = h8{1, 1, 1, 1, 1, 1, 1, 1};
+  // identity A operand of a 16x16x16 MFMA: lane supplies I[r16][4*g4 + j]
+  const h4 ident = h4{(_Float16)(r16 == 4 * g4), (_Float16)(r16 == 4 * g4 + 1), (_Float16)(r16 == 4 * g4 + 2),
+                      (_Float16)(r16 == 4 * g4 + 3)};
+  {  // held in registers, not rebuilt in the loop
+    u32x4 w = __builtin_bit_cast(u32x4, ones);
+    asm volatile("" : "+v"(w.x), "+v"(w.y), "+v"(w.z), "+v"(w.w));
+    ones = __builtin_bit_cast(h8, w);
+  }
+  // the lane's K row of tile kt: key krow + 32*(kt/2) + 4*(kt%2) of the chunk
+  const _Float16* kl = Ks + (8 * (r16 >> 2) + (r16 & 3)) * KLD + qd;
+  // V^T row r16 of O tile dt is head dim 4*NDT*(r16/4) + 4*dt + r16%4, so a lane's output dims are
+  // 4*NDT consecutive ones: its gate and its output are one vector each
+  const _Float16* vl = Vs + (4 * NDT * (r16 >> 2) + (r16 & 3)) * VLD + 8 * g4;
+  // The pair bias of the lane's query: keys 8*g4 .. +7 of a chunk's two halves (fragment order,
+  // tiled_at: 1 KB per load in lane order; queries and keys past Q are in the buffer, unwritten,
+  // and not used)
+  struct Bias {
+    h8 lo, hi;
+  };
+  const size_t btile = (size_t)Qp * 16;   // a 16-query tile's bias
+  const _Float16* bias = BIAS ? p.bias + (size_t)h * ntiles * btile : nullptr;
+  auto bias_load = [&](Bias& v, const _Float16* at) __attribute__((always_inline)) {
+    v.lo = reinterpret_cast<const h8*>(at)[lane];
+    v.hi = reinterpret_cast<const h8*>(at)[lane + 64];
+  };
+  auto bias_at = [&](int t) __attribute__((always_inline)) { return bias + t * btile; };
+  // this (b, h)'s gate rows and output columns, and where lanes without an output store theirs
+  const _Float16* grow = p.g + ((size_t)h * p.B + b) * p.Q * p.d;
+  _Float16* orow = p.o + (size_t)b * p.Q * p.HD + h * p.d;
+  const unsigned oend = (unsigned)((p.B - b) * p.Q * p.HD - h * p.d);
+  auto q_load = [&](int t) __attribute__((always_inline)) {
+    return *reinterpret_cast<const QF*>(qh + (size_t)(t * 16 + r16) * DP + qd);
+  };
+  QF qnext = q_load(tile < ntiles ? tile : 0);
+  Bias bA, bB;
+  if (BIAS) bias_load(bA, bias_at(tile < ntiles ? tile : 0));
+  __syncthreads();
+  // Per chunk (at most 64 fit the LDS) in bit masks: cmask, whose masked keys only have their
+  // weights cleared, and gmask, which take the explicit key bias (a key in between; no unmasked
+  // key in the chunk, or in the row).  Chunks after the last unmasked key are left out.
+  const int kind = lane < nkc ? Kind[lane < nkc ? lane : 0] : 0;
+  const bool some = __any(kind & 1);
+  const unsigned long long gmask = __ballot((kind & 4) || kind == 2 || (!some && kind)), cmask = __ballot(kind == 3);
+  const int nke = some ? 64 - __builtin_clzll(__ballot(kind & 5)) : nkc;
+  // GEN: with the explicit update of gmask's chunks; most blocks have none, and the loop without
+  // that path keeps its state in place
+  auto walk = [&](auto gen_tag) __attribute__((always_inline)) {
+  constexpr bool GEN = decltype(gen_tag)::value;
+  for (; tile < ntiles; tile += tstep) {
+    const int qi = tile * 16 + r16, qc = min(qi, p.Q - 1);
+    const unsigned long long vmask = __ballot(qi < p.Q);   // the others take no part in the votes
+    QF qf = qnext;   // loaded a tile ahead (rows up to Qp exist)
+    qnext = q_load(tile + tstep < ntiles ? tile + tstep : tile);
+    if (p.dq < DP) {   // uniform
+#pragma unroll
+      for (int e = 0; e < (int)(sizeof(QF) / 2); ++e)
+        if (qd + e >= p.dq) qf[e] = (_Float16)0.f;
+    }
+    // the epilogue's gate (head-major [h][row][d]), read ahead
+    QF gv;
+    if (wide) {   // uniform: a lane's dims in one load
+      gv = *reinterpret_cast<const QF*>(grow + (unsigned)(qc * DP + qd));
+    } else {
+#pragma unroll
+      for (int dt = 0; dt < NDT; ++dt) {
+        const h4 w = *reinterpret_cast<const h4*>(grow + (unsigned)(qc * p.d + min(qd + 4 * dt, p.d - 4)));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) gv[4 * dt + i] = w[i];
+      }
+    }
+    // -m in the four registers of an accumulator, the row sum l, O^T[qd + 4*dt + i][query]
+    f4 negm = f4{0.f, 0.f, 0.f, 0.f};
+    float l = 0.f;
+    f4 o[NDT];
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt) o[dt] = f4{0.f, 0.f, 0.f, 0.f};
+    bool started = false;   // uniform: an unmasked key was seen (GEN)
+    const _Float16* brow = BIAS ? bias_at(tile) : nullptr;
+    const _Float16* bnext = BIAS ? bias_at(tile + tstep < ntiles ? tile + tstep : tile) : nullptr;
+
+    // chunk c with its bias in bc; the bias of the chunk after it is loaded into bn at the top (no
+    // branch separates that load from the next chunk, so nothing waits for it before its use)
+    auto chunk = [&](int c, Bias& bc, Bias& bn) __attribute__((always_inline)) {
+      const bool fresh = GEN ? !started : c == 0;   // no unmasked key before this chunk
+      const _Float16* vc = vl + c * FA_KC;
+      QF kf[4];
+#pragma unroll
+      for (int kt = 0; kt < 4; ++kt)
+        kf[kt] = *reinterpret_cast<const QF*>(kl + (c * FA_KC + 32 * (kt >> 1) + 4 * (kt & 1)) * KLD);
+      if (BIAS) {
+        bias_load(bn, c + 1 < nke ? brow + (c + 1) * (16 * FA_KC) : bnext);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      h4 bq[4];
+      if (BIAS) {
+        bq[0] = h4{bc.lo[0], bc.lo[1], bc.lo[2], bc.lo[3]};
+        bq[1] = h4{bc.lo[4], bc.lo[5], bc.lo[6], bc.lo[7]};
+        bq[2] = h4{bc.hi[0], bc.hi[1], bc.hi[2], bc.hi[3]};
+        bq[3] = h4{bc.hi[4], bc.hi[5], bc.hi[6], bc.hi[7]};
+      }
+      f4 s[4];
+      float lc;
+      // the chunk's masked keys, as all-ones or zero halves in the order of p
+      const bool clear = (cmask >> c) & 1;   // uniform
+      const uint16_t* km = Km + c * FA_KC + 8 * g4;
+      h8 pf[2];
+      // s = x + cm: the bias lands through an identity MFMA (D = I B + C, B = the lane's bias h4 in
+      // the accumulator layout)
+      auto scores = [&](const f4& cm) __attribute__((always_inline)) {
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt) s[kt] = BIAS ? mfma16k16(ident, bq[kt], cm) : cm;
+        // (a product that accumulates onto one issued just before it finishes later than the wait
+        // states the compiler leaves before a VALU read of it: with the bias and score products
+        // of a tile back to back the exponentials read stale scores.  In two groups, each
+        // accumulates onto a product three issues old)
+        if (BIAS) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt) s[kt] = qk_mfma(kf[kt], qf, s[kt]);
+      };
+      // p = exp2(s) as the B operand of O^T += V^T P^T, and its row sum lc
+      auto probs = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) pf[kt >> 1][4 * (kt & 1) + i] = (_Float16)__builtin_amdgcn_exp2f(s[kt][i]);
+        if (__builtin_expect(clear, 0)) {
+#pragma unroll
+          for (int kh2 = 0; kh2 < 2; ++kh2)
+            pf[kh2] = __builtin_bit_cast(h8, __builtin_bit_cast(u32x4, pf[kh2]) &
+                                                 *reinterpret_cast<const u32x4*>(km + 32 * kh2));
+        }
+        // (two independent products: see scores)
+        const f4 l0 = mfma16(ones, pf[0], f4{0.f, 0.f, 0.f, 0.f}), l1 = mfma16(ones, pf[1], f4{0.f, 0.f, 0.f, 0.f});
+        lc = l0[0] + l1[0];
+      };
+      auto smax = [&]() __attribute__((always_inline)) {
+        float mx = -1e30f;
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) mx = fmaxf(mx, s[kt][i]);
+        return lanes4_max(mx);
+      };
+      // m += d: the scores, and what is accumulated, move to the new base
+      auto rebase = [&](float d, float corr) __attribute__((always_inline)) {
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) s[kt][i] -= d;
+        l *= corr;
+#pragma unroll
+        for (int dt = 0; dt < NDT; ++dt) o[dt] = o[dt] * corr;
+      };
+      if (GEN && ((gmask >> c) & 1)) {   // uniform: the clamp and the full update
+        scores(f4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt) {
+          const float4 kb4 =
+              *reinterpret_cast<const float4*>(Kb + c * FA_KC + 32 * (kt >> 1) + 8 * g4 + 4 * (kt & 1));
+          const float kbv[4] = {kb4.x, kb4.y, kb4.z, kb4.w};
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const float x = s[kt][i] + kbv[i];
+            // (keys past Q carry -1e30 and stay below every real logit)
+            s[kt][i] = kbv[i] < -1e29f ? -1e30f : __builtin_amdgcn_fmed3f(x, -FA_CLAMP, FA_CLAMP);
+          }
+        }
+        const float m_old = c == 0 ? -1e30f : -negm[0], m_new = fmaxf(m_old, smax());
+        rebase(m_new, __builtin_amdgcn_exp2f(m_old - m_new));
+        negm = f4{-m_new, -m_new, -m_new, -m_new};
+        started = started || (__ballot(m_new < -0.5f * FA_CLAMP) & vmask) == 0;
+        probs();
+      } else {
+        // The first chunk without masked keys measures against m = 0 and re-bases on its own
+        // maximum below unless its sums are fine as they are; what masked keys accumulated before
+        // it has weight 0 and is dropped (s - m would round to multiples of 16 from their -1e8)
+        if (GEN && fresh && c > 0) {
+          negm = f4{0.f, 0.f, 0.f, 0.f};
+          l = 0.f;
+#pragma unroll
+          for (int dt = 0; dt < NDT; ++dt) o[dt] = f4{0.f, 0.f, 0.f, 0.f};
+        }
+        scores(negm);
+        probs();
+        // m moves only when a query's row sum of the chunk leaves [2^-4 (first chunk), 2^12]: an f16
+        // p overflows at 2^16 and keeps 2^-15 of the sum above 2^-4, whatever m is in between
+        const float lo = fresh ? FA_LOW : -1.f;
+        if (__builtin_expect(((__ballot(!(lc <= FA_HIGH)) | __ballot(lc < lo)) & vmask) != 0, 0)) {
+          if (clear) {   // masked keys do not count
+#pragma unroll
+            for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+              for (int i = 0; i < 4; ++i)
+                s[kt][i] = km[32 * (kt >> 1) + 4 * (kt & 1) + i] ? s[kt][i] : -1e30f;
+          }
+          const float mx = smax(), d = fresh ? mx : fmaxf(mx, 0.f);
+          rebase(d, fresh ? 1.f : __builtin_amdgcn_exp2f(-d));
+          const float nm = negm[0] - d;
+          negm = f4{nm, nm, nm, nm};
+          probs();
+        }
+        started = true;
+      }
+      l += lc;
+      // O^T += V^T P^T over two 32-key halves (MFMA k index 8*g4 + j is key 32*kh2 + 8*g4 + j)
+#pragma unroll
+      for (int kh2 = 0; kh2 < 2; ++kh2)
+#pragma unroll
+        for (int dt = 0; dt < NDT; ++dt)
+          o[dt] = mfma16(*reinterpret_cast<const h8*>(vc + 4 * dt * VLD + 32 * kh2), pf[kh2], o[dt]);
+    };
+    int c = 0;
+    for (; c + 2 <= nke; c += 2) {
+      chunk(c, bA, bB);
+      chunk(c + 1, bB, bA);
+    }
+    if (c < nke) {
+      chunk(c, bA, bB);
+      if (BIAS) bA = bB;
+    }
+    // the last two products of an O tile accumulate onto each other: wait for them (see scores)
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_nop 15");
+    __builtin_amdgcn_sched_barrier(0);
+    // o[query][h*d + dd] = O / l * g; lanes past Q or d store into the row after the last
+    const float inv = __builtin_amdgcn_rcpf(l);   // (f16 results)
+    if (wide) {
+      QF ov;
+#pragma unroll
+      for (int e = 0; e < 4 * NDT; ++e) ov[e] = (_Float16)(o[e >> 2][e & 3] * inv * (float)gv[e]);
+      *reinterpret_cast<QF*>(orow + (qi < p.Q ? (unsigned)(qi * p.HD + qd) : oend)) = ov;
+    } else {
+#pragma unroll
+      for (int dt = 0; dt < NDT; ++dt) {
+        h4 ov;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) ov[i] = (_Float16)(o[dt][i] * inv * (float)gv[4 * dt + i]);
+        *reinterpret_cast<h4*>(orow + (qi < p.Q && qd + 4 * dt < p.d ? (unsigned)(qi * p.HD + qd + 4 * dt) : oend)) = ov;
+      }
+    }
+  }
+  };
+  if (gmask) walk(std::true_type{});
+  else walk(std::false_type{});
+}
+
+// Waves per block and query splits of flash_res_kernel, false when K and V do not fit the LDS.
+// Few (batch row, head) pairs have their queries split over the CUs.  A CU holds 16 waves (128
+// registers each) and as many blocks as their LDS allows; the wave count is the one that keeps
+// the most of them busy through whole rounds of query tiles, but enough to stage with.
+template <int DP>
+static bool flash_res_shape(const lf_context* ctx, int Q, int Qp, long long bh, int* nw, int* nsplit) {
+  const size_t lds = FlashRes<DP>::lds(Qp), cap = 160 * 1024;
+  if (lds > cap) return false;
+  const int tiles = (Q + 15) / 16, cus = ctx->num_cus;
+  const int split = (int)std::min<long long>(std::max<long long>(1, cus / bh), tiles);
+  const int t = (tiles + split - 1) / split;
+  double best = 0;
+  for (int w = 1; w <= 16; ++w) {
+    const int blocks = (int)std::min<long long>(std::min<long long>((long long)(cap / lds), 16 / w),
+                                                (bh * split + cus - 1) / cus);
+    const double busy = (double)blocks * w * t / (w * ((t + w - 1) / w));
+    if (busy > best * 1.001) best = busy, *nw = w;
+  }
+  *nw = std::max(*nw, std::min(8, Qp / FA_KC));
+  *nsplit = split;
+  return true;
+}
+
+template <bool BIAS, int DP>
+static int launch_flash_res(lf_context* ctx, FlashParams fp, int Qp) {
+  static const bool ok = hipFuncSetAttribute(reinterpret_cast<const void*>(flash_res_kernel<BIAS, DP>),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) == hipSuccess;
+  if (!ok) return set_error(LF_ERR_DEVICE, "flash: the device refuses 160 KB of LDS");
+  fp.nblocks = (long long)fp.nqb * fp.B * fp.H;
+  hipLaunchKernelGGL((flash_res_kernel<BIAS, DP>), dim3((unsigned)fp.nblocks), dim3(64 * fp.nw),
+                     FlashRes<DP>::lds(Qp), ctx->stream, fp);
+  return LF_OK;
+}
+
 int attention(lf_context* ctx, const lf_attention_args& a, bool no_qk, bool shared_key_mask) {
   LF_REQUIRE(a.w != nullptr, "attention: weights are NULL");
   LF_REQUIRE(a.batch > 0 && a.queries > 0 && a.channels > 0 && a.heads > 0,
@@ -692,8 +1081,10 @@ int attention(lf_context* ctx, const lf_attention_args& a, bool no_qk, bool shar
   // of 8), else 32
   const int DP = d <= 16 ? 16 : FA_DP;
   const size_t qkv = (size_t)B * H * Qp * DP * sizeof(_Float16);
-  const size_t hd = (size_t)rows * HD * sizeof(_Float16);
-  const size_t biash = (a.bias_mode == LF_BIAS_NONE) ? 0 : (size_t)H * Q * Qp * sizeof(_Float16);
+  // (o has a row beyond the last: flash_res_kernel)
+  const size_t hd = ((size_t)rows + 1) * HD * sizeof(_Float16);
+  const size_t biash =
+      (a.bias_mode == LF_BIAS_NONE) ? 0 : (size_t)H * ((Q + 15) & ~15) * Qp * sizeof(_Float16);
   // buffers: q, k, v, g, o, key bias, f16 pair bias, output weights, packed lnproj weights x 2
   void* bufs[10];
 
@@ -748,9 +1139,14 @@ int attention(lf_context* ctx, const lf_attention_args& a, bool no_qk, bool shar
   // pair-weighted averaging with d % 4 == 0: one softmax per (h, i) and an NT GEMM over the
   // sequences instead of flash attention per sequence; V^T compact, [b][h][d][Qp]
   const bool pwa = no_qk && shared_key_mask && d % 4 == 0 && !a.transpose && a.bias_mode != LF_BIAS_NONE;
+  // K and V resident in LDS: the bias is then in fragment order
+  int nw = 0, nsplit = 0;
+  const bool res = !pwa && d % 4 == 0 &&
+                   (DP == 16 ? flash_res_shape<16>(ctx, Q, Qp, (long long)B * H, &nw, &nsplit)
+                             : flash_res_shape<32>(ctx, Q, Qp, (long long)B * H, &nw, &nsplit));
   const size_t vsize = pwa ? (size_t)B * HD * Qp * sizeof(_Float16) : qkv;
   const size_t qksize = pwa ? 256 : qkv;
-  size_t sizes[10] = {qksize, qksize, vsize, hd, hd, (size_t)(shared_key_mask ? 1 : B) * Qp * sizeof(float), biash, expanded_bytes(views[4]),
+  size_t sizes[10] = {qksize, qksize, vsize, hd, hd, res ? 0 : (size_t)(shared_key_mask ? 1 : B) * Qp * sizeof(float), biash, expanded_bytes(views[4]),
                      lnproj_packed_bytes(pp), a.bias_mode == LF_BIAS_SEPARATE ? lnproj_packed_bytes(pb) : (size_t)0};
   LF_TRY(workspace(ctx, sizes, bufs, 10));
   _Float16 *qb = (_Float16*)bufs[0], *kb = (_Float16*)bufs[1], *vb = (_Float16*)bufs[2];
@@ -771,8 +1167,14 @@ int attention(lf_context* ctx, const lf_attention_args& a, bool no_qk, bool shar
   // and the head dims past d of q and k, as it reads them (FlashParams::fix)
   if (pwa && Qp != Q) LF_TRY(check_hip(hipMemsetAsync(bufs[2], 0, vsize, ctx->stream), "attention memset"));
   // f16 bias [h][i][j] (row stride Qp) from row (i, j); swapped: [h][j][i]
-  const Dst bias_dst = a.swap_bias ? Dst{bias16, DT_F16, Q, 1, Qp, 1, (long long)Q * Qp, 0}
-                                   : Dst{bias16, DT_F16, Q, Qp, 1, 1, (long long)Q * Qp, 0};
+  const long long bplane = (long long)(res ? (Q + 15) & ~15 : Q) * Qp;
+  Dst bias_dst = a.swap_bias ? Dst{bias16, DT_F16, Q, 1, Qp, 1, bplane, 0}
+                             : Dst{bias16, DT_F16, Q, Qp, 1, 1, bplane, 0};
+  if (res) {
+    bias_dst.sB = !a.swap_bias;
+    bias_dst.sN = a.swap_bias;
+    bias_dst.tile = Qp;
+  }
   if (a.bias_mode == LF_BIAS_SEPARATE) {
     pb.g[0].dst = bias_dst;
     LF_TRY(lnproj_prepare(ctx, pb, bufs[9], &xl, "attention.pair_bias"));
@@ -793,9 +1195,9 @@ int attention(lf_context* ctx, const lf_attention_args& a, bool no_qk, bool shar
   if (a.bias_mode == LF_BIAS_SEPARATE) LF_TRY(lnproj_run(ctx, pb, a.pair_dtype, "attention.pair_bias"));
   LF_TRY(lnproj_run(ctx, pp, a.act_dtype, "attention.project"));
 
-  // 3. key-mask bias (inside a stack call, computed by the first block and reused), f16 copy
-  // of the pair bias
-  {
+  // 3. key-mask bias (inside a stack call, computed by the first block and reused;
+  // flash_res_kernel computes its own), f16 copy of the pair bias
+  if (!res) {
     void* cached;
     bool filled;
     LF_TRY(mask_table(ctx, a.mask, shared_key_mask ? 1 : 2 + (a.transpose ? 1 : 0), B, Q, 0.f, sizes[5], &cached,
@@ -817,7 +1219,8 @@ int attention(lf_context* ctx, const lf_attention_args& a, bool no_qk, bool shar
   // caller-supplied f32 logits are converted (and transposed per head when swapped); the
   // projected biases were written as f16 by lnproj
   if (a.bias_mode == LF_BIAS_LOGITS)
-    LF_TRY(f32_to_f16(ctx, a.bias_logits, bias16, (long long)H * Q * Q, a.swap_bias ? Q : 0, LOG2E, Q, Qp));
+    LF_TRY(f32_to_f16(ctx, a.bias_logits, bias16, (long long)H * Q * Q, a.swap_bias ? Q : 0, LOG2E, Q, Qp,
+                      res ? Qp : 0));
 
   // 4. flash attention, or the pair-weighted averaging's softmax + GEMM
   if (pwa) {
@@ -872,7 +1275,17 @@ int attention(lf_context* ctx, const lf_attention_args& a, bool no_qk, bool shar
     // d <= 16 always zeroes (dq < 16 or Q ragged, or both: d = 16 with whole chunks is the
     // exception, and rare); the 32-wide kernel has a variant without the zeroing for the
     // usual d = 32 with whole chunks
-    if (fp.bias && DP == 16)
+    if (res) {
+      fp.nw = nw;
+      fp.mask = a.mask;
+      fp.mask_b = a.transpose ? 1 : Q;
+      fp.mask_k = a.transpose ? B : 1;
+      fp.nqb = nsplit;
+      if (fp.bias && DP == 16) LF_TRY((launch_flash_res<true, 16>(ctx, fp, Qp)));
+      else if (fp.bias) LF_TRY((launch_flash_res<true, 32>(ctx, fp, Qp)));
+      else if (DP == 16) LF_TRY((launch_flash_res<false, 16>(ctx, fp, Qp)));
+      else LF_TRY((launch_flash_res<false, 32>(ctx, fp, Qp)));
+    } else if (fp.bias && DP == 16)
       hipLaunchKernelGGL((flash_kernel<true, FA_QT_BIAS, BLD, 16, true>), grid, bb, 0, ctx->stream, fp);
     else if (fp.bias && fp.fix)
       hipLaunchKernelGGL((flash_kernel<true, FA_QT_BIAS, BLD, 32, true>), grid, bb, 0, ctx->stream, fp);

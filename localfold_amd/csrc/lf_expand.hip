@@ -3,8 +3,7 @@
 // once per op call.  The decode is the reference's readTensorRange arithmetic
 // (shared/weights/dtype.js:212-406): code*scale for int8, fma(code, scale, zero) for int5,
 // exact in float32 before the f16 rounding the MFMA operand needs.
-#include "lf_gemm.h"
-#include "lf_ops.h"
+#include "lf_rowgemm.h"
 
 namespace lf {
 
@@ -94,26 +93,31 @@ int expand_packed(lf_context* ctx, const WView* views, const int* W, const int* 
   return expand_flush(ctx, l, label);
 }
 
-// dst = (f16) (scale * src), n elements; with tq > 0 every [tq][tq] plane is transposed.
+// dst = (f16) (scale * src), n elements; with tq > 0 every [tq][tq] plane is transposed; with
+// tile > 0 planes of rowlen x rowlen are stored in the order of tiled_at with rows of tile columns.
 __global__ __launch_bounds__(256) void f32_to_f16_kernel(const float* src, _Float16* dst, long long n, int tq,
-                                                         float scale, int rowlen, int ld) {
+                                                         float scale, int rowlen, int ld, int tile) {
   for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long long)gridDim.x * 256) {
     long long s = i;
     if (tq > 0) {
       const long long plane = (long long)tq * tq, pl = i / plane, r = i % plane;
       s = pl * plane + (r % tq) * tq + r / tq;
     }
-    const long long o = ld > 0 ? (i / rowlen) * ld + i % rowlen : i;
+    long long o = ld > 0 ? (i / rowlen) * ld + i % rowlen : i;
+    if (tile > 0) {   // rows (h, i) of rowlen columns into the fragment order, 16-row blocks per h
+      const long long row = i / rowlen, hd = row / rowlen, pl = (long long)((rowlen + 15) & ~15) * tile;
+      o = hd * pl + tiled_at((unsigned)(row - hd * rowlen), (unsigned)(i % rowlen), (unsigned)tile);
+    }
     dst[o] = (_Float16)(scale * src[s]);
   }
 }
 
 int f32_to_f16(lf_context* ctx, const float* src, _Float16* dst, long long n, int tq, float scale, int rowlen,
-               int ld) {
+               int ld, int tile) {
   LaunchScope ls(ctx, "convert.f16");
   const long long blocks = std::min<long long>((n + 255) / 256, 65536);
   hipLaunchKernelGGL(f32_to_f16_kernel, dim3((unsigned)std::max<long long>(blocks, 1)), dim3(256), 0, ctx->stream,
-                     src, dst, n, tq, scale, rowlen, ld);
+                     src, dst, n, tq, scale, rowlen, ld, tile);
   return check_hip(hipGetLastError(), "f32_to_f16 launch");
 }
 

@@ -42,7 +42,7 @@ int expand_flush(lf_context* ctx, ExpandList& l, const char* label);
 // dst = scale * src as f16; tq > 0 transposes each tq x tq plane; ld > 0 writes rows of rowlen
 // values at a row stride of ld
 int f32_to_f16(lf_context* ctx, const float* src, _Float16* dst, long long n, int tq, float scale = 1.f,
-               int rowlen = 0, int ld = 0);
+               int rowlen = 0, int ld = 0, int tile = 0);
 
 inline bool act_dtype_ok(int dt) { return dt == LF_F32 || dt == LF_F16 || dt == LF_BF16; }
 inline size_t act_bytes(int dt) { return dt == LF_F32 ? 4 : 2; }

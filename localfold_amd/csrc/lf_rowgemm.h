@@ -24,7 +24,18 @@ struct Dst {
   long long sB, sN;
   int D;
   long long sH, sD;
+  int tile;        // > 0: rows are (i, j) of matrices with rows of `tile` columns stored in the
+                   // fragment order of tiled_at (then (sB, sN) = (1, 0): i = row / Q, j = row % Q,
+                   // or (0, 1): the other way round; a column's matrix starts at sH / sD)
 };
+
+// The pair bias of one head as flash attention reads it: blocks of 16 rows x 32 columns, in a
+// block 8 columns of a row after another and the rows innermost, so that the 64 lanes of a wave
+// (row lane%16, columns 8*(lane/16) .. +7) load 1 KB in lane order.  With rows of Qp the four
+// lanes of a row are 16 lanes apart, and every lane's 16 bytes are an access of their own.
+__host__ __device__ inline unsigned tiled_at(unsigned i, unsigned j, unsigned cols) {
+  return (((i >> 4) * (cols >> 5) + (j >> 5)) << 9) + (((j >> 3) & 3) << 7) + ((i & 15) << 3) + (j & 7);
+}
 
 enum GroupOp { OP_STORE = 0, OP_SIGMOID = 1, OP_RELU = 2, OP_SWIGLU = 3, OP_ROWMASK = 4 };
 

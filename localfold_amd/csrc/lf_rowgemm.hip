@@ -34,6 +34,7 @@ __device__ __forceinline__ void chunk_store(_Float16* Ws, const u32x4 (&regs)[NR
 __device__ __forceinline__ int dst_row32(const Dst& d, int row) {
   const unsigned q = (unsigned)d.Q;
   const unsigned b = (unsigned)row / q, n = (unsigned)row - b * q;
+  if (d.tile > 0) return (int)(d.sB ? tiled_at(b, n, (unsigned)d.tile) : tiled_at(n, b, (unsigned)d.tile));
   return (int)(b * (unsigned)d.sB + n * (unsigned)d.sN);   // 32 bits, read as unsigned
 }
 __device__ __forceinline__ int dst_col32(const Dst& d, int col) {
@@ -368,15 +369,16 @@ int lnproj_prepare(lf_context* ctx, LnProjParams& p, void* packed, ExpandList* x
   for (int g = 0; g < p.ngroups; ++g) {
     const Dst& d = p.g[g].dst;
     if (d.dtype != DT_F16) return set_error(LF_ERR_INVALID, std::string(label) + ": lnproj writes f16 only");
-    const long long span = (long long)((p.rows - 1) / d.Q) * d.sB + (long long)std::min(p.rows - 1, d.Q - 1) * d.sN +
+    const long long last = (p.rows - 1) / d.Q, lastq = std::min(p.rows - 1, d.Q - 1);
+    const long long span = (d.tile > 0 ? (((d.sB ? last : lastq) | 15) + 1) * d.tile : last * d.sB + lastq * d.sN) +
                            (long long)((p.g[g].ncols - 1) / d.D) * d.sH +
                            (long long)std::min(p.g[g].ncols - 1, d.D - 1) * d.sD;
     if (span >= (1LL << 31) + p.span_slack)
       return set_error(LF_ERR_INVALID, std::string(label) + ": destination above 2^31 elements");
     const bool cols_contig = d.D % 4 == 0 && d.sD == 1;
-    const bool rows_contig = d.sN == 1 && d.Q % 4 == 0;
+    const bool rows_contig = (d.tile > 0 ? d.sB == 1 : d.sN == 1) && d.Q % 4 == 0;
     p.g[g].tr = !cols_contig && rows_contig;
-    const bool aligned8 = (reinterpret_cast<uintptr_t>(d.ptr) & 7) == 0 && d.sB % 4 == 0 && d.sH % 4 == 0;
+    const bool aligned8 = (reinterpret_cast<uintptr_t>(d.ptr) & 7) == 0 && (d.tile > 0 || d.sB % 4 == 0) && d.sH % 4 == 0;
     p.g[g].vec = aligned8 && (p.g[g].tr ? d.sD % 4 == 0 : cols_contig && d.sN % 4 == 0);
   }
   // decode every group's weights into chunk order

@@ -310,3 +310,50 @@ def test_config3_full_size_sampled(ctx):
                                 batch_rows=rows)
         got = out.transpose(1, 0, 2)[rows] if ending else out[rows]
         H.assert_close(got, ref, label=f"config3 ending={ending}")
+
+
+@pytest.mark.parametrize("n,heads", [(64, 4), (130, 4), (193, 8), (257, 4)])
+@pytest.mark.parametrize("masks", ["leading", "middle", "trailing", "partial", "all"])
+def test_triangle_attention_key_masks(ctx, n, heads, masks):
+    """Every kind of 64-key chunk: without masked keys, with some, with none unmasked at the
+    start, in between or at the end of the row, fractional masks (an explicit key bias), a row
+    without any unmasked key; 1 to 5 chunks, ragged and whole, head widths 32 and 16."""
+    from localfold_amd import capi, device as D
+    rng = np.random.default_rng(n + heads)
+    w = S.config3_attention_weights(128, heads, 7 + n)
+    pair = rng.standard_normal((n, n, 128)).astype(np.float32)
+    mask = np.ones((n, n), np.float32)
+    if masks == "leading":
+        mask[:, :min(n - 1, 70)] = 0
+    elif masks == "middle":
+        mask[:, n // 4:n // 2] = 0
+        mask[::2, 64:128] = 0
+    elif masks == "trailing":
+        mask[:, n - max(1, n // 3):] = 0
+    elif masks == "partial":
+        mask[:, ::7] = 1.0 - 2e-9 * rng.random((n, len(range(0, n, 7)))).astype(np.float32)
+        mask[:, 5::9] = np.float32(1) - np.float32(2.0 ** -24)
+        mask[:, 3] = 0
+    else:
+        mask[::3] = 0
+    dw = D.DeviceWeights(ctx.device)
+    ws = D.attention_weights_af2(dw, w["attention"], w["pairBias"])
+    out, _, _ = _run(ctx, pair, mask, ws, heads, False, capi.LF_BIAS_NORMALIZED_INPUT)
+    ref = ops.attention_af2(pair, mask, w["attention"], heads, False, dict(w["pairBias"], source="normalized-input"))
+    H.assert_close(out, ref, label=f"keys {n}/{heads}/{masks}")
+
+
+@pytest.mark.parametrize("s,n,gain", [(3, 200, 6.0), (2, 1300, 1.0), (40, 17, 6.0)])
+def test_msa_row_attention_large_logits(ctx, blockw, s, n, gain):
+    """Logits that move the running maximum within and between chunks (queries scaled up), a row
+    longer than the keys that fit the LDS, and a row of one ragged chunk."""
+    from localfold_amd import capi, device as D
+    act = S.synthetic_activations(s, n, 256, 128, seed=3 * s + n)
+    row = blockw["msaRowAttention"]
+    att = dict(row["attention"], queryWeight=row["attention"]["queryWeight"] * np.float32(gain))
+    dw = D.DeviceWeights(ctx.device)
+    ws = D.attention_weights_af2(dw, att, row["pairBias"])
+    out, _, _ = _run(ctx, act["msa"], act["msaMask"], ws, 8, False, capi.LF_BIAS_SEPARATE, act["pair"])
+    pb = dict(row["pairBias"], source="separate", activations=act["pair"])
+    ref = ops.attention_af2(act["msa"], act["msaMask"], att, 8, False, pb)
+    H.assert_close(out, ref, label=f"row {s}x{n} gain {gain}")
