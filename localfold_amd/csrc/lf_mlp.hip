@@ -4,20 +4,27 @@
 // webgpu/kernels/transition.js:745-766, 1080-1085) or swish(h_gate) * h_value (AF3 SwiGLU,
 // cpu/af3/trunk/pairformer.js:180-201).
 //
-// A block of 8 waves owns 256 rows, a wave 32 (two 16-row tiles).  A wave LayerNorms its rows
-// into f16 MFMA fragments (lane: row lane%16, channels 32j + 8*(lane/16) .. +7) that stay in
-// registers.  The hidden dimension streams through double-buffered LDS in chunks of 32 units:
-// W1^T rows [32 (64 for SwiGLU: gate, then value)][C] and W2^T rows [C][32].
+// A wave owns RT 16-row tiles, a block four waves.  A wave LayerNorms its rows into f16 MFMA
+// fragments (lane: row lane%16, channels 32j + 8*(lane/16) .. +7) that stay in registers.  The
+// hidden dimension streams through two LDS buffers in chunks of 32 units, packed so that a
+// fragment is 1 KB in lane order.
 //   GEMM1, weights as the A operand: the lane gets H[row][16t + 4g + i] (g = lane/16, i < 4) of
 //          the chunk's two 16-unit tiles t, starting from b1; then ReLU or swish-gating.
 //   GEMM2: those 8 values are the lane's B fragment as they stand: MFMA k index 8g + e stands
 //          for hidden unit 4g + e (e < 4) or 16 + 4g + e - 4 (e >= 4) of the chunk, and the
-//          packed W2^T rows hold the hidden units in that order, so A fragments are plain
-//          16-byte LDS reads.
+//          packed W2^T rows hold the hidden units in that order.
 //   Output: the lane holds out[row][16ct + 4g + i], started at b2; the residual is added and
 //          four channels stored as one vector at the end.
-// The next chunk's weights are loaded into registers during the current chunk's MFMAs and
-// written to the other LDS buffer before the chunk's barrier.
+// The next chunk is copied straight to the other buffer during the current chunk's products.
+//
+// What bounds it: the matrix pipes and, in the same issue slots, the vector instructions (the two
+// do not overlap: at 262144 rows of 256, bf16, hidden 1024, MFMA 262 k and the others 130 k of 517 k
+// cycles).  Copies that skip the registers leave room for two blocks of 128 rows a CU, whose
+// LayerNorm, store and product phases interleave; with one block of 8 waves, weights staged
+// through registers and the activation in f32 the same call took 332 us, now 274 us (1.0 PFLOP/s),
+// and 512 x 384 rows of 256 in f32 went from 337 to 258 us, 512 x 512 of 128 with SwiGLU in bf16
+// from 163 to 142 us.  Eight waves sharing a buffer (305), 64 rows a wave (350), three or four
+// buffers and wider read-ahead (275 to 280) were no better.
 #include <algorithm>
 #include <cmath>
 
@@ -26,19 +33,16 @@
 
 namespace lf {
 
-constexpr int MLP_WAVES = 8, MLP_ROWS = 32 * MLP_WAVES, MLP_HC = 32;
+constexpr int MLP_WAVES = 4, MLP_NT = 64 * MLP_WAVES, MLP_HC = 32;
+
+typedef float f8 __attribute__((ext_vector_type(8)));
 
 template <int C, int NG>
 struct MlpShape {
   static constexpr int KS = C / 32, CT = C / 16;
-  static constexpr int W1P = C + 8, W2P = MLP_HC + 8;          // LDS row pitches (halves)
-  static constexpr int W1E = NG * MLP_HC * W1P;                // W1^T section of a buffer
-  static constexpr int BUF = W1E + C * W2P;                    // halves per LDS buffer
-  static constexpr int CE = (NG * MLP_HC + MLP_HC) * C;        // packed halves per chunk
-  // 16-byte pieces of a packed chunk per thread: P1 of the W1^T rows, then P2 of the W2^T rows
-  static constexpr int NT = 64 * MLP_WAVES;
-  static constexpr int P1 = NG * MLP_HC * C / 8 / NT, P2 = MLP_HC * C / 8 / NT;
-  static_assert(P1 * NT * 8 == NG * MLP_HC * C && P2 * NT * 8 == MLP_HC * C, "pieces must divide over the block");
+  static constexpr int F1 = KS * NG * 2, NF = F1 + CT;         // 1 KB fragments of a chunk: W1^T, all
+  static constexpr int CE = 512 * NF;                          // packed halves per chunk
+  static_assert(NF % MLP_WAVES == 0 && F1 % 4 == 0 && CT % 4 == 0, "fragments must divide over the waves and groups");
 };
 
 struct MlpParams {
@@ -57,13 +61,16 @@ __host__ __device__ constexpr int mlp_q_of(int hl) {
   return hl < 16 ? 8 * (hl >> 2) + (hl & 3) : 8 * ((hl - 16) >> 2) + 4 + (hl & 3);
 }
 
-// Packed weights, chunk s of 32 hidden units: NG x 32 rows of W1^T (row r of group grp =
-// hidden unit 32s + r of the gate (grp 0) or value (grp 1) half, over the C inputs), then C
-// rows of W2^T, each holding the chunk's 32 hidden units in GEMM2's k order.  Decoding from
-// f32/f16/bf16/int8/int5 happens here, on the device, one thread per run of 8 stored weights
-// (wrun_fetch / wrun_decode): W1 runs are 8 inputs of one hidden unit (a 16-byte store) or 8
-// hidden units of one input (8 rows); W2 runs 8 hidden units of one output (two 4-wide pieces
-// of the k order) or 8 outputs of one hidden unit (8 rows).
+// Packed weights, chunk s of 32 hidden units: the A fragments in the order and lane layout the
+// kernel reads them, 512 halves each (lane l's 8 halves at 8l), so that a wave's read is 1 KB in
+// lane order (no padding, no bank conflicts) and a chunk is copied to LDS as it stands.  First
+// W1^T: k-step j of tile ht of group grp (gate, value) is fragment (j*NG + grp)*2 + ht, its lane
+// (r16, g4) holding hidden unit 32s + 16ht + r16, inputs 32j + 8g4 + e; then W2^T: tile ct, its
+// lane holding output 16ct + r16, positions 8g4 + e of GEMM2's k order.
+// Decoding from f32/f16/bf16/int8/int5 happens here, on the device, one thread per run of 8 stored
+// weights (wrun_fetch / wrun_decode): W1 runs are 8 inputs of one hidden unit (a 16-byte store) or
+// 8 hidden units of one input (8 lanes); W2 runs 8 hidden units of one output (two 4-wide pieces
+// of the k order) or 8 outputs of one hidden unit (8 lanes).
 __global__ __launch_bounds__(256) void mlp_pack_kernel(WView w1g, WView w1v, WView w2, int C, int H, int NG,
                                                        _Float16* dst) {
   const long long ce = (long long)(NG * MLP_HC + MLP_HC) * C, w1e = (long long)NG * MLP_HC * C;
@@ -75,190 +82,170 @@ __global__ __launch_bounds__(256) void mlp_pack_kernel(WView w1g, WView w1v, WVi
       const int u = k1 ? j / (C / 8) : 8 * (j / C), c = k1 ? 8 * (j % (C / 8)) : j % C;
       const WView& w = grp ? w1v : w1g;
       const h8 h = wrun_decode(w, wrun_fetch(w, c, u, 1.f), c, u, 1.f);
-      _Float16* base = dst + (long long)(u / MLP_HC) * ce + (long long)grp * MLP_HC * C + c;
+      const int ht = (u % MLP_HC) >> 4, lane = ((c % 32) >> 3) * 16 + (u & 15);
+      _Float16* base = dst + (long long)(u / MLP_HC) * ce + (((c / 32) * NG + grp) * 2 + ht) * 512 + lane * 8 + (c & 7);
       if (k1) {
-        *reinterpret_cast<h8*>(base + (long long)(u % MLP_HC) * C) = h;
+        *reinterpret_cast<h8*>(base) = h;
       } else {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) base[(long long)((u + e) % MLP_HC) * C] = h[e];
+        for (int e = 0; e < 8; ++e) base[8 * e] = h[e];
       }
     } else {        // W2: (hidden unit u, output c)
       const int j = (int)(i - r1);
       const int c = k2 ? j / (H / 8) : 8 * (j % (C / 8)), u = k2 ? 8 * (j % (H / 8)) : j / (C / 8);
       const h8 h = wrun_decode(w2, wrun_fetch(w2, u, c, 1.f), u, c, 1.f);
-      _Float16* base = dst + (long long)(u / MLP_HC) * ce + w1e;
       const int q = mlp_q_of(u % MLP_HC);
-      if (k2) {   // hidden units u..u+3 and u+4..u+7 sit 8 apart in the k order
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          base[(long long)c * MLP_HC + q + e] = h[e];
-          base[(long long)c * MLP_HC + q + 8 + e] = h[4 + e];
-        }
+      _Float16* base = dst + (long long)(u / MLP_HC) * ce + w1e + (c >> 4) * 512 + ((q >> 3) * 16 + (c & 15)) * 8 + (q & 7);
+      if (k2) {   // hidden units u..u+3 and u+4..u+7 sit 8 apart in the k order: the next 16 lanes
+        *reinterpret_cast<h4*>(base) = __builtin_shufflevector(h, h, 0, 1, 2, 3);
+        *reinterpret_cast<h4*>(base + 128) = __builtin_shufflevector(h, h, 4, 5, 6, 7);
       } else {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) base[(long long)(c + e) * MLP_HC + q] = h[e];
+        for (int e = 0; e < 8; ++e) base[8 * e] = h[e];
       }
     }
   }
 }
 
-template <int ACT, int C, int NG>
-__global__ __launch_bounds__(64 * MLP_WAVES) void mlp_kernel(MlpParams p) {
+template <int ACT, int C, int NG, int RT>
+__global__ __launch_bounds__(MLP_NT, 2) void mlp_kernel(MlpParams p) {
   using S = MlpShape<C, NG>;
-  constexpr int KS = S::KS, CT = S::CT, P1 = S::P1, P2 = S::P2, NT = S::NT;
-  // two buffers of two chunks each: one block barrier per pair of chunks
-  __shared__ __attribute__((aligned(16))) _Float16 Wb[2][2 * S::BUF];
-  __shared__ __attribute__((aligned(16))) float Gs[2 * C];   // LN scale, offset
+  constexpr int KS = S::KS, CT = S::CT, NF = S::NF, F1 = S::F1, PER = NF / MLP_WAVES;
+    // separate objects: reads of one buffer are then known not to wait for copies into the other
+  __shared__ __attribute__((aligned(16))) _Float16 W0[S::CE], W1[S::CE];
+  __shared__ __attribute__((aligned(16))) float B0[64], B1[64];   // b1 of the chunk: gate, then value
+  __shared__ __attribute__((aligned(16))) float Gs[3 * C];        // LN scale, offset, b2
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int r16 = lane & 15, g4 = lane >> 4;
   const int nch = p.H / MLP_HC;
-  const long long row_base = (long long)blockIdx.x * MLP_ROWS + wave * 32;
+  const long long row_base = ((long long)blockIdx.x * MLP_WAVES + wave) * (16 * RT);
 
-  // this thread's pieces of a chunk: W1^T piece k is packed element 8 * (tid + k * NT), LDS
-  // row tid / (C/8) + k * NT / (C/8); W2^T piece k the same past the W1^T part, LDS row
-  // tid / 4 + k * NT / 4 of the W2^T section (offsets: one base register plus constants)
-  const int lw1 = (tid / (C / 8)) * S::W1P + (tid % (C / 8)) * 8;
-  const int lw2 = S::W1E + (tid >> 2) * S::W2P + (tid & 3) * 8;
-  auto load_w1 = [&](const _Float16* src, h8 (&r)[P1]) __attribute__((always_inline)) {
+  // chunk s straight to an LDS buffer, PER fragments a wave
+  const _Float16* wsrc = p.w + wave * (PER * 512) + lane * 8;
+  const float* bsrc = (NG == 2 && lane >= 32 ? p.b1v : p.b1g) + (lane & 31);
+  auto issue = [&](int s, _Float16* W, float* B) __attribute__((always_inline)) {
+#if __HIP_DEVICE_COMPILE__   // a target builtin: the host pass, which only emits the launch stub, lacks it
 #pragma unroll
-    for (int k = 0; k < P1; ++k) r[k] = *reinterpret_cast<const h8*>(src + 8 * (tid + k * NT));
+    for (int k = 0; k < PER; ++k)
+      __builtin_amdgcn_global_load_lds(wsrc + (size_t)s * S::CE + k * 512, W + (wave * PER + k) * 512, 16, 0, 0);
+    if (wave == 0 && p.b1g) __builtin_amdgcn_global_load_lds(bsrc + s * MLP_HC, B, 4, 0, 0);
+#endif
   };
-  auto load_w2 = [&](const _Float16* src, h8 (&r)[P2]) __attribute__((always_inline)) {
-#pragma unroll
-    for (int k = 0; k < P2; ++k) r[k] = *reinterpret_cast<const h8*>(src + NG * MLP_HC * C + 8 * (tid + k * NT));
-  };
-  auto put_w1 = [&](_Float16* dst, const h8 (&r)[P1]) __attribute__((always_inline)) {
-#pragma unroll
-    for (int k = 0; k < P1; ++k) *reinterpret_cast<h8*>(dst + lw1 + k * (NT / (C / 8)) * S::W1P) = r[k];
-  };
-  auto put_w2 = [&](_Float16* dst, const h8 (&r)[P2]) __attribute__((always_inline)) {
-#pragma unroll
-    for (int k = 0; k < P2; ++k) *reinterpret_cast<h8*>(dst + lw2 + k * (NT / 4) * S::W2P) = r[k];
-  };
-  stage_vec(Gs, p.ln_s, C, 1.f, C, tid, NT);
-  stage_vec(Gs + C, p.ln_o, C, 0.f, C, tid, NT);
-#pragma unroll
-  for (int c = 0; c < 2; ++c) {   // chunks 0 and 1 (clamped) into buffer 0
-    h8 a1[P1], a2[P2];   // (native vector types: a struct array would be copied through scratch)
-    const _Float16* src = p.w + (size_t)(c < nch ? c : nch - 1) * S::CE;
-    load_w1(src, a1);
-    load_w2(src, a2);
-    put_w1(&Wb[0][c * S::BUF], a1);
-    put_w2(&Wb[0][c * S::BUF], a2);
-  }
-  FragTile<ACT, KS> xt[2];
-#pragma unroll
-  for (int rt = 0; rt < 2; ++rt) {
-    const long long row = std::min(row_base + rt * 16 + r16, (long long)p.rows - 1);
-    frag_load_row(xt[rt], p.x, (size_t)row, C, lane);
-  }
+  issue(0, W0, B0);
+  if (!p.b1g && tid < 64) B0[tid] = B1[tid] = 0.f;
+  stage_vec(Gs, p.ln_s, C, 1.f, C, tid, MLP_NT);
+  stage_vec(Gs + C, p.ln_o, C, 0.f, C, tid, MLP_NT);
+  stage_vec(Gs + 2 * C, p.b2, C, 0.f, C, tid, MLP_NT);
   __syncthreads();
-  h8 xf[2][KS];
-  frag_ln_raw2(xt[0], xt[1], xf[0], xf[1], C, Gs, Gs + C, p.eps, p.fast_var, lane);
-  __builtin_amdgcn_sched_barrier(0);   // the raw rows die before the accumulators are born
+  h8 xf[RT][KS];
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) {
+    const long long row = std::min(row_base + rt * 16 + r16, (long long)p.rows - 1);
+    FragTile<ACT, KS> xt;
+    frag_load_row(xt, p.x, (size_t)row, C, lane);
+    frag_ln_raw1(xt, xf[rt], C, Gs, Gs + C, p.eps, p.fast_var, lane);
+    __builtin_amdgcn_sched_barrier(0);   // one raw tile live at a time
+  }
 
-  f4 acc[2][CT];
+  f4 acc[RT][CT];
 #pragma unroll
   for (int ct = 0; ct < CT; ++ct) {
-    const float4 b = p.b2 ? *reinterpret_cast<const float4*>(p.b2 + ct * 16 + 4 * g4) : make_float4(0.f, 0.f, 0.f, 0.f);
-    acc[0][ct] = f4{b.x, b.y, b.z, b.w};
-    acc[1][ct] = acc[0][ct];
+    const f4 b = *reinterpret_cast<const f4*>(Gs + 2 * C + ct * 16 + 4 * g4);
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) acc[rt][ct] = b;
   }
 
-  for (int s = 0; s < nch; ++s) {
-    // chunk s in slot s % 2 of buffer (s / 2) % 2; chunk s + 2 goes to the same slot of the
-    // other buffer, which every wave left at the previous pair's barrier
-    const _Float16* cur = &Wb[(s >> 1) & 1][(s & 1) * S::BUF];
-    _Float16* nxt = &Wb[((s >> 1) & 1) ^ 1][(s & 1) * S::BUF];
-    // chunk s + 2's W1^T pieces now, its W2^T pieces after GEMM1 (the last pair reloads the
-    // last chunk into a buffer nothing reads again: loads stay unconditional)
-    const _Float16* src = p.w + (size_t)(s + 2 < nch ? s + 2 : nch - 1) * S::CE;
-    h8 n1[P1];
-    load_w1(src, n1);
-
-    // GEMM1: hacc[grp][rt][ht] = H^T tile (hidden 32s + 16ht + 4g4 + i, row r16)
-    f4 hacc[NG][2][2];
+  auto chunk = [&](int s, const _Float16* W, const float* B, _Float16* Wn, float* Bn) __attribute__((always_inline)) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();   // chunk s in LDS for every wave; every wave done with the other buffer
+    issue(min(s + 1, nch - 1), Wn, Bn);
+    const _Float16* cur = W + lane * 8;
+    const float* Bc = B + 4 * g4;
+    h8 fr[2][4];
 #pragma unroll
-    for (int grp = 0; grp < NG; ++grp) {
-      const float* b1 = grp == 0 ? p.b1g : p.b1v;
+    for (int t = 0; t < 4; ++t) fr[0][t] = *reinterpret_cast<const h8*>(cur + t * 512);
+    // GEMM1: hacc[grp][rt][ht] = H^T tile (hidden 32s + 16ht + 4g4 + i, row r16)
+    f4 hacc[NG][RT][2];
+#pragma unroll
+    for (int grp = 0; grp < NG; ++grp)
 #pragma unroll
       for (int ht = 0; ht < 2; ++ht) {
-        const float4 b =
-            b1 ? *reinterpret_cast<const float4*>(b1 + s * MLP_HC + ht * 16 + 4 * g4) : make_float4(0.f, 0.f, 0.f, 0.f);
-        hacc[grp][0][ht] = f4{b.x, b.y, b.z, b.w};
-        hacc[grp][1][ht] = hacc[grp][0][ht];
+        const f4 b = *reinterpret_cast<const f4*>(Bc + grp * 32 + ht * 16);
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) hacc[grp][rt][ht] = b;
       }
-    }
+    h8 hb[RT];
 #pragma unroll
-    for (int j = 0; j < KS; ++j) {
-      h8 wa[NG][2];
+    for (int f = 0; f < NF; f += 4) {
+      // the next group of fragments is read while this group's products run
+      if (f + 4 < NF) {
 #pragma unroll
-      for (int grp = 0; grp < NG; ++grp)
+        for (int t = 0; t < 4; ++t) fr[(f / 4 + 1) & 1][t] = *reinterpret_cast<const h8*>(cur + (f + 4 + t) * 512);
+      }
+      if (f == F1) {
+        // activation -> GEMM2 B fragments (k order: hidden 4g4 + i, then 16 + 4g4 + i).  The wait
+        // covers a product whose addend comes from the product just before it: it ends later
+        // than the wait states the compiler leaves before a vector instruction reads it
+        asm volatile("s_nop 15" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int ht = 0; ht < 2; ++ht)
-          wa[grp][ht] = *reinterpret_cast<const h8*>(cur + (grp * MLP_HC + ht * 16 + r16) * S::W1P + 32 * j + 8 * g4);
+        for (int rt = 0; rt < RT; ++rt) {
+          f8 v;
 #pragma unroll
-      for (int grp = 0; grp < NG; ++grp)
-#pragma unroll
-        for (int ht = 0; ht < 2; ++ht)
-#pragma unroll
-          for (int rt = 0; rt < 2; ++rt) hacc[grp][rt][ht] = mfma16(wa[grp][ht], xf[rt][j], hacc[grp][rt][ht]);
-    }
-    // activation -> GEMM2 B fragments (k order: hidden 4g4 + i, then 16 + 4g4 + i)
-    h8 hb[2];
-#pragma unroll
-    for (int rt = 0; rt < 2; ++rt)
-#pragma unroll
-      for (int ht = 0; ht < 2; ++ht)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          float v;
-          if constexpr (NG == 1) {
-            v = fmaxf(hacc[0][rt][ht][i], 0.f);
-          } else {
-            const float gt = hacc[0][rt][ht][i];
-            v = gt * sigmoidf_(gt) * hacc[1][rt][ht][i];
+          for (int e = 0; e < 8; ++e) {
+            v[e] = hacc[0][rt][e >> 2][e & 3];
+            if constexpr (NG == 2) v[e] *= sigmoidf_(v[e]) * hacc[NG - 1][rt][e >> 2][e & 3];
           }
-          hb[rt][4 * ht + i] = (_Float16)v;
+          hb[rt] = __builtin_convertvector(v, h8);
+          if constexpr (NG == 1) hb[rt] = __builtin_elementwise_max(hb[rt], (h8)(_Float16)0.f);   // rounding keeps the sign
         }
-    put_w1(nxt, n1);
-    h8 n2[P2];
-    load_w2(src, n2);
-    __builtin_amdgcn_sched_barrier(0);
-    // GEMM2, four output tiles at a time
+      }
 #pragma unroll
-    for (int c4 = 0; c4 < CT; c4 += 4) {
-      h8 wb[4];
+      for (int t = 0; t < 4; ++t) {
+        const h8 w = fr[(f / 4) & 1][t];
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
-        wb[t] = *reinterpret_cast<const h8*>(cur + S::W1E + ((c4 + t) * 16 + r16) * S::W2P + 8 * g4);
-#pragma unroll
-      for (int t = 0; t < 4; ++t)
-#pragma unroll
-        for (int rt = 0; rt < 2; ++rt) acc[rt][c4 + t] = mfma16(wb[t], hb[rt], acc[rt][c4 + t]);
+        for (int rt = 0; rt < RT; ++rt) {
+          if (f < F1) {
+            const int q = f + t, j = q / (2 * NG), grp = q / 2 % NG, ht = q & 1;
+            hacc[grp][rt][ht] = mfma16(w, xf[rt][j], hacc[grp][rt][ht]);
+          } else {
+            const int ct = f + t - F1;
+            acc[rt][ct] = mfma16(w, hb[rt], acc[rt][ct]);
+          }
+        }
+      }
       __builtin_amdgcn_sched_barrier(0);
     }
-    put_w2(nxt, n2);
-    if (s & 1) __syncthreads();   // block-uniform: the pair's reads done, the next pair's writes visible
+  };
+  for (int s = 0;;) {
+    chunk(s, W0, B0, W1, B1);
+    if (++s == nch) break;
+    chunk(s, W1, B1, W0, B0);
+    if (++s == nch) break;
   }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the last copy, which nothing reads
 
   // residual and store: lane -> row r16 of tile rt, channels 16ct + 4g4 .. +3
 #pragma unroll
-  for (int rt = 0; rt < 2; ++rt) {
+  for (int rt = 0; rt < RT; ++rt) {
     const long long row = row_base + rt * 16 + r16;
     if (row >= p.rows) continue;
 #pragma unroll
-    for (int ct = 0; ct < CT; ++ct) {
-      const size_t idx = (size_t)row * C + ct * 16 + 4 * g4;
-      float v[4] = {acc[rt][ct][0], acc[rt][ct][1], acc[rt][ct][2], acc[rt][ct][3]};
+    for (int c4 = 0; c4 < CT; c4 += 4) {   // four tiles' residual in flight at a time
+      float r[4][4];
+      for (int t = 0; t < 4; ++t)
+        for (int i = 0; i < 4; ++i) r[t][i] = 0.f;
       if (p.accumulate) {
-        float r[4];
-        ld4v<ACT>(p.x, idx, r);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] += r[i];
+        for (int t = 0; t < 4; ++t) ld4v<ACT>(p.x, (size_t)row * C + (c4 + t) * 16 + 4 * g4, r[t]);
       }
-      st4v<ACT>(p.out, idx, v);
-      __builtin_amdgcn_sched_barrier(0);   // one tile's residual in flight at a time
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const f4 a = acc[rt][c4 + t];
+        const float v[4] = {a[0] + r[t][0], a[1] + r[t][1], a[2] + r[t][2], a[3] + r[t][3]};
+        st4v<ACT>(p.out, (size_t)row * C + (c4 + t) * 16 + 4 * g4, v);
+      }
+      __builtin_amdgcn_sched_barrier(0);
     }
   }
 }
@@ -271,14 +258,23 @@ size_t mlp_packed_bytes(int C, int H, bool swiglu) {
   return (size_t)(H / MLP_HC) * (size_t)((swiglu ? 2 : 1) * MLP_HC + MLP_HC) * C * sizeof(_Float16);
 }
 
+template <int ACT, int C, int NG>
+static void launch_mlp(lf_context* ctx, const MlpParams& mp) {
+  // Rows a wave: 32 read a weight fragment from LDS once for two products, but need two blocks of
+  // 128 rows on every CU; below that 16 leave fewer CUs idle.  Measured 16 against 32: 8192 rows of
+  // 256, bf16 34 / 43 us, 25578 of 256, f32 50 / 55, 41209 of 128 with SwiGLU, f32 34 / 40; 65536 of
+  // 128, bf16 30.5 / 28.5, 196608 of 256, f32 290 / 258.
+  const int rt = mp.rows >= 2LL * ctx->num_cus * 32 * MLP_WAVES ? 2 : 1;
+  const dim3 grid((unsigned)((mp.rows + 16 * rt * MLP_WAVES - 1) / (16 * rt * MLP_WAVES)));
+  auto k = rt == 2 ? mlp_kernel<ACT, C, NG, 2> : mlp_kernel<ACT, C, NG, 1>;
+  hipLaunchKernelGGL(k, grid, dim3(MLP_NT), 0, ctx->stream, mp);
+}
+
 template <int ACT>
-static void launch_mlp(lf_context* ctx, const MlpParams& mp, int C, bool swiglu, dim3 grid) {
-  if (C == 256)
-    hipLaunchKernelGGL((mlp_kernel<ACT, 256, 1>), grid, dim3(64 * MLP_WAVES), 0, ctx->stream, mp);
-  else if (swiglu)
-    hipLaunchKernelGGL((mlp_kernel<ACT, 128, 2>), grid, dim3(64 * MLP_WAVES), 0, ctx->stream, mp);
-  else
-    hipLaunchKernelGGL((mlp_kernel<ACT, 128, 1>), grid, dim3(64 * MLP_WAVES), 0, ctx->stream, mp);
+static void launch_mlp(lf_context* ctx, const MlpParams& mp, int C, bool swiglu) {
+  if (C == 256) launch_mlp<ACT, 256, 1>(ctx, mp);
+  else if (swiglu) launch_mlp<ACT, 128, 2>(ctx, mp);
+  else launch_mlp<ACT, 128, 1>(ctx, mp);
 }
 
 int transition_fused(lf_context* ctx, const lf_transition_args& a, const WView* views, void* packed) {
@@ -308,12 +304,11 @@ int transition_fused(lf_context* ctx, const lf_transition_args& a, const WView* 
   mp.b1g = w.b1;
   mp.b1v = swiglu && w.b1 ? w.b1 + H : nullptr;
   mp.b2 = w.b2;
-  const dim3 grid((unsigned)((a.rows + MLP_ROWS - 1) / MLP_ROWS));
   {
     LaunchScope ls(ctx, "transition.fused");
-    if (a.act_dtype == LF_F32) launch_mlp<DT_F32>(ctx, mp, C, swiglu, grid);
-    else if (a.act_dtype == LF_F16) launch_mlp<DT_F16>(ctx, mp, C, swiglu, grid);
-    else launch_mlp<DT_BF16>(ctx, mp, C, swiglu, grid);
+    if (a.act_dtype == LF_F32) launch_mlp<DT_F32>(ctx, mp, C, swiglu);
+    else if (a.act_dtype == LF_F16) launch_mlp<DT_F16>(ctx, mp, C, swiglu);
+    else launch_mlp<DT_BF16>(ctx, mp, C, swiglu);
   }
   return check_hip(hipGetLastError(), "transition fused launch");
 }

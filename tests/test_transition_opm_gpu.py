@@ -93,6 +93,41 @@ def test_transition_swiglu(ctx, c, n):
     H.assert_close(xt.cpu().numpy(), ref, label=f"swiglu {c}")
 
 
+@pytest.mark.parametrize("c,kind,dt", [(256, "relu", "float32"), (256, "relu", "bfloat16"), (128, "relu", "float32"),
+                                       (128, "swiglu", "float32")])
+def test_transition_fused_many_rows(ctx, c, kind, dt):
+    """Row counts around the change from 16 to 32 rows a wave (two blocks of 128 rows a compute
+    unit), with a partial last block, without the residual: the rows at both ends and in the middle
+    against the oracle, which takes every row by itself."""
+    import torch
+    from localfold_amd import capi, device as D
+    hidden = 96 if kind == "relu" else 4 * c
+    st = S.Stream(c + 3)
+    if kind == "relu":
+        w = {"layerNormScale": st.values(c, 0.2, 1), "layerNormOffset": st.values(c, 0.1),
+             "firstWeight": st.normal(c * hidden, 1 / np.sqrt(c)).reshape(c, hidden), "firstBias": st.values(hidden, 0.1),
+             "secondWeight": st.normal(hidden * c, 1 / np.sqrt(hidden)).reshape(hidden, c),
+             "secondBias": st.values(c, 0.05)}
+    else:
+        w = {"inputLayerNormScale": st.values(c, 0.2, 1.0), "inputLayerNormOffset": st.values(c, 0.1),
+             "transition1": st.normal(c * 2 * hidden, 1 / np.sqrt(c)).reshape(c, 2 * hidden),
+             "transition2": st.normal(hidden * c, 1 / np.sqrt(hidden)).reshape(hidden, c)}
+    edge = 2 * torch.cuda.get_device_properties(ctx.device).multi_processor_count * 128
+    base = st.values(4096 * c, 1.5).reshape(4096, c)
+    code = capi.LF_TRANSITION_RELU if kind == "relu" else capi.LF_TRANSITION_SWIGLU
+    dw = D.DeviceWeights(ctx.device)
+    ws = D.transition_weights(dw, w, code)
+    for rows in (edge - 1, edge + 37):
+        rot = np.arange(rows) % 4095   # a period that no block size divides
+        xt = _dev(ctx, base, getattr(torch, dt))[torch.as_tensor(rot).to(ctx.device)].contiguous()
+        pick = np.unique(np.concatenate([np.arange(70), np.arange(rows // 2, rows // 2 + 70), np.arange(rows - 140, rows)]))
+        x16 = xt[torch.as_tensor(pick).to(ctx.device)].float().cpu().numpy()
+        out = D.transition(ctx, xt, ws, hidden, code, fast_variance=kind == "swiglu")
+        got = out[torch.as_tensor(pick).to(ctx.device)].float().cpu().numpy()
+        ref = (ops.transition_af2 if kind == "relu" else ops.transition_af3)(x16, w)
+        H.assert_close(got, ref, label=f"c={c} {kind} {dt} rows={rows}")
+
+
 @pytest.mark.parametrize("s,n", [(1, 16), (5, 37), (16, 64), (64, 96), (128, 64)])
 def test_opm_af2(ctx, blockw, s, n):
     import torch
