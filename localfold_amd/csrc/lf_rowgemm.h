@@ -92,6 +92,8 @@ struct RowGemmParams {
   int wview;
   const float* bias;  // [N] nullable
   int op;             // OP_STORE or OP_RELU
+  const float* amul;    // [amulN][K]: row r of A is multiplied by row r % amulN and rounded to f16 again
+  int amulN;            // (nullable; weight-resident form with K = 64 only)
   const float* rowden;  // divide row r by rowden[r] (nullable; OPM's norm_eps + sum_s m_si m_sj)
   const void* resid;  // residual added when non-null (same layout and dtype as dst)
   Dst dst;

@@ -649,7 +649,8 @@ __global__ __launch_bounds__(512) void rowgemm_kernel(RowGemmParams p) {
 }
 
 // Weight-resident form for K = 32 KS <= 256 and N = 64 NP <= 256 (the attention output
-// projections): a block stages the whole W (N x K f16, up to 132 KB) in LDS once -- copied from
+// projections; K = N = 64 for global column attention, where the streamed form's 128-column tiles
+// leave half of its waves without a column): a block stages the whole W (N x K f16, up to 132 KB) in LDS once -- copied from
 // the f16 expansion, or decoded from the stored codes (int8 / int5 / f16 runs, the codec
 // arithmetic of lf_gemm.h) -- and
 // each of its 8 waves then walks 16-row tiles w, w + nw, ... with no block barrier.  A tile's
@@ -658,7 +659,9 @@ __global__ __launch_bounds__(512) void rowgemm_kernel(RowGemmParams p) {
 // the columns run in passes of 64 (4 accumulator tiles), each followed by its epilogue.
 // W is the MFMA A operand, so a lane holds 4 consecutive columns of one row: one 8- or
 // 16-byte store per column tile.  Rows past the end are clamped for the loads and not stored.
-template <int DACT, int KS, int NP, int NWV>
+// MUL: the rows of A are multiplied by p.amul on the way in (global column attention's gate by its
+// column's attended values: as a pass of its own that read and wrote the gate once more).
+template <int DACT, int KS, int NP, int NWV, bool MUL>
 __global__ __launch_bounds__(64 * NWV) void rowgemm_res_kernel(RowGemmParams p) {
   constexpr int NT = 64 * NWV, K = 32 * KS, N = 64 * NP, LDW = K + 8;
   __shared__ __attribute__((aligned(16))) _Float16 Ws[N * LDW];
@@ -666,15 +669,28 @@ __global__ __launch_bounds__(64 * NWV) void rowgemm_res_kernel(RowGemmParams p) 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int r16 = lane & 15, g4 = lane >> 4, kq = g4 * 8;
   const int ntiles = (p.rows + 15) >> 4, nw = (int)gridDim.x * NWV;
+  typedef float f8 __attribute__((ext_vector_type(8)));
+  f8 am[MUL ? KS : 1];
   auto aload = [&](int tl, h8 (&a)[KS]) __attribute__((always_inline)) {
     const int row = min(tl * 16 + r16, p.rows - 1);
     const _Float16* ar = p.A + (size_t)row * p.K + kq;
 #pragma unroll
     for (int j = 0; j < KS; ++j) a[j] = *reinterpret_cast<const h8*>(ar + 32 * j);
+    if constexpr (MUL) {
+      const float* mr = p.amul + (size_t)(row % p.amulN) * p.K + kq;
+#pragma unroll
+      for (int j = 0; j < KS; ++j) am[j] = *reinterpret_cast<const f8*>(mr + 32 * j);
+    }
+  };
+  auto scaled = [&](const h8& v, int j) __attribute__((always_inline)) {
+    if constexpr (MUL) return __builtin_convertvector(__builtin_convertvector(v, f8) * am[j], h8);
+    else return v;
   };
   int tile = (int)blockIdx.x * NWV + wave;
   h8 a[KS];
   aload(tile < ntiles ? tile : 0, a);
+#pragma unroll
+  for (int j = 0; j < KS; ++j) a[j] = scaled(a[j], j);
   if (p.wview) {
     // the whole W decoded from its stored codes (zeros past the view's columns)
     stage_view(Ws, LDW, p.wv, N, 0, K, 1.f, tid, NT);
@@ -744,29 +760,29 @@ __global__ __launch_bounds__(64 * NWV) void rowgemm_res_kernel(RowGemmParams p) 
       __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
-    for (int j = 0; j < KS; ++j) a[j] = an[j];
+    for (int j = 0; j < KS; ++j) a[j] = scaled(an[j], j);
   }
 }
 
 // As many blocks as are resident at once (the tiles are dealt out by block id, so every
 // launched block must be resident together).
-template <int DACT, int KS, int NP>
+template <int DACT, int KS, int NP, bool MUL = false>
 static void launch_rowgemm_res(lf_context* ctx, const RowGemmParams& p) {
   constexpr int NWV = 8;   // 12 measured no faster in the N = 384 Evoformer block, 16 slower
   static const int per_cu = [] {
     int n = 1;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, rowgemm_res_kernel<DACT, KS, NP, NWV>, 64 * NWV, 0) !=
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, rowgemm_res_kernel<DACT, KS, NP, NWV, MUL>, 64 * NWV, 0) !=
         hipSuccess)
       n = 1;
     return n < 1 ? 1 : n;
   }();
   const dim3 g((unsigned)std::min((p.rows + 16 * NWV - 1) / (16 * NWV), per_cu * ctx->num_cus));
-  hipLaunchKernelGGL((rowgemm_res_kernel<DACT, KS, NP, NWV>), g, dim3(64 * NWV), 0, ctx->stream, p);
+  hipLaunchKernelGGL((rowgemm_res_kernel<DACT, KS, NP, NWV, MUL>), g, dim3(64 * NWV), 0, ctx->stream, p);
 }
 
 bool rowgemm_resident(const lf_context* ctx, int rows, int K, int N, const Dst& dst) {
   const int np = N / 64, ks = K / 32;
-  return N % 64 == 0 && K % 32 == 0 && (np == 2 || np == 4) && (ks == 4 || ks == 8) && dst.D >= 64 * np &&
+  return N % 64 == 0 && K % 32 == 0 && (((np == 2 || np == 4) && (ks == 4 || ks == 8)) || (np == 1 && ks == 2)) && dst.D >= 64 * np &&
          (rows + 15) / 16 >= 8 * ctx->num_cus;
 }
 
@@ -783,11 +799,14 @@ int launch_rowgemm(lf_context* ctx, const RowGemmParams& p, const char* label) {
   // weight-resident form: the whole W in LDS, N and K whole multiples of the tiles
   const int np = p.N / 64, ks = p.K / 32;
   const bool resident = rowgemm_resident(ctx, p.rows, p.K, p.N, p.dst);
+  if (p.amul && !(resident && np == 1)) return set_error(LF_ERR_INVALID, l + ": row factors need the weight-resident form, K = 64");
   if (p.wview && !resident) return set_error(LF_ERR_INVALID, l + ": stored weights need the weight-resident form");
   if (resident && (p.wview || p.w.kp >= p.K)) {
 #define LF_RR(D, KS_, NP_) launch_rowgemm_res<D, KS_, NP_>(ctx, p)
 #define LF_RRD(D)                                      \
-  if (ks == 4 && np == 2) LF_RR(D, 4, 2);               \
+  if (np == 1 && p.amul) launch_rowgemm_res<D, 2, 1, true>(ctx, p); \
+  else if (np == 1) LF_RR(D, 2, 1);                     \
+  else if (ks == 4 && np == 2) LF_RR(D, 4, 2);          \
   else if (ks == 4) LF_RR(D, 4, 4);                     \
   else if (np == 2) LF_RR(D, 8, 2);                     \
   else LF_RR(D, 8, 4);

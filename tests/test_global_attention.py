@@ -101,6 +101,28 @@ def test_global_column_attention(ctx, s, n, c, heads, dt):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("s,n,heads,dt,accumulate", [(1030, 32, 8, "float32", False), (1030, 32, 4, "bfloat16", True),
+                                                     (993, 33, 8, "float32", True), (992, 33, 2, "float16", False)])
+def test_global_column_attention_many_rows(ctx, s, n, heads, dt, accumulate):
+    """Both sides of the 32768 rows from which the output kernel holds its weights and multiplies the
+    gate by the attended values itself (993 x 33 = 32769, 992 x 33 just below), with and without the
+    residual, with a partial last tile of 16 rows."""
+    import torch
+    from localfold_amd import device as D
+    g, msa, mask = _inputs(s, n, 64, heads, s + n)
+    dw = D.DeviceWeights(ctx.device)
+    ws = D.global_attention_weights(dw, g["attention"])
+    x = _dev(ctx, msa, getattr(torch, dt))
+    x0 = x.float().cpu().numpy()
+    out = D.global_column_attention(ctx, x, _dev(ctx, mask), ws, heads, accumulate=accumulate)
+    torch.cuda.synchronize()
+    ref = ops.global_column_attention_af2(x0, mask, g["attention"], heads)
+    # bfloat16 keeps 8 bits: half an ulp of the largest output (below 8) is 2^-7
+    tol = {"max_abs": H.MAX_ABS + 2.0 ** -7} if dt == "bfloat16" else {}
+    H.assert_close(out.float().cpu().numpy(), ref + x0 if accumulate else ref, label=f"global {s}x{n} {dt}", **tol)
+
+
+@pytest.mark.gpu
 def test_global_column_attention_in_place(ctx):
     import torch
     from localfold_amd import device as D
