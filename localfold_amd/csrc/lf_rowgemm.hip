@@ -648,6 +648,60 @@ __global__ __launch_bounds__(512) void rowgemm_kernel(RowGemmParams p) {
   }
 }
 
+// Few rows (the single track): a block of four waves takes 16 rows x 32 columns and splits K, wave w
+// the k-steps w, w + 4, ...; the operands come straight from the caches as MFMA fragments with no
+// barrier in the loop, so several steps' loads are in flight, and the partial sums meet in LDS.
+// The streamed form waits once a 64-deep slice for its loads, in a handful of blocks: 512 rows,
+// K = 1536, N = 384, bf16 took 45 us, here 12.5.
+constexpr int RS_LD = 36;   // pitch of a row of 32 partial sums
+template <int DACT>
+__global__ __launch_bounds__(256) void rowgemm_small_kernel(RowGemmParams p) {
+  __shared__ __attribute__((aligned(16))) float red[4][16 * RS_LD];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int r16 = lane & 15, g4 = lane >> 4, kq = g4 * 8;
+  const int row0 = (int)blockIdx.x * 16, col0 = (int)blockIdx.y * 32;
+  const int nsteps = (p.K + 31) >> 5;
+  // rows and columns past the end are clamped for the loads and not stored
+  const _Float16* ar = p.A + (size_t)min(row0 + r16, p.rows - 1) * p.K;
+  const _Float16* wr[2];
+#pragma unroll
+  for (int t = 0; t < 2; ++t) wr[t] = p.w.p + (size_t)min(col0 + 16 * t + r16, p.w.N - 1) * p.w.kp + kq;
+  f4 acc[2] = {f4{0.f, 0.f, 0.f, 0.f}, f4{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll 6
+  for (int j = wave; j < nsteps; j += 4) {
+    const int k = 32 * j + kq;   // K is a multiple of 8; the weights are zero from K to kp
+    h8 a = *reinterpret_cast<const h8*>(ar + min(k, p.K - 8));
+    const h8 w0 = *reinterpret_cast<const h8*>(wr[0] + 32 * j), w1 = *reinterpret_cast<const h8*>(wr[1] + 32 * j);
+    if (k >= p.K) a = h8{0, 0, 0, 0, 0, 0, 0, 0};
+    acc[0] = mfma16(w0, a, acc[0]);
+    acc[1] = mfma16(w1, a, acc[1]);
+  }
+  // a chain of products whose last one feeds a store: longer than the compiler's wait states
+  asm volatile("s_nop 15" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int t = 0; t < 2; ++t) *reinterpret_cast<f4*>(&red[wave][r16 * RS_LD + 16 * t + 4 * g4]) = acc[t];
+  __syncthreads();
+  const int r = tid >> 3, cl = (tid & 7) * 4, row = row0 + r, c = col0 + cl;
+  if (tid >= 128 || row >= p.rows || c >= p.N) return;
+  f4 s = *reinterpret_cast<const f4*>(&red[0][r * RS_LD + cl]);
+#pragma unroll
+  for (int w = 1; w < 4; ++w) s += *reinterpret_cast<const f4*>(&red[w][r * RS_LD + cl]);
+  const unsigned q = (unsigned)p.dst.Q;
+  const unsigned b = (unsigned)row / q, n = (unsigned)row - b * q;
+  const int at = (int)b * (int)p.dst.sB + (int)n * (int)p.dst.sN + c;
+  const float inv = p.rowden ? 1.f / p.rowden[row] : 1.f;
+  float res[4] = {0.f, 0.f, 0.f, 0.f}, v[4];
+  if (p.resid) ld4<DACT>(p.resid, at, res);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    float y = s[i] + (p.bias ? p.bias[c + i] : 0.f);
+    if (p.op == OP_RELU) y = fmaxf(y, 0.f);
+    v[i] = y * inv + res[i];
+  }
+  st4<DACT>(p.dst.ptr, at, v);
+}
+
 // Weight-resident form for K = 32 KS <= 256 and N = 64 NP <= 256 (the attention output
 // projections; K = N = 64 for global column attention, where the streamed form's 128-column tiles
 // leave half of its waves without a column): a block stages the whole W (N x K f16, up to 132 KB) in LDS once -- copied from
@@ -819,6 +873,15 @@ int launch_rowgemm(lf_context* ctx, const RowGemmParams& p, const char* label) {
   }
   const int nt = p.N <= 128 ? 4 : 8;
   dim3 grid((p.rows + 127) / 128, (p.N + 32 * nt - 1) / (32 * nt));
+  // few blocks: the split-K form.  K = 1536, N = 384, bf16, split against streamed: 16 rows 9.5 / 33 us,
+  // 512 12.5 / 45, 1000 17 / 43, 2048 (32 blocks here) 28 / 43, 3000 (48 blocks) 44 / 43
+  if ((long long)grid.x * grid.y * 8 <= ctx->num_cus) {
+    const dim3 sg((p.rows + 15) / 16, (p.N + 31) / 32);
+    if (d.dtype == DT_F32) hipLaunchKernelGGL(rowgemm_small_kernel<DT_F32>, sg, dim3(256), 0, ctx->stream, p);
+    else if (d.dtype == DT_F16) hipLaunchKernelGGL(rowgemm_small_kernel<DT_F16>, sg, dim3(256), 0, ctx->stream, p);
+    else hipLaunchKernelGGL(rowgemm_small_kernel<DT_BF16>, sg, dim3(256), 0, ctx->stream, p);
+    return check_hip(hipGetLastError(), label);
+  }
 #define LF_RG(D, T) hipLaunchKernelGGL((rowgemm_kernel<D, T>), grid, dim3(512), 0, ctx->stream, p)
   if (d.dtype == DT_F32) { if (nt == 4) LF_RG(DT_F32, 4); else LF_RG(DT_F32, 8); }
   else if (d.dtype == DT_F16) { if (nt == 4) LF_RG(DT_F16, 4); else LF_RG(DT_F16, 8); }

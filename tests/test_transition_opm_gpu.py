@@ -128,6 +128,27 @@ def test_transition_fused_many_rows(ctx, c, kind, dt):
         H.assert_close(got, ref, label=f"c={c} {kind} {dt} rows={rows}")
 
 
+@pytest.mark.parametrize("c,hidden,rows,dt", [(384, 1536, 17, "float32"), (36, 200, 1, "float32"),
+                                              (36, 200, 45, "float16"), (100, 72, 4096, "float32"),
+                                              (100, 72, 4097, "float32")])
+def test_transition_few_rows(ctx, c, hidden, rows, dt):
+    """The output product of the unfused widths in its split-K form (up to 32 tiles of 128 rows: 4096
+    is the last with one column tile): partial row, column and k tiles, with the residual."""
+    import torch
+    from localfold_amd import device as D
+    st = S.Stream(c + rows)
+    w = {"layerNormScale": st.values(c, 0.2, 1), "layerNormOffset": st.values(c, 0.1),
+         "firstWeight": st.normal(c * hidden, 1 / np.sqrt(c)).reshape(c, hidden), "firstBias": st.values(hidden, 0.1),
+         "secondWeight": st.normal(hidden * c, 1 / np.sqrt(hidden)).reshape(hidden, c),
+         "secondBias": st.values(c, 0.05)}
+    x = _dev(ctx, st.values(rows * c, 1.5).reshape(rows, c), getattr(torch, dt))
+    dw = D.DeviceWeights(ctx.device)
+    out = D.transition(ctx, x, D.transition_weights(dw, w), hidden, accumulate=True)
+    torch.cuda.synchronize()
+    x0 = x.float().cpu().numpy()
+    H.assert_close(out.float().cpu().numpy(), x0 + ops.transition_af2(x0, w), label=f"c={c} hidden={hidden} rows={rows} {dt}")
+
+
 @pytest.mark.parametrize("s,n", [(1, 16), (5, 37), (16, 64), (64, 96), (128, 64)])
 def test_opm_af2(ctx, blockw, s, n):
     import torch
