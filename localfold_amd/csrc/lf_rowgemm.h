@@ -68,7 +68,7 @@ struct LnProjParams {
   int rmN;            // when > 0: a batch holds rmN <= rmQ rows and is padded to rmQ; storage row
                       // q*rmB + b or b*rmN + q.  A padding row repeats the last one (times zero with
                       // OP_ROWMASK): it is stored, so every destination has room for rmQ rows.
-                      // With rmQ a multiple of 4 (lnproj_pad) the four rows or columns of a lane
+                      // With rmQ a multiple of 4 the four rows or columns of a lane
                       // never straddle a batch and every store is a vector, whatever rmN is
   long long span_slack;   // elements that padded rows add to a destination beyond its limit of 2^31
   const float *ln_s, *ln_o;
@@ -103,7 +103,6 @@ struct RowGemmParams {
 // workspace of lnproj_packed_bytes(p) bytes for the decoded weights; repeated launches with
 // the same weights (row chunks) pass decode = false after the first.
 size_t lnproj_packed_bytes(const LnProjParams& p);
-inline int lnproj_pad(int rows) { return (rows + 3) & ~3; }
 // Whether launch_rowgemm takes the weight-resident form for this shape: then the caller may
 // pass the stored weights (RowGemmParams::wv, wview = 1) instead of an f16 expansion, and each
 // block decodes them into LDS once.
