@@ -768,8 +768,9 @@ __global__ __launch_bounds__(1024) void flash_res_kernel(FlashParams p) {
   // 4*NDT consecutive ones: its gate and its output are one vector each
   const _Float16* vl = Vs + (4 * NDT * (r16 >> 2) + (r16 & 3)) * VLD + 8 * g4;
   // The pair bias of the lane's query: keys 8*g4 .. +7 of a chunk's two halves (fragment order,
-  // tiled_at: 1 KB per load in lane order; queries and keys past Q are in the buffer, unwritten,
-  // and not used)
+  // tiled_at: 1 KB per load in lane order).  Queries and keys past Q are in the buffer, unwritten: a
+  // query's garbage stays in its own column of the scores, a key's would reach the other keys of its
+  // tile through the identity product (0 * NaN) and is cleared or left out before that
   struct Bias {
     h8 lo, hi;
   };
@@ -847,29 +848,38 @@ __global__ __launch_bounds__(1024) void flash_res_kernel(FlashParams p) {
         bias_load(bn, c + 1 < nke ? brow + (c + 1) * (16 * FA_KC) : bnext);
         __builtin_amdgcn_sched_barrier(0);
       }
-      h4 bq[4];
-      if (BIAS) {
-        bq[0] = h4{bc.lo[0], bc.lo[1], bc.lo[2], bc.lo[3]};
-        bq[1] = h4{bc.lo[4], bc.lo[5], bc.lo[6], bc.lo[7]};
-        bq[2] = h4{bc.hi[0], bc.hi[1], bc.hi[2], bc.hi[3]};
-        bq[3] = h4{bc.hi[4], bc.hi[5], bc.hi[6], bc.hi[7]};
-      }
       f4 s[4];
       float lc;
-      // the chunk's masked keys, as all-ones or zero halves in the order of p
+      // the chunk's masked keys and those past Q, as zero halves among all-ones in the order of p
       const bool clear = (cmask >> c) & 1;   // uniform
       const uint16_t* km = Km + c * FA_KC + 8 * g4;
+      auto keep_keys = [&](h8 v, int kh2) __attribute__((always_inline)) {
+        return __builtin_bit_cast(h8, __builtin_bit_cast(u32x4, v) & *reinterpret_cast<const u32x4*>(km + 32 * kh2));
+      };
+      h4 bq[4];
+      if (BIAS) {
+        h8 lo = bc.lo, hi = bc.hi;
+        if (__builtin_expect(clear, 0)) {
+          lo = keep_keys(lo, 0);
+          hi = keep_keys(hi, 1);
+        }
+        bq[0] = h4{lo[0], lo[1], lo[2], lo[3]};
+        bq[1] = h4{lo[4], lo[5], lo[6], lo[7]};
+        bq[2] = h4{hi[0], hi[1], hi[2], hi[3]};
+        bq[3] = h4{hi[4], hi[5], hi[6], hi[7]};
+      }
       h8 pf[2];
       // s = x + cm: the bias lands through an identity MFMA (D = I B + C, B = the lane's bias h4 in
-      // the accumulator layout)
-      auto scores = [&](const f4& cm) __attribute__((always_inline)) {
+      // the accumulator layout).  General chunks add it themselves, key by key
+      auto scores = [&](const f4& cm, auto bias_tag) __attribute__((always_inline)) {
+        constexpr bool MBIAS = decltype(bias_tag)::value;
 #pragma unroll
-        for (int kt = 0; kt < 4; ++kt) s[kt] = BIAS ? mfma16k16(ident, bq[kt], cm) : cm;
+        for (int kt = 0; kt < 4; ++kt) s[kt] = MBIAS ? mfma16k16(ident, bq[kt], cm) : cm;
         // (a product that accumulates onto one issued just before it finishes later than the wait
         // states the compiler leaves before a VALU read of it: with the bias and score products
         // of a tile back to back the exponentials read stale scores.  In two groups, each
         // accumulates onto a product three issues old)
-        if (BIAS) __builtin_amdgcn_sched_barrier(0);
+        if (MBIAS) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int kt = 0; kt < 4; ++kt) s[kt] = qk_mfma(kf[kt], qf, s[kt]);
       };
@@ -881,9 +891,7 @@ __global__ __launch_bounds__(1024) void flash_res_kernel(FlashParams p) {
           for (int i = 0; i < 4; ++i) pf[kt >> 1][4 * (kt & 1) + i] = (_Float16)__builtin_amdgcn_exp2f(s[kt][i]);
         if (__builtin_expect(clear, 0)) {
 #pragma unroll
-          for (int kh2 = 0; kh2 < 2; ++kh2)
-            pf[kh2] = __builtin_bit_cast(h8, __builtin_bit_cast(u32x4, pf[kh2]) &
-                                                 *reinterpret_cast<const u32x4*>(km + 32 * kh2));
+          for (int kh2 = 0; kh2 < 2; ++kh2) pf[kh2] = keep_keys(pf[kh2], kh2);
         }
         // (two independent products: see scores)
         const f4 l0 = mfma16(ones, pf[0], f4{0.f, 0.f, 0.f, 0.f}), l1 = mfma16(ones, pf[1], f4{0.f, 0.f, 0.f, 0.f});
@@ -908,7 +916,7 @@ __global__ __launch_bounds__(1024) void flash_res_kernel(FlashParams p) {
         for (int dt = 0; dt < NDT; ++dt) o[dt] = o[dt] * corr;
       };
       if (GEN && ((gmask >> c) & 1)) {   // uniform: the clamp and the full update
-        scores(f4{0.f, 0.f, 0.f, 0.f});
+        scores(f4{0.f, 0.f, 0.f, 0.f}, std::false_type{});
 #pragma unroll
         for (int kt = 0; kt < 4; ++kt) {
           const float4 kb4 =
@@ -916,7 +924,8 @@ __global__ __launch_bounds__(1024) void flash_res_kernel(FlashParams p) {
           const float kbv[4] = {kb4.x, kb4.y, kb4.z, kb4.w};
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            const float x = s[kt][i] + kbv[i];
+            float x = s[kt][i] + kbv[i];
+            if (BIAS) x = bias_add(bq[kt], i, x);
             // (keys past Q carry -1e30 and stay below every real logit)
             s[kt][i] = kbv[i] < -1e29f ? -1e30f : __builtin_amdgcn_fmed3f(x, -FA_CLAMP, FA_CLAMP);
           }
@@ -936,7 +945,7 @@ __global__ __launch_bounds__(1024) void flash_res_kernel(FlashParams p) {
 #pragma unroll
           for (int dt = 0; dt < NDT; ++dt) o[dt] = f4{0.f, 0.f, 0.f, 0.f};
         }
-        scores(negm);
+        scores(negm, std::integral_constant<bool, BIAS>{});
         probs();
         // m moves only when a query's row sum of the chunk leaves [2^-4 (first chunk), 2^12]: an f16
         // p overflows at 2^16 and keeps 2^-15 of the sum above 2^-4, whatever m is in between

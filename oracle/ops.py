@@ -171,7 +171,8 @@ def attention_af2(activations, mask, w, heads, transpose=False, pair_bias=None, 
       o = softmax(logit) v * g;  update = o Wo + bo
     pair_bias: None | {"source": "separate", "activations": pair [Q,Q,Cz], "layerNormScale",
     "layerNormOffset", "projectionWeight" [Cz, H]} | {"source": "normalized-input",
-    "projectionWeight" [C, H]}  (`attention.js:695-783`: bias[h][i][j] = LN(z_ij) . W[:, h]).
+    "projectionWeight" [C, H]}  (`attention.js:695-783`: bias[h][i][j] = LN(z_ij) . W[:, h])
+    | {"source": "logits", "logits": [H, Q, Q]} (the bias itself).
     Weights are (in,out).  Returns the update in the storage layout.
     `batch_rows` restricts the result to those logical batch rows (returned as
     [len(batch_rows), queries, C], logical order) - batch rows are independent given the
@@ -188,7 +189,9 @@ def attention_af2(activations, mask, w, heads, transpose=False, pair_bias=None, 
     x = layer_norm(act, w["queryNormScale"], w["queryNormOffset"], eps)
     bias = None
     if pair_bias is not None:
-        if pair_bias["source"] == "separate":
+        if pair_bias["source"] == "logits":
+            bias = np.asarray(pair_bias["logits"], F32).transpose(1, 2, 0)
+        elif pair_bias["source"] == "separate":
             pn = layer_norm(pair_bias["activations"], pair_bias["layerNormScale"],
                             pair_bias["layerNormOffset"], eps)
             bias = linear(pn, pair_bias["projectionWeight"])          # [Q, Q, H]
