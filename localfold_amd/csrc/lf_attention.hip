@@ -250,6 +250,37 @@ __global__ __launch_bounds__(256) void pwa_average_kernel(PwaParams p) {
 __device__ __forceinline__ f4 qk_mfma(h8 k, h8 q, f4 c) { return mfma16(k, q, c); }
 __device__ __forceinline__ f4 qk_mfma(h4 k, h4 q, f4 c) { return mfma16k16(k, q, c); }
 
+// S^T tile kt = the pair bias + c, in the accumulator layout: row 4*g + i of the tile is key 4*kt + i
+// of the lane group g's keys, and a lane holds its query's biases of those keys in b[kt].  A product
+// of the same shape as the score product that follows (see mfma16k16), with zeros and ones as the A
+// operand: 16x16x16, where lane (r16, g4) supplies I[r16][4*g4 + j], or 16x16x32 over the lane's 8
+// biases of tiles kt & ~1 and kt | 1, of which the ones pick tile kt's.
+template <int DP>
+struct BiasPick;
+template <>
+struct BiasPick<16> {
+  h4 one;
+  __device__ __forceinline__ explicit BiasPick(int r16, int g4) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) one[j] = (_Float16)(r16 == 4 * g4 + j);
+  }
+  __device__ __forceinline__ f4 add(const h4 (&b)[4], int kt, f4 c) const { return mfma16k16(one, b[kt], c); }
+};
+template <>
+struct BiasPick<32> {
+  h8 even, odd;
+  __device__ __forceinline__ explicit BiasPick(int r16, int g4) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      even[j] = (_Float16)(r16 == 4 * g4 + j && j < 4);
+      odd[j] = (_Float16)(r16 + 4 == 4 * g4 + j && j >= 4);
+    }
+  }
+  __device__ __forceinline__ f4 add(const h4 (&b)[4], int kt, f4 c) const {
+    return mfma16(kt & 1 ? odd : even, __builtin_shufflevector(b[kt & 2], b[kt | 1], 0, 1, 2, 3, 4, 5, 6, 7), c);
+  }
+};
+
 // (float)v[i] + c in one instruction (i is a constant once the caller's loop is unrolled)
 __device__ __forceinline__ float bias_add(const h4& v, int i, float c) {
   const uint2 u = __builtin_bit_cast(uint2, v);
@@ -357,9 +388,7 @@ __global__ __launch_bounds__(64 * (8 / QT)) void flash_kernel(FlashParams p) {
     if (DP == 32 && 16 + 4 * g4 < p.d) gp1 = *reinterpret_cast<const h4*>(p.g + grow + 16 + 4 * g4);
   }
   const h8 ones = h8{1, 1, 1, 1, 1, 1, 1, 1};
-  // identity A operand of a 16x16x16 MFMA: lane supplies I[r16][4*g4 + j]
-  const h4 ident = h4{(_Float16)(r16 == 4 * g4), (_Float16)(r16 == 4 * g4 + 1), (_Float16)(r16 == 4 * g4 + 2),
-                      (_Float16)(r16 == 4 * g4 + 3)};
+  const BiasPick<DP> pick(r16, g4);
 
   // Staging: a chunk is 16 DP 16-byte pieces: piece t < 8 DP is K row t / SEGS (dims
   // 8 (t % SEGS) .. +8), piece t >= 8 DP V^T row (t - 8 DP) / 8 (keys 8 ((t - 8 DP) % 8) .. +8).
@@ -533,8 +562,7 @@ __global__ __launch_bounds__(64 * (8 / QT)) void flash_kernel(FlashParams p) {
           for (int dt = 0; dt <= NDT; ++dt) o[dt][qt] = o[dt][qt] * corr;
         }
       } else {
-        // S accumulators start at bias - m, so the MFMA yields x - m; the bias lands through an
-        // identity MFMA (D = I B + C, B = the lane's bias h4 in the accumulator layout)
+        // S accumulators start at bias - m (BiasPick), so the MFMA yields x - m
         // (a first chunk measures against m = 0 and re-bases on its own maximum below unless
         // that lies within FA_RESCALE of 0)
         f4 s[QT][4];
@@ -543,7 +571,7 @@ __global__ __launch_bounds__(64 * (8 / QT)) void flash_kernel(FlashParams p) {
           if (c == 0) m_run[qt] = 0.f;
           const f4 negm = f4{-m_run[qt], -m_run[qt], -m_run[qt], -m_run[qt]};
 #pragma unroll
-          for (int kt = 0; kt < 4; ++kt) s[qt][kt] = BIAS ? mfma16k16(ident, bq[qt][kt], negm) : negm;
+          for (int kt = 0; kt < 4; ++kt) s[qt][kt] = BIAS ? pick.add(bq[qt], kt, negm) : negm;
         }
 #pragma unroll
         for (int kt = 0; kt < 4; ++kt) {
@@ -754,9 +782,7 @@ __global__ __launch_bounds__(1024) void flash_res_kernel(FlashParams p) {
   const int qd = DP == 32 ? 8 * g4 : 4 * g4;   // the lane's head dims of a Q / K fragment, and of O
   const bool wide = p.d == DP;
   h8 ones = h8{1, 1, 1, 1, 1, 1, 1, 1};
-  // identity A operand of a 16x16x16 MFMA: lane supplies I[r16][4*g4 + j]
-  const h4 ident = h4{(_Float16)(r16 == 4 * g4), (_Float16)(r16 == 4 * g4 + 1), (_Float16)(r16 == 4 * g4 + 2),
-                      (_Float16)(r16 == 4 * g4 + 3)};
+  const BiasPick<DP> pick(r16, g4);
   {  // held in registers, not rebuilt in the loop
     u32x4 w = __builtin_bit_cast(u32x4, ones);
     asm volatile("" : "+v"(w.x), "+v"(w.y), "+v"(w.z), "+v"(w.w));
@@ -869,17 +895,11 @@ __global__ __launch_bounds__(1024) void flash_res_kernel(FlashParams p) {
         bq[3] = h4{hi[4], hi[5], hi[6], hi[7]};
       }
       h8 pf[2];
-      // s = x + cm: the bias lands through an identity MFMA (D = I B + C, B = the lane's bias h4 in
-      // the accumulator layout).  General chunks add it themselves, key by key
+      // s = x + cm, the bias through the matrix core (general chunks add it themselves, key by key)
       auto scores = [&](const f4& cm, auto bias_tag) __attribute__((always_inline)) {
         constexpr bool MBIAS = decltype(bias_tag)::value;
 #pragma unroll
-        for (int kt = 0; kt < 4; ++kt) s[kt] = MBIAS ? mfma16k16(ident, bq[kt], cm) : cm;
-        // (a product that accumulates onto one issued just before it finishes later than the wait
-        // states the compiler leaves before a VALU read of it: with the bias and score products
-        // of a tile back to back the exponentials read stale scores.  In two groups, each
-        // accumulates onto a product three issues old)
-        if (MBIAS) __builtin_amdgcn_sched_barrier(0);
+        for (int kt = 0; kt < 4; ++kt) s[kt] = MBIAS ? pick.add(bq, kt, cm) : cm;
 #pragma unroll
         for (int kt = 0; kt < 4; ++kt) s[kt] = qk_mfma(kf[kt], qf, s[kt]);
       };
@@ -893,7 +913,6 @@ __global__ __launch_bounds__(1024) void flash_res_kernel(FlashParams p) {
 #pragma unroll
           for (int kh2 = 0; kh2 < 2; ++kh2) pf[kh2] = keep_keys(pf[kh2], kh2);
         }
-        // (two independent products: see scores)
         const f4 l0 = mfma16(ones, pf[0], f4{0.f, 0.f, 0.f, 0.f}), l1 = mfma16(ones, pf[1], f4{0.f, 0.f, 0.f, 0.f});
         lc = l0[0] + l1[0];
       };
@@ -983,10 +1002,6 @@ __global__ __launch_bounds__(1024) void flash_res_kernel(FlashParams p) {
       chunk(c, bA, bB);
       if (BIAS) bA = bB;
     }
-    // the last two products of an O tile accumulate onto each other: wait for them (see scores)
-    __builtin_amdgcn_sched_barrier(0);
-    asm volatile("s_nop 15");
-    __builtin_amdgcn_sched_barrier(0);
     // o[query][h*d + dd] = O / l * g; lanes past Q or d store into the row after the last
     const float inv = __builtin_amdgcn_rcpf(l);   // (f16 results)
     if (wide) {

@@ -110,6 +110,11 @@ __device__ __forceinline__ float wave_sum(float v) {
 
 
 // 16x16x16 f16 MFMA: lane l supplies A[l%16][4(l/16)+j] and B[4(l/16)+j][l%16], j < 4.
+// Never chain it with the 16x16x32 form through an accumulator: the two finish their rows in
+// different orders, the compiler leaves no wait between them, and a product that accumulates onto
+// one of the other shape fewer than 5 wait states earlier reads half of its addend before it is
+// written (measured on gfx950: rows 2 and 3 of a lane's four after 16x16x16, 0 and 1 after
+// 16x16x32, on every pass; same-shape chains and vector reads are right at any distance).
 __device__ __forceinline__ f4 mfma16k16(h4 a, h4 b, f4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x16f16(a, b, c, 0, 0, 0);
 }

@@ -183,11 +183,7 @@ __global__ __launch_bounds__(MLP_NT, 2) void mlp_kernel(MlpParams p) {
         for (int t = 0; t < 4; ++t) fr[(f / 4 + 1) & 1][t] = *reinterpret_cast<const h8*>(cur + (f + 4 + t) * 512);
       }
       if (f == F1) {
-        // activation -> GEMM2 B fragments (k order: hidden 4g4 + i, then 16 + 4g4 + i).  The wait
-        // covers a product whose addend comes from the product just before it: it ends later
-        // than the wait states the compiler leaves before a vector instruction reads it
-        asm volatile("s_nop 15" ::: "memory");
-        __builtin_amdgcn_sched_barrier(0);
+        // activation -> GEMM2 B fragments (k order: hidden 4g4 + i, then 16 + 4g4 + i)
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
           f8 v;

@@ -676,9 +676,6 @@ __global__ __launch_bounds__(256) void rowgemm_small_kernel(RowGemmParams p) {
     acc[0] = mfma16(w0, a, acc[0]);
     acc[1] = mfma16(w1, a, acc[1]);
   }
-  // a chain of products whose last one feeds a store: longer than the compiler's wait states
-  asm volatile("s_nop 15" ::: "memory");
-  __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int t = 0; t < 2; ++t) *reinterpret_cast<f4*>(&red[wave][r16 * RS_LD + 16 * t + 4 * g4]) = acc[t];
   __syncthreads();
