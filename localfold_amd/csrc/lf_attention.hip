@@ -794,9 +794,9 @@ __global__ __launch_bounds__(1024) void flash_res_kernel(FlashParams p) {
   // 4*NDT consecutive ones: its gate and its output are one vector each
   const _Float16* vl = Vs + (4 * NDT * (r16 >> 2) + (r16 & 3)) * VLD + 8 * g4;
   // The pair bias of the lane's query: keys 8*g4 .. +7 of a chunk's two halves (fragment order,
-  // tiled_at: 1 KB per load in lane order).  Queries and keys past Q are in the buffer, unwritten: a
-  // query's garbage stays in its own column of the scores, a key's would reach the other keys of its
-  // tile through the identity product (0 * NaN) and is cleared or left out before that
+  // tiled_at: 1 KB per load in lane order).  Queries past Q are in the buffer, unwritten: what is there
+  // stays in their own columns of the scores.  Keys past Q hold zeros: anything that is not finite
+  // would reach the other keys of its tile through BiasPick's product (0 * NaN)
   struct Bias {
     h8 lo, hi;
   };
@@ -879,20 +879,12 @@ __global__ __launch_bounds__(1024) void flash_res_kernel(FlashParams p) {
       // the chunk's masked keys and those past Q, as zero halves among all-ones in the order of p
       const bool clear = (cmask >> c) & 1;   // uniform
       const uint16_t* km = Km + c * FA_KC + 8 * g4;
-      auto keep_keys = [&](h8 v, int kh2) __attribute__((always_inline)) {
-        return __builtin_bit_cast(h8, __builtin_bit_cast(u32x4, v) & *reinterpret_cast<const u32x4*>(km + 32 * kh2));
-      };
       h4 bq[4];
       if (BIAS) {
-        h8 lo = bc.lo, hi = bc.hi;
-        if (__builtin_expect(clear, 0)) {
-          lo = keep_keys(lo, 0);
-          hi = keep_keys(hi, 1);
-        }
-        bq[0] = h4{lo[0], lo[1], lo[2], lo[3]};
-        bq[1] = h4{lo[4], lo[5], lo[6], lo[7]};
-        bq[2] = h4{hi[0], hi[1], hi[2], hi[3]};
-        bq[3] = h4{hi[4], hi[5], hi[6], hi[7]};
+        bq[0] = h4{bc.lo[0], bc.lo[1], bc.lo[2], bc.lo[3]};
+        bq[1] = h4{bc.lo[4], bc.lo[5], bc.lo[6], bc.lo[7]};
+        bq[2] = h4{bc.hi[0], bc.hi[1], bc.hi[2], bc.hi[3]};
+        bq[3] = h4{bc.hi[4], bc.hi[5], bc.hi[6], bc.hi[7]};
       }
       h8 pf[2];
       // s = x + cm, the bias through the matrix core (general chunks add it themselves, key by key)
@@ -911,7 +903,9 @@ __global__ __launch_bounds__(1024) void flash_res_kernel(FlashParams p) {
           for (int i = 0; i < 4; ++i) pf[kt >> 1][4 * (kt & 1) + i] = (_Float16)__builtin_amdgcn_exp2f(s[kt][i]);
         if (__builtin_expect(clear, 0)) {
 #pragma unroll
-          for (int kh2 = 0; kh2 < 2; ++kh2) pf[kh2] = keep_keys(pf[kh2], kh2);
+          for (int kh2 = 0; kh2 < 2; ++kh2)
+            pf[kh2] = __builtin_bit_cast(h8, __builtin_bit_cast(u32x4, pf[kh2]) &
+                                                 *reinterpret_cast<const u32x4*>(km + 32 * kh2));
         }
         const f4 l0 = mfma16(ones, pf[0], f4{0.f, 0.f, 0.f, 0.f}), l1 = mfma16(ones, pf[1], f4{0.f, 0.f, 0.f, 0.f});
         lc = l0[0] + l1[0];
@@ -1199,6 +1193,9 @@ int attention(lf_context* ctx, const lf_attention_args& a, bool no_qk, bool shar
     bias_dst.sN = a.swap_bias;
     bias_dst.tile = Qp;
   }
+  // (the keys past Q of every 16 rows: flash_res_kernel needs finite values there)
+  if (res && biash && Q != Qp)
+    expand_add_zero(xl, bias16 + Q / 32 * 512, (long)H * ((Q + 15) / 16), (long)Qp * 16, (Qp / 32 - Q / 32) * 512);
   if (a.bias_mode == LF_BIAS_SEPARATE) {
     pb.g[0].dst = bias_dst;
     LF_TRY(lnproj_prepare(ctx, pb, bufs[9], &xl, "attention.pair_bias"));

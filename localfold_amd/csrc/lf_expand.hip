@@ -14,7 +14,12 @@ namespace lf {
 // multiple of 8 for such views).
 __global__ __launch_bounds__(256) void expand_weights_kernel(ExpandBatch b) {
   const int m = blockIdx.y;
-  if (m >= b.count) return;
+  if (m >= b.count) {
+    const int per = b.zlen >> 3;
+    for (long e = (long)blockIdx.x * 256 + threadIdx.x; e < b.zruns * per; e += (long)gridDim.x * 256)
+      *reinterpret_cast<h8*>(b.zero + e / per * b.zpitch + e % per * 8) = h8{0, 0, 0, 0, 0, 0, 0, 0};
+    return;
+  }
   const WView& v = b.v[m];
   const int kp = b.kp[m], W = b.W[m], off = b.off[m];
   const float sc = b.scale[m];
@@ -38,10 +43,11 @@ __global__ __launch_bounds__(256) void expand_weights_kernel(ExpandBatch b) {
 }
 
 int expand_flush(lf_context* ctx, ExpandList& l, const char* label) {
-  if (l.b.count == 0) return LF_OK;
+  if (l.b.count == 0 && l.b.zruns == 0) return LF_OK;
   {
     LaunchScope ls(ctx, label);
-    dim3 grid((unsigned)std::min<long>(std::max<long>((l.most / 8 + 255) / 256, 1), 1024), l.b.count);
+    dim3 grid((unsigned)std::min<long>(std::max<long>((l.most / 8 + 255) / 256, 1), 1024),
+              l.b.count + (l.b.zruns > 0 ? 1 : 0));
     hipLaunchKernelGGL(expand_weights_kernel, grid, dim3(256), 0, ctx->stream, l.b);
   }
   l = ExpandList{};
@@ -61,6 +67,13 @@ static int expand_add(lf_context* ctx, ExpandList& l, const WView& v, _Float16* 
   l.b.scale[i] = scale;
   l.most = std::max(l.most, (long)ncols * kp);
   return LF_OK;
+}
+
+void expand_add_zero(ExpandList& l, _Float16* dst, long runs, long pitch, int len) {
+  l.b.zero = dst;
+  l.b.zruns = runs;
+  l.b.zpitch = pitch;
+  l.b.zlen = len;
 }
 
 int expand_add_plain(lf_context* ctx, ExpandList& l, const WView& v, void* dst, WExp* out, float scale,

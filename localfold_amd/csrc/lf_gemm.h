@@ -32,6 +32,11 @@ struct ExpandBatch {
   int W[8], off[8], ncols[8];
   float scale[8];   // multiplies the decoded value before the f16 rounding
   int count;
+  // a buffer's padding to clear in the same launch: zlen halves (a multiple of 8, aligned to 16
+  // bytes) at zero + r * zpitch, r < zruns
+  _Float16* zero;
+  long zruns, zpitch;
+  int zlen;
 };
 
 // ---- in-kernel dequantisation ----------------------------------------------------------

@@ -38,6 +38,7 @@ int expand_add_plain(lf_context* ctx, ExpandList& l, const WView& v, void* dst, 
                      const char* label);
 int expand_add_packed(lf_context* ctx, ExpandList& l, const WView* views, const int* W, const int* off,
                       const long long* row0, int count, _Float16* dst, int kp, const char* label);
+void expand_add_zero(ExpandList& l, _Float16* dst, long runs, long pitch, int len);   // one per list
 int expand_flush(lf_context* ctx, ExpandList& l, const char* label);
 // dst = scale * src as f16; tq > 0 transposes each tq x tq plane; ld > 0 writes rows of rowlen
 // values at a row stride of ld
