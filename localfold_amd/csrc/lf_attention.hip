@@ -61,6 +61,11 @@ constexpr float FA_CLAMP = 1e8f * LOG2E;
 // units): until then p = exp2(x - m) <= 2^FA_RESCALE, well inside f16 range, and the
 // O rescale is skipped.
 constexpr float FA_RESCALE = 8.f;
+// A running maximum below this (log2 units) comes from masked keys alone, whose logits are far below
+// any other: scores measured against it (x - m) would lose their bits to m (ulp(1e8) = 8; ulp(256)
+// is 2^-15, below f16's rounding of p).  The next chunk then takes the general update, which
+// measures against 0 first, and the masked keys' weight becomes 0.
+constexpr float FA_FAR = -256.f;
 // flash_res_kernel's bounds on a chunk's row sums of p (see there)
 constexpr float FA_LOW = 0.0625f, FA_HIGH = 4096.f;
 
@@ -316,14 +321,15 @@ __device__ __forceinline__ void bias_fetch(const _Float16* const (&brow)[QT], in
 // lies more than FA_RESCALE below 0) p = exp2(x - m) needs no subtraction and O no rescale:
 // the standard update with a stale max m, which only scales numerator and denominator alike.
 // Otherwise m moves to the new maximum (O rescaled).  Chunks holding masked or past-the-end
-// keys take the general update (explicit key bias, clamp, max).  The row sums come from the
+// keys, and those after keys that were all masked (FA_FAR), take the general update (explicit key
+// bias, clamp, max).  The row sums come from the
 // PV MFMAs themselves, through an all-ones operand (third d tile).
 //
 // Key order within a chunk: row 4*g + i of S^T tile kt is key 16*g + 4*kt + i (K rows are
 // stored to LDS in that order), so the 16 scores a lane holds per query are the contiguous
 // keys 16*(lane/16) .. +15: its bias, key bias and V^T pieces are single vector loads.
 template <bool BIAS, int QT, bool BL = BIAS && QT == 1, int DP = FA_DP, bool FIX = false>
-__global__ __launch_bounds__(64 * (8 / QT)) void flash_kernel(FlashParams p) {
+__global__ __launch_bounds__(64 * (8 / QT), 4) void flash_kernel(FlashParams p) {
   static_assert(!BL || (BIAS && QT == 1), "the LDS-staged bias is for one query tile per wave");
   static_assert(DP == 16 || DP == 32, "padded head dim 16 or 32");
   // DP = 16 (d <= 16): QK^T on 16x16x16 MFMAs (4 head dims a lane), one O tile; DP = 32: QK^T
@@ -500,6 +506,7 @@ __global__ __launch_bounds__(64 * (8 / QT)) void flash_kernel(FlashParams p) {
     for (int dt = 0; dt <= NDT; ++dt) o[dt][qt] = f4{0.f, 0.f, 0.f, 0.f};
   }
 
+  bool far = false;   // uniform: a query's m_run came from masked keys alone (FA_FAR)
   // one chunk; RS = c % 2 is a compile-time constant so every register-set index is static
   auto chunk = [&](int c, auto rs_tag) __attribute__((always_inline)) {
       constexpr int rs = decltype(rs_tag)::value;
@@ -521,9 +528,10 @@ __global__ __launch_bounds__(64 * (8 / QT)) void flash_kernel(FlashParams p) {
       }
       if constexpr (rs == 0) kv_load(cn, st0, kb0);
       else kv_load(cn, st1, kb1);
-      const bool general = Kmasked[buf] != 0;   // wave-uniform
+      const bool general = far || Kmasked[buf] != 0;   // wave-uniform
       _Float16 pv[QT][4][4];
       if (general) {
+        far = false;
         f4 s[QT][4];
 #pragma unroll
         for (int kt = 0; kt < 4; ++kt) {
@@ -558,6 +566,7 @@ __global__ __launch_bounds__(64 * (8 / QT)) void flash_kernel(FlashParams p) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) pv[qt][kt][i] = (_Float16)__builtin_amdgcn_exp2f(s[qt][kt][i] - m_new);
           m_run[qt] = m_new;
+          far |= __any(m_new < FA_FAR);
 #pragma unroll
           for (int dt = 0; dt <= NDT; ++dt) o[dt][qt] = o[dt][qt] * corr;
         }
@@ -857,14 +866,15 @@ __global__ __launch_bounds__(1024) void flash_res_kernel(FlashParams p) {
     f4 o[NDT];
 #pragma unroll
     for (int dt = 0; dt < NDT; ++dt) o[dt] = f4{0.f, 0.f, 0.f, 0.f};
-    bool started = false;   // uniform: an unmasked key was seen (GEN)
+    bool far = false;   // uniform: a query's m came from masked keys alone (FA_FAR; GEN)
     const _Float16* brow = BIAS ? bias_at(tile) : nullptr;
     const _Float16* bnext = BIAS ? bias_at(tile + tstep < ntiles ? tile + tstep : tile) : nullptr;
 
     // chunk c with its bias in bc; the bias of the chunk after it is loaded into bn at the top (no
     // branch separates that load from the next chunk, so nothing waits for it before its use)
     auto chunk = [&](int c, Bias& bc, Bias& bn) __attribute__((always_inline)) {
-      const bool fresh = GEN ? !started : c == 0;   // no unmasked key before this chunk
+      // uniform: the explicit key bias, the clamp and the full update
+      const bool full = GEN && (((gmask >> c) & 1) || far);
       const _Float16* vc = vl + c * FA_KC;
       QF kf[4];
 #pragma unroll
@@ -928,7 +938,7 @@ __global__ __launch_bounds__(1024) void flash_res_kernel(FlashParams p) {
 #pragma unroll
         for (int dt = 0; dt < NDT; ++dt) o[dt] = o[dt] * corr;
       };
-      if (GEN && ((gmask >> c) & 1)) {   // uniform: the clamp and the full update
+      if (full) {
         scores(f4{0.f, 0.f, 0.f, 0.f}, std::false_type{});
 #pragma unroll
         for (int kt = 0; kt < 4; ++kt) {
@@ -946,23 +956,16 @@ __global__ __launch_bounds__(1024) void flash_res_kernel(FlashParams p) {
         const float m_old = c == 0 ? -1e30f : -negm[0], m_new = fmaxf(m_old, smax());
         rebase(m_new, __builtin_amdgcn_exp2f(m_old - m_new));
         negm = f4{-m_new, -m_new, -m_new, -m_new};
-        started = started || (__ballot(m_new < -0.5f * FA_CLAMP) & vmask) == 0;
+        far = (__ballot(m_new < FA_FAR) & vmask) != 0;
         probs();
       } else {
-        // The first chunk without masked keys measures against m = 0 and re-bases on its own
-        // maximum below unless its sums are fine as they are; what masked keys accumulated before
-        // it has weight 0 and is dropped (s - m would round to multiples of 16 from their -1e8)
-        if (GEN && fresh && c > 0) {
-          negm = f4{0.f, 0.f, 0.f, 0.f};
-          l = 0.f;
-#pragma unroll
-          for (int dt = 0; dt < NDT; ++dt) o[dt] = f4{0.f, 0.f, 0.f, 0.f};
-        }
+        // The first chunk measures against m = 0 and re-bases on its own maximum below unless its
+        // sums are fine as they are
         scores(negm, std::integral_constant<bool, BIAS>{});
         probs();
         // m moves only when a query's row sum of the chunk leaves [2^-4 (first chunk), 2^12]: an f16
         // p overflows at 2^16 and keeps 2^-15 of the sum above 2^-4, whatever m is in between
-        const float lo = fresh ? FA_LOW : -1.f;
+        const float lo = c == 0 ? FA_LOW : -1.f;
         if (__builtin_expect(((__ballot(!(lc <= FA_HIGH)) | __ballot(lc < lo)) & vmask) != 0, 0)) {
           if (clear) {   // masked keys do not count
 #pragma unroll
@@ -971,13 +974,12 @@ __global__ __launch_bounds__(1024) void flash_res_kernel(FlashParams p) {
               for (int i = 0; i < 4; ++i)
                 s[kt][i] = km[32 * (kt >> 1) + 4 * (kt & 1) + i] ? s[kt][i] : -1e30f;
           }
-          const float mx = smax(), d = fresh ? mx : fmaxf(mx, 0.f);
-          rebase(d, fresh ? 1.f : __builtin_amdgcn_exp2f(-d));
+          const float mx = smax(), d = c == 0 ? mx : fmaxf(mx, 0.f);
+          rebase(d, c == 0 ? 1.f : __builtin_amdgcn_exp2f(-d));
           const float nm = negm[0] - d;
           negm = f4{nm, nm, nm, nm};
           probs();
         }
-        started = true;
       }
       l += lc;
       // O^T += V^T P^T over two 32-key halves (MFMA k index 8*g4 + j is key 32*kh2 + 8*g4 + j)
@@ -988,11 +990,13 @@ __global__ __launch_bounds__(1024) void flash_res_kernel(FlashParams p) {
           o[dt] = mfma16(*reinterpret_cast<const h8*>(vc + 4 * dt * VLD + 32 * kh2), pf[kh2], o[dt]);
     };
     int c = 0;
-    for (; c + 2 <= nke; c += 2) {
-      chunk(c, bA, bB);
-      chunk(c + 1, bB, bA);
+    if constexpr (!GEN) {   // (the general loop is rarer: less code and fewer registers)
+      for (; c + 2 <= nke; c += 2) {
+        chunk(c, bA, bB);
+        chunk(c + 1, bB, bA);
+      }
     }
-    if (c < nke) {
+    for (; c < nke; ++c) {
       chunk(c, bA, bB);
       if (BIAS) bA = bB;
     }
@@ -1014,7 +1018,7 @@ __global__ __launch_bounds__(1024) void flash_res_kernel(FlashParams p) {
     }
   }
   };
-  if (gmask) walk(std::true_type{});
+  if (__builtin_expect(gmask != 0, 0)) walk(std::true_type{});
   else walk(std::false_type{});
 }
 

@@ -334,6 +334,10 @@ def test_triangle_attention_key_masks(ctx, n, heads, masks):
         mask[:, ::7] = 1.0 - 2e-9 * rng.random((n, len(range(0, n, 7)))).astype(np.float32)
         mask[:, 5::9] = np.float32(1) - np.float32(2.0 ** -24)
         mask[:, 3] = 0
+        # (beside keys of mask 1 these weigh nothing; in these rows they are all there is)
+        some = np.float32(1) - np.float32([2.0 ** -24, 2.0 ** -23, 1])
+        mask[1::2] = some[rng.integers(0, 3, mask[1::2].shape)]
+        assert ((mask > 0) & (mask < 1)).any(1).all()
     else:
         mask[::3] = 0
     dw = D.DeviceWeights(ctx.device)
@@ -357,3 +361,41 @@ def test_msa_row_attention_large_logits(ctx, blockw, s, n, gain):
     pb = dict(row["pairBias"], source="separate", activations=act["pair"])
     ref = ops.attention_af2(act["msa"], act["msaMask"], att, 8, False, pb)
     H.assert_close(out, ref, label=f"row {s}x{n} gain {gain}")
+
+
+@pytest.mark.parametrize("n,heads", [(193, 4), (257, 8), (1160, 4), (2000, 8), (1160, 128)])
+@pytest.mark.parametrize("masks", ["leading", "nearly", "fractional"])
+def test_first_keys_of_little_weight(ctx, n, heads, masks):
+    """A first chunk (or two) of 64 keys that are masked, or nearly (0.99, 0.97, 0.9999), before
+    unmasked ones: their logits of -1e5 to -1e8 must not cost the others' scores their low bits.
+    And keys that are all fractional, so that their explicit biases decide the softmax.  K and V
+    in LDS (193, 257) and not (1160, 2000); heads of 32, 16 and 1 (no multiple of 4)."""
+    from localfold_amd import capi, device as D
+    rng = np.random.default_rng(n)
+    w = S.config3_attention_weights(128, heads, n)
+    att = dict(w["attention"], queryWeight=w["attention"]["queryWeight"] * np.float32(2))
+    act = rng.standard_normal((3, n, 128)).astype(np.float32)
+    mask = np.ones((3, n), np.float32)
+    if masks == "leading":
+        mask[:, :70] = 0
+        mask[1, :128] = 0
+    elif masks == "nearly":
+        mask[0, :64] = 0.99
+        mask[1, :128] = 0.97
+        mask[2, :64] = np.float32(0.9999)
+    else:   # key biases of -60, -119 and -1e9 on every key of a row, and on a first chunk
+        some = np.float32(1) - np.float32([2.0 ** -24, 2.0 ** -23, 1])
+        mask[0] = some[rng.integers(0, 3, n)]
+        mask[1] = some[rng.integers(0, 2, n)]
+        mask[2, :64] = some[rng.integers(0, 2, 64)]
+    dw = D.DeviceWeights(ctx.device)
+    pair = rng.standard_normal((n, n, 128)).astype(np.float32) if n < 1000 else None
+    pb = dict(w["pairBias"], layerNormScale=att["queryNormScale"], layerNormOffset=att["queryNormOffset"],
+              source="separate", activations=pair)
+    ws = D.attention_weights_af2(dw, att, pb if pair is not None else None)
+    out, _, _ = _run(ctx, act, mask, ws, heads, False, capi.LF_BIAS_NONE if pair is None else capi.LF_BIAS_SEPARATE, pair)
+    ref = ops.attention_af2(act, mask, att, heads, False, None if pair is None else pb)
+    if masks == "fractional":   # the fractions matter: as 0 they would give another result
+        plain = ops.attention_af2(act, np.where(mask == 1, mask, 0), att, heads, False, None if pair is None else pb)
+        assert ((mask > 0) & (mask < 1)).any() and H.metrics(plain, ref)["relativeFrobenius"] > 0.05
+    H.assert_close(out, ref, label=f"{masks} {n}/{heads}")
