@@ -45,6 +45,7 @@ struct FlashParams {
   int fix;                // dq < DP or Q not a whole number of chunks: the kernel (the FIX
                           // instantiation) zeroes the unwritten parts of q, k and v^T as it
                           // reads them
+  int logits;             // flash_kernel: the bias holds a caller's logits, which may be infinite in f16
   int nqb;                // query blocks per (b, h); flash_res_kernel: query splits
   int nw;                 // flash_res_kernel: waves per block
   const float* mask;      // flash_res_kernel: key k of batch row b is mask[b * mask_b + k * mask_k]
@@ -285,6 +286,31 @@ struct BiasPick<32> {
     return mfma16(kt & 1 ? odd : even, __builtin_shufflevector(b[kt & 2], b[kt | 1], 0, 1, 2, 3, 4, 5, 6, 7), c);
   }
 };
+
+// One of a lane's biases is NaN, of those keys that km keeps (flash_res_kernel's all-ones halves).
+// (What is above infinity carries into its sign bit, and no half into the next.)
+__device__ __forceinline__ bool bias_nan(const h4 (&b)[4], const uint16_t* km) {
+  uint32_t top = 0;
+#pragma unroll
+  for (int kt = 0; kt < 4; ++kt) {
+    const uint2 w = __builtin_bit_cast(uint2, b[kt]);
+    const uint2 m = *reinterpret_cast<const uint2*>(km + 32 * (kt >> 1) + 4 * (kt & 1));
+    top |= ((w.x & m.x & 0x7fff7fffu) + 0x03ff03ffu) | ((w.y & m.y & 0x7fff7fffu) + 0x03ff03ffu);
+  }
+  return (top & 0x80008000u) != 0;
+}
+
+// One of a lane's biases is infinite (or NaN): a caller's logit beyond f16, 45 400.  (A half with all
+// exponent bits set carries into its sign bit, and no half into the next.)
+__device__ __forceinline__ bool bias_infinite(const h4 (&b)[4]) {
+  uint32_t top = 0;
+#pragma unroll
+  for (int kt = 0; kt < 4; ++kt) {
+    const uint2 w = __builtin_bit_cast(uint2, b[kt]);
+    top |= ((w.x & 0x7c007c00u) + 0x04000400u) | ((w.y & 0x7c007c00u) + 0x04000400u);
+  }
+  return (top & 0x80008000u) != 0;
+}
 
 // (float)v[i] + c in one instruction (i is a constant once the caller's loop is unrolled)
 __device__ __forceinline__ float bias_add(const h4& v, int i, float c) {
@@ -528,7 +554,11 @@ __global__ __launch_bounds__(64 * (8 / QT), 4) void flash_kernel(FlashParams p) 
       }
       if constexpr (rs == 0) kv_load(cn, st0, kb0);
       else kv_load(cn, st1, kb1);
-      const bool general = far || Kmasked[buf] != 0;   // wave-uniform
+      bool general = far || Kmasked[buf] != 0;   // wave-uniform
+      if (BIAS && p.logits) {
+#pragma unroll
+        for (int qt = 0; qt < QT; ++qt) general |= __any(bias_infinite(bq[qt]));
+      }
       _Float16 pv[QT][4][4];
       if (general) {
         far = false;
@@ -833,11 +863,16 @@ __global__ __launch_bounds__(1024) void flash_res_kernel(FlashParams p) {
   const int kind = lane < nkc ? Kind[lane < nkc ? lane : 0] : 0;
   const bool some = __any(kind & 1);
   const unsigned long long gmask = __ballot((kind & 4) || kind == 2 || (!some && kind)), cmask = __ballot(kind == 3);
-  const int nke = some ? 64 - __builtin_clzll(__ballot(kind & 5)) : nkc;
+  int nke = some ? 64 - __builtin_clzll(__ballot(kind & 5)) : nkc;
   // GEN: with the explicit update of gmask's chunks; most blocks have none, and the loop without
-  // that path keeps its state in place
-  auto walk = [&](auto gen_tag) __attribute__((always_inline)) {
-  constexpr bool GEN = decltype(gen_tag)::value;
+  // that path keeps its state in place.
+  // A bias beyond f16 (a caller's logit of -1e9, say) is infinite and makes its tile's scores NaN
+  // (BiasPick), which shows in the row sums: such a wave starts over with every chunk explicit,
+  // where an infinite logit is clamped like any other, and with all keys, which a query whose
+  // unmasked keys are all at the clamp sees alike
+  bool redo = false;   // uniform
+  auto walk = [&](auto gen_tag, auto every_tag) __attribute__((always_inline)) {
+  constexpr bool GEN = decltype(gen_tag)::value, EVERY = decltype(every_tag)::value;
   for (; tile < ntiles; tile += tstep) {
     const int qi = tile * 16 + r16, qc = min(qi, p.Q - 1);
     const unsigned long long vmask = __ballot(qi < p.Q);   // the others take no part in the votes
@@ -873,8 +908,6 @@ __global__ __launch_bounds__(1024) void flash_res_kernel(FlashParams p) {
     // chunk c with its bias in bc; the bias of the chunk after it is loaded into bn at the top (no
     // branch separates that load from the next chunk, so nothing waits for it before its use)
     auto chunk = [&](int c, Bias& bc, Bias& bn) __attribute__((always_inline)) {
-      // uniform: the explicit key bias, the clamp and the full update
-      const bool full = GEN && (((gmask >> c) & 1) || far);
       const _Float16* vc = vl + c * FA_KC;
       QF kf[4];
 #pragma unroll
@@ -887,7 +920,6 @@ __global__ __launch_bounds__(1024) void flash_res_kernel(FlashParams p) {
       f4 s[4];
       float lc;
       // the chunk's masked keys and those past Q, as zero halves among all-ones in the order of p
-      const bool clear = (cmask >> c) & 1;   // uniform
       const uint16_t* km = Km + c * FA_KC + 8 * g4;
       h4 bq[4];
       if (BIAS) {
@@ -896,6 +928,10 @@ __global__ __launch_bounds__(1024) void flash_res_kernel(FlashParams p) {
         bq[2] = h4{bc.hi[0], bc.hi[1], bc.hi[2], bc.hi[3]};
         bq[3] = h4{bc.hi[4], bc.hi[5], bc.hi[6], bc.hi[7]};
       }
+      // uniform: the explicit key bias, the clamp and the full update, in which masked keys keep the
+      // weights that leaves them
+      const bool full = EVERY || (GEN && (((gmask >> c) & 1) || far));
+      const bool clear = !full && ((cmask >> c) & 1);   // uniform
       h8 pf[2];
       // s = x + cm, the bias through the matrix core (general chunks add it themselves, key by key)
       auto scores = [&](const f4& cm, auto bias_tag) __attribute__((always_inline)) {
@@ -953,6 +989,7 @@ __global__ __launch_bounds__(1024) void flash_res_kernel(FlashParams p) {
             s[kt][i] = kbv[i] < -1e29f ? -1e30f : __builtin_amdgcn_fmed3f(x, -FA_CLAMP, FA_CLAMP);
           }
         }
+        if (BIAS && EVERY && bias_nan(bq, km)) s[0][0] = __builtin_nanf("");   // (the clamp would hide it)
         const float m_old = c == 0 ? -1e30f : -negm[0], m_new = fmaxf(m_old, smax());
         rebase(m_new, __builtin_amdgcn_exp2f(m_old - m_new));
         negm = f4{-m_new, -m_new, -m_new, -m_new};
@@ -967,6 +1004,7 @@ __global__ __launch_bounds__(1024) void flash_res_kernel(FlashParams p) {
         // p overflows at 2^16 and keeps 2^-15 of the sum above 2^-4, whatever m is in between
         const float lo = c == 0 ? FA_LOW : -1.f;
         if (__builtin_expect(((__ballot(!(lc <= FA_HIGH)) | __ballot(lc < lo)) & vmask) != 0, 0)) {
+          if (BIAS) redo |= (__ballot(lc != lc) & vmask) != 0;
           if (clear) {   // masked keys do not count
 #pragma unroll
             for (int kt = 0; kt < 4; ++kt)
@@ -1018,8 +1056,15 @@ __global__ __launch_bounds__(1024) void flash_res_kernel(FlashParams p) {
     }
   }
   };
-  if (__builtin_expect(gmask != 0, 0)) walk(std::true_type{});
-  else walk(std::false_type{});
+  if (__builtin_expect(gmask != 0, 0)) walk(std::true_type{}, std::false_type{});
+  else walk(std::false_type{}, std::false_type{});
+  if (BIAS && __builtin_expect(redo, 0)) {
+    nke = nkc;
+    tile = wave * p.nqb + split;
+    qnext = q_load(tile);
+    bias_load(bA, bias_at(tile));
+    walk(std::true_type{}, std::true_type{});
+  }
 }
 
 // Waves per block and query splits of flash_res_kernel, false when K and V do not fit the LDS.
@@ -1292,6 +1337,7 @@ int attention(lf_context* ctx, const lf_attention_args& a, bool no_qk, bool shar
     fp.HD = HD;
     fp.dq = no_qk ? 0 : d;
     fp.fix = fp.dq < DP || Q != Qp;
+    fp.logits = a.bias_mode == LF_BIAS_LOGITS;
     fp.nqb = (Q + FA_QPB - 1) / FA_QPB;
     fp.nblocks = (long long)fp.nqb * B * H;
     LaunchScope ls(ctx, "attention.flash");

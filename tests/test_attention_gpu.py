@@ -399,3 +399,69 @@ def test_first_keys_of_little_weight(ctx, n, heads, masks):
         plain = ops.attention_af2(act, np.where(mask == 1, mask, 0), att, heads, False, None if pair is None else pb)
         assert ((mask > 0) & (mask < 1)).any() and H.metrics(plain, ref)["relativeFrobenius"] > 0.05
     H.assert_close(out, ref, label=f"{masks} {n}/{heads}")
+
+
+@pytest.mark.parametrize("n,heads", [(40, 4), (64, 8), (130, 4), (130, 8), (1300, 4)])
+@pytest.mark.parametrize("swap", [False, True])
+def test_caller_logits(ctx, n, heads, swap):
+    """Bias logits from the caller, some at -1e9 (far beyond f16) to mask a key for one query, a
+    query all of whose logits are, beside keys masked for every query; whole and ragged chunks,
+    keys that fit the LDS and (1300) that don't."""
+    from localfold_amd import capi, device as D
+    rng = np.random.default_rng(n + heads)
+    w = S.config3_attention_weights(128, heads, n)["attention"]
+    act = rng.standard_normal((2, n, 128)).astype(np.float32)
+    mask = np.ones((2, n), np.float32)
+    mask[1, ::3] = 0
+    logits = rng.standard_normal((heads, n, n)).astype(np.float32)
+    logits[rng.random(logits.shape) < 0.2] = -1e9
+    logits[0, n // 2] = -1e9
+    logits[0, :, n // 3] = -1e9
+    dw = D.DeviceWeights(ctx.device)
+    ws = D.attention_weights_af2(dw, w)
+    out, _, _ = _run(ctx, act, mask, ws, heads, False, capi.LF_BIAS_LOGITS, swap_bias=swap,
+                     bias_logits=_dev(ctx, logits))
+    ref = ops.attention_af2(act, mask, w, heads, False,
+                            {"source": "logits", "logits": logits.transpose(0, 2, 1) if swap else logits})
+    H.assert_close(out, ref, label=f"logits {n}/{heads} swap={swap}")
+
+
+@pytest.mark.parametrize("n", [40, 64, 130])
+@pytest.mark.parametrize("source", ["separate", "input"])
+def test_pair_bias_beyond_f16(ctx, n, source):
+    """Projected pair biases far beyond f16: one key of every query at about +1e6, the others at
+    -1e6.  The softmax picks that key."""
+    from localfold_amd import capi, device as D
+    rng = np.random.default_rng(n)
+    w = S.config3_attention_weights(128, 4, n)
+    att = dict(w["attention"], queryNormScale=np.ones(128, np.float32), queryNormOffset=np.zeros(128, np.float32))
+    proj = np.zeros((128, 4), np.float32)
+    proj[0] = 1e5
+    pair = rng.standard_normal((n, n, 128)).astype(np.float32)
+    pair[:, :, 0] = -300
+    pair[np.arange(n), (7 * np.arange(n)) % n, 0] = 300
+    pb = {"layerNormScale": att["queryNormScale"], "layerNormOffset": att["queryNormOffset"], "projectionWeight": proj}
+    separate = source == "separate"
+    act = rng.standard_normal((3, n, 128)).astype(np.float32) if separate else pair
+    mask = np.ones(act.shape[:2], np.float32)
+    dw = D.DeviceWeights(ctx.device)
+    ws = D.attention_weights_af2(dw, att, pb)
+    out, _, _ = _run(ctx, act, mask, ws, 4, False,
+                     capi.LF_BIAS_SEPARATE if separate else capi.LF_BIAS_NORMALIZED_INPUT, pair if separate else None)
+    ref = ops.attention_af2(act, mask, att, 4, False, dict(pb, source="separate", activations=pair))
+    H.assert_close(out, ref, label=f"large bias {n} {source}")
+
+
+@pytest.mark.parametrize("n", [40, 130])
+def test_nan_pair_stays_nan(ctx, blockw, n):
+    """A NaN in the pair tensor reaches the queries it biases, and only those."""
+    from localfold_amd import capi, device as D
+    act = S.synthetic_activations(3, n, 256, 128, seed=n)
+    row = blockw["msaRowAttention"]
+    pair = act["pair"].copy()
+    pair[7, n - 1, 5] = np.nan
+    pair[9, 2, 5] = np.inf      # LayerNorm of it is NaN as well
+    dw = D.DeviceWeights(ctx.device)
+    ws = D.attention_weights_af2(dw, row["attention"], row["pairBias"])
+    out, _, _ = _run(ctx, act["msa"], np.ones((3, n), np.float32), ws, 8, False, capi.LF_BIAS_SEPARATE, pair)
+    assert np.isnan(out[:, [7, 9]]).all() and np.isfinite(np.delete(out, [7, 9], 1)).all()
