@@ -68,7 +68,7 @@ constexpr float FA_RESCALE = 8.f;
 // measures against 0 first, and the masked keys' weight becomes 0.
 constexpr float FA_FAR = -256.f;
 // flash_res_kernel's bounds on a chunk's row sums of p (see there)
-constexpr float FA_LOW = 0.0625f, FA_HIGH = 4096.f;
+constexpr float FA_LOW = 0.25f, FA_HIGH = 4096.f;
 
 // kb[b][k] for k < Qp (keys padded to whole chunks): 1e9 log2(e) (mask - 1), and -1e30 past Q
 __global__ __launch_bounds__(256) void keybias_kernel(const float* mask, float* kb, int B, int Q, int Qp,
@@ -1000,8 +1000,9 @@ __global__ __launch_bounds__(1024) void flash_res_kernel(FlashParams p) {
         // sums are fine as they are
         scores(negm, std::integral_constant<bool, BIAS>{});
         probs();
-        // m moves only when a query's row sum of the chunk leaves [2^-4 (first chunk), 2^12]: an f16
-        // p overflows at 2^16 and keeps 2^-15 of the sum above 2^-4, whatever m is in between
+        // m moves only when a query's row sum of the chunk leaves [2^-2 (first chunk), 2^12]: an f16 p
+        // overflows at 2^16, and of 64 summing to 2^-2 the largest is at least 2^-8 (flash_kernel's
+        // bound), 2^-16 of which is f16's smallest step
         const float lo = c == 0 ? FA_LOW : -1.f;
         if (__builtin_expect(((__ballot(!(lc <= FA_HIGH)) | __ballot(lc < lo)) & vmask) != 0, 0)) {
           if (BIAS) redo |= (__ballot(lc != lc) & vmask) != 0;
@@ -1039,7 +1040,7 @@ __global__ __launch_bounds__(1024) void flash_res_kernel(FlashParams p) {
       if (BIAS) bA = bB;
     }
     // o[query][h*d + dd] = O / l * g; lanes past Q or d store into the row after the last
-    const float inv = __builtin_amdgcn_rcpf(l);   // (f16 results)
+    const float inv = 1.f / l;
     if (wide) {
       QF ov;
 #pragma unroll
