@@ -1024,13 +1024,10 @@ template <int ACT, int NWV, bool ST, bool WHOLE, typename OFS>
 __global__ __launch_bounds__(64 * NWV) void tri_project_v3_kernel(TriProjectParams p) {
   constexpr int NT = 64 * NWV;
   __shared__ __attribute__((aligned(16))) _Float16 Ws[4 * 128 * RS_LD];  // a-proj, a-gate', b-proj, b-gate' [h][k]
-  __shared__ __attribute__((aligned(16))) h8 Bt[4 * 128];                 // the four bias vectors (gates scaled), f16 hi + lo
+  __shared__ __attribute__((aligned(16))) float Bs[4 * 128];              // the four bias vectors (gates scaled)
   __shared__ __attribute__((aligned(16))) float Gs[2 * 128];              // LN_in scale, offset
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int r16 = lane & 15, g4 = lane >> 4, q4 = g4 * 4, kq = g4 * 8;
-  // A operand of the bias MFMA: ones at k = 0, 1 (lanes 0-15 supply k 0..7), zeros elsewhere
-  const _Float16 one = (_Float16)(g4 == 0 ? 1.f : 0.f);
-  const h8 ones = h8{one, one, 0, 0, 0, 0, 0, 0};
   const int ntiles = p.N * (p.ld >> 4), nw = gridDim.x * NWV;
   auto fetch = [&](const TileGeom& g, FragTile<ACT, 4>& t, float (&m)[4]) __attribute__((always_inline)) {
     frag_load_row(t, p.z, (size_t)g.src0 + (size_t)(WHOLE ? r16 : min(r16, g.nvalid - 1)) * g.sstride, 128, lane);
@@ -1044,18 +1041,11 @@ __global__ __launch_bounds__(64 * NWV) void tri_project_v3_kernel(TriProjectPara
   TileGeom tg = tile_geom<WHOLE>(p.N, p.ld, p.kmajor_out, tile < ntiles ? tile : 0);
   fetch(tg, tc, mc);
   stage_project_weights<NT>(Ws, p, tid);
-  // a bias b as the B operand of an MFMA (of the shape of the products it starts: see mfma16k16):
-  // k rows 0 and 1 hold hi = f16(b) and lo = f16(b - hi), which the ones in the A operand sum back
-  // to b within 2^-22 relative
-  auto split = [](float b) {
-    const _Float16 hi = (_Float16)b;
-    return h8{hi, (_Float16)(b - (float)hi), 0, 0, 0, 0, 0, 0};
-  };
   for (int i = tid; i < 128; i += NT) {
-    Bt[i] = split(p.bp[0] ? p.bp[0][i] : 0.f);
-    Bt[128 + i] = split(p.bg[0] ? TRI_NLOG2E * p.bg[0][i] : 0.f);
-    Bt[256 + i] = split(p.bp[1] ? p.bp[1][i] : 0.f);
-    Bt[384 + i] = split(p.bg[1] ? TRI_NLOG2E * p.bg[1][i] : 0.f);
+    Bs[i] = p.bp[0] ? p.bp[0][i] : 0.f;
+    Bs[128 + i] = p.bg[0] ? TRI_NLOG2E * p.bg[0][i] : 0.f;
+    Bs[256 + i] = p.bp[1] ? p.bp[1][i] : 0.f;
+    Bs[384 + i] = p.bg[1] ? TRI_NLOG2E * p.bg[1][i] : 0.f;
   }
   stage_vec(Gs, p.ln_s, 128, 1.f, 128, tid, NT);
   stage_vec(Gs + 128, p.ln_o, 128, 0.f, 128, tid, NT);
@@ -1084,13 +1074,14 @@ __global__ __launch_bounds__(64 * NWV) void tri_project_v3_kernel(TriProjectPara
       constexpr int PS = decltype(pass_tag)::value, which = PS >> 1, hh = (PS & 1) * 64;
       const _Float16* Wp = Ws + (which * 2) * 128 * RS_LD;
       const _Float16* Wg = Wp + 128 * RS_LD;
-      // the accumulators start at the biases, through the matrix core (no per-register moves)
-      const h8* btp = Bt + which * 256 + hh + r16;
+      // the accumulators start at the biases, in f32 whatever their size
+      const float* bp = Bs + which * 256 + hh + r16;
       f4 acc[8];
 #pragma unroll
       for (int t4 = 0; t4 < 4; ++t4) {
-        acc[t4] = mfma16(ones, btp[t4 * 16], f4{0.f, 0.f, 0.f, 0.f});
-        acc[4 + t4] = mfma16(ones, btp[128 + t4 * 16], f4{0.f, 0.f, 0.f, 0.f});
+        const float b0 = bp[t4 * 16], b1 = bp[128 + t4 * 16];
+        acc[t4] = f4{b0, b0, b0, b0};
+        acc[4 + t4] = f4{b1, b1, b1, b1};
       }
 #pragma unroll
       for (int j = 0; j < 4; ++j) {

@@ -113,6 +113,22 @@ def test_padded_plane_rows(ctx, n, direction, act):
     H.assert_close(z.float().cpu().numpy(), ref, max_abs=2e-2, label=f"padded {n}/{direction}/{act}")
 
 
+@pytest.mark.parametrize("n", [59, 64])
+@pytest.mark.parametrize("direction", ["outgoing", "incoming"])
+def test_biases_beyond_f16(ctx, n, direction):
+    """Linear biases of 1e5 behind gates of about 2^-11, and gate biases of +-6e4: the operands are
+    well within f16, the biases are not.  Lengths with partial and with whole 16-pair tiles."""
+    inp = S.deterministic_triangle_input(n, 128, 128, 60 + n)
+    w = {k: np.array(v, np.float32) for k, v in inp["weights"].items()}
+    w["linearAPBias"][::7], w["linearAGBias"][::7] = 1e5, -8
+    w["linearBPBias"][2::7], w["linearBGBias"][2::7] = -1e5, -8
+    w["linearAGBias"][3::7], w["linearBGBias"][5::7] = 6e4, -6e4
+    out, _ = _run(ctx, inp["z"], inp["mask"], w, direction)
+    ref = ops.tri_mult_af2(inp["z"], inp["mask"], w, direction)
+    assert np.isfinite(ref).all()
+    H.assert_close(out, ref, label=f"{n}/{direction}")
+
+
 def test_af3_dialect_large_contraction_tiles(ctx):
     """AF3 at N = 768 (incoming, divided by the length, bf16 pair): the split projection of
     the interleaved tensors feeding the 256 x 256-tile contraction; against the oracle."""
