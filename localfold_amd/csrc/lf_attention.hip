@@ -69,6 +69,7 @@ constexpr float FA_RESCALE = 8.f;
 constexpr float FA_FAR = -256.f;
 // flash_res_kernel's bounds on a chunk's row sums of p (see there)
 constexpr float FA_LOW = 0.25f, FA_HIGH = 4096.f;
+constexpr int FA_RES_SMEM = 160 * 1024;   // the LDS its K, V^T and key tables may take
 
 // kb[b][k] for k < Qp (keys padded to whole chunks): 1e9 log2(e) (mask - 1), and -1e30 past Q
 __global__ __launch_bounds__(256) void keybias_kernel(const float* mask, float* kb, int B, int Q, int Qp,
@@ -1068,14 +1069,27 @@ __global__ __launch_bounds__(1024) void flash_res_kernel(FlashParams p) {
   }
 }
 
+// flash_res_kernel's dynamic LDS (above the 64 KB default) is opted into once per process; where it
+// is refused, flash_kernel serves every call.
+static bool flash_res_smem_ok() {
+  auto opt = [](const void* k) {
+    return hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, FA_RES_SMEM) == hipSuccess;
+  };
+  static const bool ok = opt(reinterpret_cast<const void*>(flash_res_kernel<true, 16>)) &&
+                         opt(reinterpret_cast<const void*>(flash_res_kernel<true, 32>)) &&
+                         opt(reinterpret_cast<const void*>(flash_res_kernel<false, 16>)) &&
+                         opt(reinterpret_cast<const void*>(flash_res_kernel<false, 32>));
+  return ok;
+}
+
 // Waves per block and query splits of flash_res_kernel, false when K and V do not fit the LDS.
 // Few (batch row, head) pairs have their queries split over the CUs.  A CU holds 16 waves (128
 // registers each) and as many blocks as their LDS allows; the wave count is the one that keeps
 // the most of them busy through whole rounds of query tiles, but enough to stage with.
 template <int DP>
 static bool flash_res_shape(const lf_context* ctx, int Q, int Qp, long long bh, int* nw, int* nsplit) {
-  const size_t lds = FlashRes<DP>::lds(Qp), cap = 160 * 1024;
-  if (lds > cap) return false;
+  const size_t lds = FlashRes<DP>::lds(Qp), cap = FA_RES_SMEM;
+  if (lds > cap || !flash_res_smem_ok()) return false;
   const int tiles = (Q + 15) / 16, cus = ctx->num_cus;
   const int split = (int)std::min<long long>(std::max<long long>(1, cus / bh), tiles);
   const int t = (tiles + split - 1) / split;
@@ -1092,14 +1106,10 @@ static bool flash_res_shape(const lf_context* ctx, int Q, int Qp, long long bh, 
 }
 
 template <bool BIAS, int DP>
-static int launch_flash_res(lf_context* ctx, FlashParams fp, int Qp) {
-  static const bool ok = hipFuncSetAttribute(reinterpret_cast<const void*>(flash_res_kernel<BIAS, DP>),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) == hipSuccess;
-  if (!ok) return set_error(LF_ERR_DEVICE, "flash: the device refuses 160 KB of LDS");
+static void launch_flash_res(lf_context* ctx, FlashParams fp, int Qp) {
   fp.nblocks = (long long)fp.nqb * fp.B * fp.H;
   hipLaunchKernelGGL((flash_res_kernel<BIAS, DP>), dim3((unsigned)fp.nblocks), dim3(64 * fp.nw),
                      FlashRes<DP>::lds(Qp), ctx->stream, fp);
-  return LF_OK;
 }
 
 int attention(lf_context* ctx, const lf_attention_args& a, bool no_qk, bool shared_key_mask) {
@@ -1353,10 +1363,10 @@ int attention(lf_context* ctx, const lf_attention_args& a, bool no_qk, bool shar
       fp.mask_b = a.transpose ? 1 : Q;
       fp.mask_k = a.transpose ? B : 1;
       fp.nqb = nsplit;
-      if (fp.bias && DP == 16) LF_TRY((launch_flash_res<true, 16>(ctx, fp, Qp)));
-      else if (fp.bias) LF_TRY((launch_flash_res<true, 32>(ctx, fp, Qp)));
-      else if (DP == 16) LF_TRY((launch_flash_res<false, 16>(ctx, fp, Qp)));
-      else LF_TRY((launch_flash_res<false, 32>(ctx, fp, Qp)));
+      if (fp.bias && DP == 16) launch_flash_res<true, 16>(ctx, fp, Qp);
+      else if (fp.bias) launch_flash_res<true, 32>(ctx, fp, Qp);
+      else if (DP == 16) launch_flash_res<false, 16>(ctx, fp, Qp);
+      else launch_flash_res<false, 32>(ctx, fp, Qp);
     } else if (fp.bias && DP == 16)
       hipLaunchKernelGGL((flash_kernel<true, FA_QT_BIAS, BLD, 16, true>), grid, bb, 0, ctx->stream, fp);
     else if (fp.bias && fp.fix)
