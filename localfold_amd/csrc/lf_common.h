@@ -588,39 +588,12 @@ __device__ __forceinline__ void frag_stats_raw(FragTile<ACT, KS>& t, int C, floa
   launder(t);
 }
 
-// LayerNorm of two raw tiles into MFMA fragments, gamma/beta read once per k-step for both.
-// Padding channels normalise to finite values that meet zero weight rows; rows past the end
-// are normalised too (their outputs are never stored).
-template <int ACT, int KS>
-__device__ __forceinline__ void frag_ln_raw2(FragTile<ACT, KS>& t0, FragTile<ACT, KS>& t1, h8 (&a0)[KS],
-                                             h8 (&a1)[KS], int C, const float* gamma, const float* beta,
-                                             float eps, bool fast_var, int lane) {
-  const int g = lane >> 4;
-  float m0, i0, m1, i1;
-  frag_stats_raw(t0, C, eps, fast_var, m0, i0);
-  frag_stats_raw(t1, C, eps, fast_var, m1, i1);
-#pragma unroll
-  for (int j = 0; j < KS; ++j) {
-    const float4 g0 = *reinterpret_cast<const float4*>(gamma + 32 * j + 8 * g);
-    const float4 g1 = *reinterpret_cast<const float4*>(gamma + 32 * j + 8 * g + 4);
-    const float4 b0 = *reinterpret_cast<const float4*>(beta + 32 * j + 8 * g);
-    const float4 b1 = *reinterpret_cast<const float4*>(beta + 32 * j + 8 * g + 4);
-    const float gg[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
-    const float bb[8] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      a0[j][e] = (_Float16)((t0.get(j, e) - m0) * i0 * gg[e] + bb[e]);
-      a1[j][e] = (_Float16)((t1.get(j, e) - m1) * i1 * gg[e] + bb[e]);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-  }
-}
-
 template <int ACT, int KS>
 __device__ __forceinline__ void frag_ln_given(FragTile<ACT, KS>& t0, h8 (&a0)[KS], const float* gamma,
                                               const float* beta, float m0, float i0, int lane);
 
-// LayerNorm of one raw tile into MFMA fragments (frag_ln_raw2 for a single tile).
+// LayerNorm of one raw tile into MFMA fragments.  Padding channels normalise to finite values that
+// meet zero weight rows; rows past the end are normalised too (their outputs are never stored).
 template <int ACT, int KS>
 __device__ __forceinline__ void frag_ln_raw1(FragTile<ACT, KS>& t0, h8 (&a0)[KS], int C, const float* gamma,
                                              const float* beta, float eps, bool fast_var, int lane) {

@@ -6,10 +6,11 @@
 //   lnproj    LN(msa) -> l, r stored [i][a][s] (sequence-contiguous: the contraction's K axis)
 //   count     den[i*N + j] = norm_eps + sum_s m_si m_sj
 //   outer     O[(i,j)][a*c + b] = sum_s l[i][a][s] r[j][b][s]: one NT GEMM of (N*c) x (N*c) x S on
-//             MFMA, 256x256 tiles (128x128 when N*c is not a multiple of 256), written
+//             MFMA, 256x256 tiles (128x128 when N*c is not a multiple of 256 or S, rounded
+//             up to 8, not one of 64), written
 //             pair-major f16 (the next GEMM's rows)
 //   rowgemm   O W_out + b, / den, + pair residual
-//   fused     (c_outer 32, c_z 128, whole 256 tiles) the outer tile kept in LDS and the output
+//   fused     (c_outer 32, c_z 128, any N and S) the outer tile kept in LDS and the output
 //             GEMM, /den and residual run in the same kernel: O never reaches memory
 #include <algorithm>
 #include <cmath>

@@ -65,8 +65,8 @@ struct LnProjParams {
   const void* x;
   int rows, C;        // logical rows, channels (LN width == K)
   int rmQ, rmB;       // row map: logical row r = b*rmQ + q reads storage row q*rmB + b (rmB > 0) or r
-  int rmN;            // when > 0: a batch holds rmN <= rmQ rows and is padded to rmQ; storage row
-                      // q*rmB + b or b*rmN + q.  A padding row repeats the last one (times zero with
+  int rmN;            // when > 0 (with rmB > 0): a batch holds rmN <= rmQ rows and is padded to rmQ;
+                      // storage row q*rmB + b.  A padding row repeats the last one (times zero with
                       // OP_ROWMASK): it is stored, so every destination has room for rmQ rows.
                       // With rmQ a multiple of 4 the four rows or columns of a lane
                       // never straddle a batch and every store is a vector, whatever rmN is

@@ -253,7 +253,7 @@ __global__ __launch_bounds__(512, KS <= 4 ? 4 : 2) void lnproj_kernel(LnProjPara
   auto srow_of = [&](int r) {
     if (p.rmN > 0) {
       const int bb = r / p.rmQ, q = min(r - bb * p.rmQ, p.rmN - 1);
-      return p.rmB > 0 ? q * p.rmB + bb : bb * p.rmN + q;
+      return q * p.rmB + bb;
     }
     return p.rmB > 0 ? (r % p.rmQ) * p.rmB + r / p.rmQ : r;
   };

@@ -247,54 +247,43 @@ __device__ __forceinline__ void ct_load(_Float16* S, const _Float16* src, int N,
   }
 }
 
-// Vector form (N % 8 == 0) split in two: global -> registers (issued before the current K
-// step's MFMAs so the loads are in flight during them) and registers -> LDS.  PER = TM / 32
-// 16-byte pieces per thread and operand.
+// Vector form for k-major operands (N % 8 == 0) split in two: global -> registers (issued before
+// the current K step's MFMAs so the loads are in flight during them) and registers -> LDS.
+// PER = TM / 32 16-byte pieces per thread and operand.
 // The piece it of a thread: its (m, k) origin in the [TM x 64] slice at (m0, k0).
-template <int TM, int BK, bool KMAJOR>
+template <int TM, int BK>
 __device__ __forceinline__ void ct_piece(int it, int tid, int m0, int k0, int& gm, int& gk) {
-  if (!KMAJOR) {
-    const int e = tid + it * 256;
-    gm = m0 + e / (BK / 8);
-    gk = k0 + (e % (BK / 8)) * 8;
-  } else {
-    const int e = tid + it * 256;
-    gk = k0 + e % BK;
-    gm = m0 + (e / BK) * 8;
-  }
+  const int e = tid + it * 256;
+  gk = k0 + e % BK;
+  gm = m0 + (e / BK) * 8;
 }
 
 // Branch-free: a clamped address always loads and an out-of-range piece is zeroed when it is
 // written to LDS (ct_store), not here: a select on the loaded value at this point would make
 // the compiler wait for the loads before the MFMAs they are meant to overlap, and a branch
 // per load lets it serialise them with vmcnt(0) waits.
-template <int TM, int BK, bool KMAJOR>
+template <int TM, int BK>
 __device__ __forceinline__ void ct_fetch(h8 (&r)[TM * BK / 2048], const _Float16* src, int N, int m0, int k0, int tid) {
 #pragma unroll
   for (int it = 0; it < TM * BK / 2048; ++it) {
     int gm, gk;
-    ct_piece<TM, BK, KMAJOR>(it, tid, m0, k0, gm, gk);
+    ct_piece<TM, BK>(it, tid, m0, k0, gm, gk);
     const bool ok = gm < N && gk < N;
-    const int cm = ok ? gm : 0, ck = ok ? gk : 0;
-    r[it] = *reinterpret_cast<const h8*>(src + (KMAJOR ? (size_t)ck * N + cm : (size_t)cm * N + ck));
+    r[it] = *reinterpret_cast<const h8*>(src + (ok ? (size_t)gk * N + gm : 0));
   }
 }
 
-template <int TM, int BK, bool KMAJOR>
+template <int TM, int BK>
 __device__ __forceinline__ void ct_store(_Float16* S, const h8 (&r)[TM * BK / 2048], int N, int m0, int k0, int tid) {
   constexpr int LD = BK + 8;
 #pragma unroll
   for (int it = 0; it < TM * BK / 2048; ++it) {
     int gm, gk;
-    ct_piece<TM, BK, KMAJOR>(it, tid, m0, k0, gm, gk);
+    ct_piece<TM, BK>(it, tid, m0, k0, gm, gk);
     const h8 v = (gm < N && gk < N) ? r[it] : h8{0, 0, 0, 0, 0, 0, 0, 0};
-    if (!KMAJOR) {
-      *reinterpret_cast<h8*>(S + (gm - m0) * LD + (gk - k0)) = v;
-    } else {
-      // lane -> k, so the eight 2-byte LDS stores of a wave hit consecutive k
+    // lane -> k, so the eight 2-byte LDS stores of a wave hit consecutive k
 #pragma unroll
-      for (int j = 0; j < 8; ++j) S[(gm - m0 + j) * LD + (gk - k0)] = v[j];
-    }
+    for (int j = 0; j < 8; ++j) S[(gm - m0 + j) * LD + (gk - k0)] = v[j];
   }
 }
 
@@ -305,9 +294,11 @@ __device__ __forceinline__ void ct_store(_Float16* S, const h8 (&r)[TM * BK / 20
 // longer blocks hide less latency), 32-wide K steps and 8-wave blocks.  The 1-D grid is
 // remapped so that consecutive logical blocks (the tiles of one channel, which share their
 // A rows and B rows) run on the same XCD: the hardware deals block ids round-robin over the
-// 8 XCDs, each with its own L2.
+// 8 XCDs, each with its own L2.  VEC: N % 8 == 0, k-major operands only (with k contiguous such
+// lengths take the direct-to-LDS kernels below).
 template <int TM, int BK, int MINW, bool KMAJOR, bool VEC>
 __global__ __launch_bounds__(256, MINW) void tri_contract_kernel(TriContractParams p) {
+  static_assert(KMAJOR || !VEC, "whole 16-byte pieces of k take the direct-to-LDS kernels");
   constexpr int FM = TM / 32, WT = TM / 2, CT_LD = BK + 8, PER = TM * BK / 2048;
   __shared__ __attribute__((aligned(16))) _Float16 Ls[TM * CT_LD];
   __shared__ __attribute__((aligned(16))) _Float16 Rs[TM * CT_LD];
@@ -330,22 +321,22 @@ __global__ __launch_bounds__(256, MINW) void tri_contract_kernel(TriContractPara
   const int r16 = lane & 15, kq = (lane >> 4) * 8;
   h8 rl[PER], rr[PER];
   if (VEC) {
-    ct_fetch<TM, BK, KMAJOR>(rl, L, p.N, m0, 0, tid);
-    ct_fetch<TM, BK, KMAJOR>(rr, R, p.N, n0, 0, tid);
+    ct_fetch<TM, BK>(rl, L, p.N, m0, 0, tid);
+    ct_fetch<TM, BK>(rr, R, p.N, n0, 0, tid);
   }
   for (int k0 = 0; k0 < p.N; k0 += BK) {
     __syncthreads();
     if (VEC) {
-      ct_store<TM, BK, KMAJOR>(Ls, rl, p.N, m0, k0, tid);
-      ct_store<TM, BK, KMAJOR>(Rs, rr, p.N, n0, k0, tid);
+      ct_store<TM, BK>(Ls, rl, p.N, m0, k0, tid);
+      ct_store<TM, BK>(Rs, rr, p.N, n0, k0, tid);
     } else {
       ct_load<TM, BK, KMAJOR>(Ls, L, p.N, m0, k0, tid);
       ct_load<TM, BK, KMAJOR>(Rs, R, p.N, n0, k0, tid);
     }
     __syncthreads();
     if (VEC && k0 + BK < p.N) {
-      ct_fetch<TM, BK, KMAJOR>(rl, L, p.N, m0, k0 + BK, tid);
-      ct_fetch<TM, BK, KMAJOR>(rr, R, p.N, n0, k0 + BK, tid);
+      ct_fetch<TM, BK>(rl, L, p.N, m0, k0 + BK, tid);
+      ct_fetch<TM, BK>(rr, R, p.N, n0, k0 + BK, tid);
     }
 #pragma unroll
     for (int kk = 0; kk < BK; kk += 32) {
@@ -384,11 +375,11 @@ __global__ __launch_bounds__(256, MINW) void tri_contract_kernel(TriContractPara
   }
 }
 
-// The contraction of operands with k contiguous and a row pitch that is a multiple of 16 (the
-// columns from N to the pitch hold zeros): TM x TM tiles (TM = 128 or 96), K steps of BK double-buffered in LDS and filled by direct global -> LDS
-// loads (16 bytes a lane, no register staging), one barrier a step, the next step's loads in
-// flight during the current step's MFMAs.  A wave's load instruction fills 1 KB of LDS
-// contiguously, so the 16-byte chunks of a row are XOR-swizzled by the row (chunk c of row r
+// The contraction of operands with k contiguous and a row pitch that is a multiple of 8 (the
+// columns from N to the pitch hold zeros): TM x TM tiles (TM = 128 or 96), K steps of BK
+// double-buffered in LDS and filled by direct global -> LDS loads (16 bytes a lane, no register
+// staging), one barrier a step, the next step's loads in flight during the current step's MFMAs.
+// A wave's load instruction fills 1 KB of LDS contiguously, so the 16-byte chunks of a row are XOR-swizzled by the row (chunk c of row r
 // sits in slot c ^ swz(r)) to keep the MFMA fragment reads of 16 rows off a single bank group.
 // Rows past N are clamped to row N - 1: they only feed output rows that are never stored, or
 // columns between N and the pitch.  In a last K step that reaches past the pitch the pieces
@@ -602,21 +593,21 @@ __global__ __launch_bounds__(512) void tri_contract_big_kernel(TriContractParams
   }
 }
 
-template <int TM, int BK = 64, int MINW = 1>
 static void launch_contract(lf_context* ctx, const TriContractParams& cp, int H, bool kmajor) {
+  constexpr int TM = 128, BK = 64, MINW = 3;
   const int tm = (cp.N + TM - 1) / TM;
   const dim3 grid((unsigned)(tm * tm * H));
   const bool vec = (cp.N % 8) == 0;
   if (!kmajor) {
     const long long t256 = (cp.N + 255) / 256, t128 = (cp.N + 127) / 128;
     const bool dma = cp.ld % 8 == 0, tail = cp.ld % 64 != 0;   // rows of whole 16-byte pieces; of whole K steps
-    if (TM == 128 && dma && cp.N >= 768 && t256 * t256 * 65536 * 10 <= t128 * t128 * 16384 * 11) {
+    if (dma && cp.N >= 768 && t256 * t256 * 65536 * 10 <= t128 * t128 * 16384 * 11) {
       const dim3 g((unsigned)(t256 * t256 * H));
       auto k = tail ? tri_contract_big_kernel<64, true> : tri_contract_big_kernel<64, false>;
       hipLaunchKernelGGL(k, g, dim3(512), 0, ctx->stream, cp);
       return;
     }
-    if (TM == 128 && dma) {
+    if (dma) {
       // 128-row tiles at two blocks per CU, or, when the grid is only a few waves of blocks
       // and the last one would run mostly empty, 96-row tiles at three per CU.  Measured: at
       // N = 384 (1152 tiles of 128 in 512 slots: 2.25 waves) the 96-row kernel is 3-4%
@@ -997,7 +988,7 @@ constexpr int tri_o_nwv() { return ACT == DT_F32 ? 8 : 12; }
 // Plane rows are padded to 16 (pitch ld), so a tile always stores 16 aligned columns, whatever
 // N is: with the pitch N, lengths that are not a multiple of 16 needed element-wise stores here,
 // element-wise transposes in the output kernel and an element-wise contraction (N = 825, f32:
-// 352 / 1697 / 303 us per direction for the three kernels against 214 / 258 / 192).
+// 352, 303 and 1697 us per direction for the three kernels against 214, 192 and 258).
 struct TileGeom {
   int src0, sstride, out0, nvalid;
 };
@@ -1525,7 +1516,7 @@ static int tri_mult_impl(lf_context* ctx, const lf_tri_mult_args& a, void* scrat
   cp.R = outgoing ? pp.out[1] : pp.out[0];
   {
     LaunchScope ls(ctx, outgoing ? "tri_out.contract" : "tri_in.contract");
-    launch_contract<128, 64, 3>(ctx, cp, H, !(outgoing || pp.kmajor_out));
+    launch_contract(ctx, cp, H, !(outgoing || pp.kmajor_out));
   }
   LF_TRY(check_hip(hipGetLastError(), "tri_contract launch"));
 
@@ -1565,7 +1556,7 @@ int tri_mult(lf_context* ctx, const lf_tri_mult_args& a) { return tri_mult_impl(
 // tri_noalloc_init, which lf_context_create calls; host code only ever passes that address,
 // never the array's name, which on the host is a stand-in and not a device address.
 // Beyond the documented size it holds the plane rows' padding to 16 and the LayerNorm statistics:
-// at most 5.3 MiB over the shapes accepted (N = 417: 3 * 128 * 417 * 432 f16 and 8 * 417^2).
+// at most 5.6 MiB over the shapes accepted (N = 418: 3 * 128 * 418 * 432 f16 and 8 * 418^2).
 constexpr size_t TRI_NOALLOC_BYTES = (size_t)LF_TRI_NOALLOC_SCRATCH_BYTES + ((size_t)6 << 20);
 static __device__ __align__(256) unsigned char scratch[TRI_NOALLOC_BYTES];
 
