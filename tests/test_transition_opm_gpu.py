@@ -41,8 +41,8 @@ def test_transition_relu(ctx, blockw, rows_shape, which, chunk):
 
 @pytest.mark.parametrize("c,hidden", [(128, 96), (256, 96), (128, 32)])
 def test_transition_fused_odd_chunk_count(ctx, c, hidden):
-    """Hidden widths of 3 and 1 chunks of 32: the fused kernel stages its weight chunks two to
-    an LDS buffer, so a count that is not a multiple of two ends on a half-used buffer."""
+    """Hidden widths of 3 and 1 chunks of 32: the fused kernel takes its weight chunks from two LDS
+    buffers in turn, so an odd count leaves its loop in the middle of a pair."""
     import torch
     from localfold_amd import device as D
     st = S.Stream(c + hidden)
@@ -60,7 +60,7 @@ def test_transition_fused_odd_chunk_count(ctx, c, hidden):
 @pytest.mark.parametrize("which,dt", [("pairTransition", "bfloat16"), ("msaTransition", "bfloat16"),
                                       ("msaTransition", "float16")])
 def test_transition_fused_dtypes(ctx, blockw, which, dt):
-    """16-bit activations, 700 rows (a partial 256-row block); the update alone is compared, so
+    """16-bit activations, 700 rows (a partial last block of 64 rows); the update alone is compared, so
     the output rounding is that of the update's magnitude."""
     import torch
     from localfold_amd import device as D
@@ -188,7 +188,7 @@ def test_opm_ragged(ctx, blockw, s, n):
 
 @pytest.mark.parametrize("dt,accumulate", [("bfloat16", True), ("float16", False), ("float32", False)])
 def test_opm_fused_output(ctx, blockw, dt, accumulate):
-    """c_outer 32, c_z 128 with whole 256-row outer tiles (N = 64, S = 64) takes the fused kernel:
+    """c_outer 32, c_z 128 takes the fused kernel, here with whole 256-row outer tiles (N = 64, S = 64):
     the output GEMM, the /den and the residual run on the outer-product tile in LDS.  Pair in
     each activation dtype, accumulated in place or written to a separate output."""
     import torch
@@ -217,9 +217,11 @@ def test_opm_fused_output(ctx, blockw, dt, accumulate):
                    label=f"opm fused {dt} accumulate={accumulate}")
 
 
-@pytest.mark.parametrize("s,n", [(13, 21), (64, 24)])
+@pytest.mark.parametrize("s,n", [(13, 21), (64, 24), (64, 16), (121, 64)])
 def test_opm_other_widths(ctx, s, n):
-    """c_outer 16, c_z 64: the materialised outer product, ragged and whole sequences."""
+    """c_outer 16, c_z 64: the materialised outer product on 128-row tiles, ragged (N = 21) and whole
+    (N = 24), and on 256-row tiles (N a multiple of 16, S up to a multiple of 64 once rounded up to
+    8): one tile of one K step, and 16 tiles of two."""
     import torch
     from localfold_amd import device as D
     w = S.synthetic_block_weights(c_m=64, c_z=64, c_outer=16, heads_msa=4, heads_pair=4, tri_hidden=64, msa_hidden=64,
