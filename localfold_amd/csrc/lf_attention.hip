@@ -9,13 +9,17 @@
 // from the normalised attention input itself.
 //
 // Kernels:
-//   lnproj  LN + the q/k/v/g (+ bias) projections in one pass over the rows
-//           (q, k: [b][h][n][32] f16; v: [b][h][32][n] f16 (transposed for P.V); g: [h][rows][d], head-major)
-//   keybias kb[b][k] = 1e9 (mask - 1)
-//   flash   per (b, h, 128 queries): S^T = K Q^T on MFMA, online softmax with each lane
-//           owning one query (statistics: two cross-lane shuffles), O^T += V^T P^T on MFMA;
-//           the N^2 x heads logits never leave registers
-//   rowgemm o Wo + bo, + residual, stored through the row map
+//   lnproj    LN + the q/k/v/g (+ bias) projections in one pass over the rows
+//             (q, k: [b][h][n][DP] f16, DP = 16 or 32; v: [b][h][DP][n] f16 (transposed for P.V);
+//             g: [h][rows][d], head-major; bias: [h][i][j], or in fragment order for flash_res)
+//   flash_res (nearly every call: head widths of whole 4, K and V of a row and head within the LDS)
+//             per (b, h, split of the queries): K, V^T and the key bias, which it computes from the
+//             mask, stay in LDS; S^T = K Q^T on MFMA, softmax against a lazily raised base with each
+//             lane owning one query, O^T += V^T P^T on MFMA; the logits never leave registers
+//   keybias   kb[b][k] = 1e9 (mask - 1) for the two below
+//   flash     the others: per (b, h, 128 queries), the keys staged chunk by chunk
+//   pwa_*     pair-weighted averaging (no q and k): one softmax per (h, i), then an NT GEMM
+//   rowgemm   o Wo + bo, + residual, stored through the row map
 #include <algorithm>
 #include <cstdlib>
 #include <type_traits>
@@ -39,7 +43,8 @@ struct FlashParams {
   _Float16* o;
   const float* kb;        // [B][Qp] at a row stride of kb_stride (0: one row shared by every b)
   long long kb_stride;
-  const _Float16* bias;   // [H][Q][Q] or null
+  const _Float16* bias;   // null, or [H][Q][Qp] (flash_kernel), or per head ceil(Q / 16) tiles of
+                          // 16 queries x Qp keys in fragment order (tiled_at; flash_res_kernel)
   int B, H, Q, d, HD;
   int dq;                 // head dims q and k hold (d; 0 when every logit is the bias alone)
   int fix;                // dq < DP or Q not a whole number of chunks: the kernel (the FIX
@@ -725,10 +730,11 @@ __global__ __launch_bounds__(64 * (8 / QT), 4) void flash_kernel(FlashParams p) 
 // core) is flash_kernel's.  That kernel gives a block 128 queries and restages every 64-key
 // chunk for each of them: K/V cross L2 once per 128 queries, each chunk costs 8 waves a barrier,
 // and a block's prologue and epilogue (a quarter of its time at 8 chunks) are paid per 128
-// queries.  Measured (us per launch): triangle attention at
-// N = 512 with 4 x 32 heads 219 -> 157, N = 1024 1374 -> 974, MSA row attention 512 x 384 259 -> 197,
-// column attention 508 x 259 181 -> 129.  There the SIMDs issue 224 cycles of MFMA and 250 of VALU per
-// 16 queries x 64 keys, in 590: the two overlap little, so every VALU instruction left out counts.
+// queries.  Measured (us per launch): triangle attention at N = 512 with 4 x 32 heads 219 -> 157,
+// N = 1024 1374 -> 974, MSA row attention 512 x 384 259 -> 197, column attention 508 x 259 181 -> 129.
+// Counters at N = 512: per 16 queries x 64 keys 14 products (221 cycles of the matrix pipe, which is
+// busy 32% of the time) and 68 vector instructions, 16 of them exponentials.  The two overlap little,
+// so every vector instruction left out counts.
 //
 // S^T tile kt of a chunk holds in row 4*g + i the key 32*(kt/2) + 8*g + 4*(kt%2) + i, so a lane's
 // 16 scores are keys 8*g4 .. +7 of each 32-key half: its V^T pieces are two 16-byte LDS reads.

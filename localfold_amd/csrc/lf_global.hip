@@ -228,7 +228,7 @@ int global_attention(lf_context* ctx, const lf_global_attention_args& a) {
   LF_TRY(expand_flush(ctx, xl, "global.expand"));
   LF_TRY(lnproj_run(ctx, pp, a.act_dtype, "global.project"));
 
-    // where the output kernel holds its weights it multiplies the gate by the attended values as it
+  // where the output kernel holds its weights it multiplies the gate by the attended values as it
   // reads it, which saves a pass over the gate (1024 x 384, bf16: this kernel 52 -> 32 us, the output
   // 55 -> 44 us with its weights held; 5120 x 384: 296 -> 128 and 253 -> 210 us)
   float* att = wo_inkernel && Hd == 64 && C == 64 ? static_cast<float*>(bufs[6]) : nullptr;

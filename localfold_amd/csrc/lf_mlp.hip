@@ -17,14 +17,15 @@
 //          four channels stored as one vector at the end.
 // The next chunk is copied straight to the other buffer during the current chunk's products.
 //
-// What bounds it: the matrix pipes and, in the same issue slots, the vector instructions (the two
-// do not overlap: at 262144 rows of 256, bf16, hidden 1024, MFMA 262 k and the others 130 k of 517 k
-// cycles).  Copies that skip the registers leave room for two blocks of 128 rows a CU, whose
-// LayerNorm, store and product phases interleave; with one block of 8 waves, weights staged
-// through registers and the activation in f32 the same call took 332 us, now 274 us (1.0 PFLOP/s),
-// and 512 x 384 rows of 256 in f32 went from 337 to 258 us, 512 x 512 of 128 with SwiGLU in bf16
-// from 163 to 142 us.  Eight waves sharing a buffer (305), 64 rows a wave (350), three or four
-// buffers and wider read-ahead (275 to 280) were no better.
+// What bounds it: the matrix pipes, and the vector instructions and waits that they do not overlap
+// with.  Counters at 196608 rows of 256, f32, hidden 1024: matrix pipes busy 36% of the time (197 k of
+// 543 k cycles), 2.2 vector instructions to a product.  Copies that skip the registers leave room for
+// two blocks of 128 rows a CU, whose LayerNorm, store and product phases interleave; against one block
+// of 8 waves, weights staged through registers and the activation in f32, 262144 rows of 256 in bf16
+// went from 332 to 274 us (1.0 PFLOP/s), 512 x 384 rows of 256 in f32 from 337 to 258 us (on another
+// box 326 to 247), 512 x 512 of 128 with SwiGLU in bf16 from 163 to 142 us.  Eight waves sharing a
+// buffer (305), 64 rows a wave (350), three or four buffers and wider read-ahead (275 to 280) were no
+// better.
 #include <algorithm>
 #include <cmath>
 
@@ -111,7 +112,7 @@ template <int ACT, int C, int NG, int RT>
 __global__ __launch_bounds__(MLP_NT, 2) void mlp_kernel(MlpParams p) {
   using S = MlpShape<C, NG>;
   constexpr int KS = S::KS, CT = S::CT, NF = S::NF, F1 = S::F1, PER = NF / MLP_WAVES;
-    // separate objects: reads of one buffer are then known not to wait for copies into the other
+  // separate objects: reads of one buffer are then known not to wait for copies into the other
   __shared__ __attribute__((aligned(16))) _Float16 W0[S::CE], W1[S::CE];
   __shared__ __attribute__((aligned(16))) float B0[64], B1[64];   // b1 of the chunk: gate, then value
   __shared__ __attribute__((aligned(16))) float Gs[3 * C];        // LN scale, offset, b2
