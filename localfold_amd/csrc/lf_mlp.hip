@@ -23,7 +23,7 @@
 // two blocks of 128 rows a CU, whose LayerNorm, store and product phases interleave; against one block
 // of 8 waves, weights staged through registers and the activation in f32, 262144 rows of 256 in bf16
 // went from 332 to 274 us (1.0 PFLOP/s), 512 x 384 rows of 256 in f32 from 337 to 258 us (on another
-// box 326 to 247), 512 x 512 of 128 with SwiGLU in bf16 from 163 to 142 us.  Eight waves sharing a
+// card 326 to 247), 512 x 512 of 128 with SwiGLU in bf16 from 163 to 142 us.  Eight waves sharing a
 // buffer (305), 64 rows a wave (350), three or four buffers and wider read-ahead (275 to 280) were no
 // better.
 #include <algorithm>
